@@ -582,12 +582,16 @@ int h1pa_form_assemble(h1pa_form *form, void *stream) {
     even_odd_tables(D, Q, B.data(), G.data(), pack.data() + 4 * Q * D);
     f.basis.upload(pack.data(), pack.size(), s);
     const int64_t nq = (int64_t)Q * Q * Q;
-    if (f.desc.integrators & H1PA_INTEG_DIFFUSION) f.pa_diff.alloc(nq * 6 * sp.ne);
+    // a re-assembly keeps its buffers: a hipFree waits for the whole device
+    auto keep = [](DevBuf<double> &b, int64_t n) {
+        if (b.n != (size_t)n) b.alloc((size_t)n);
+    };
+    if (f.desc.integrators & H1PA_INTEG_DIFFUSION) keep(f.pa_diff, nq * 6 * sp.ne);
     else f.pa_diff.release();
-    if (f.desc.integrators & H1PA_INTEG_MASS) f.pa_mass.alloc(nq * sp.ne);
+    if (f.desc.integrators & H1PA_INTEG_MASS) keep(f.pa_mass, nq * sp.ne);
     else f.pa_mass.release();
     kern::pa_setup(*sp.mesh, f, s);
-    f.ework0.alloc(sp.ne * sp.dof);
+    keep(f.ework0, sp.ne * sp.dof);
     H1PA_HIP(hipStreamSynchronize(s));
     f.assembled = true;
     if (f.desc.integrators & H1PA_INTEG_DIFFUSION) autotune_diffusion(f, s);

@@ -8,22 +8,12 @@
 // J is never stored: at 32M DOFs and p = 1 it alone would be 61 GB.
 #include <cmath>
 
+#include "apply_body.hpp"
+#include "geom_body.hpp"
 #include "internal.hpp"
 
 namespace h1pa {
 namespace kern {
-
-namespace {
-
-constexpr int kBlock = 256;
-inline unsigned nblocks(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
-
-struct GeomBasis {          // geometry basis at the Q Gauss-Legendre points
-    int Q, Dg;
-    double B[10 * 10];      // B[q + Q*d]
-    double G[10 * 10];
-    double w[10];           // 1D Gauss-Legendre weights
-};
 
 GeomBasis make_geom_basis(int Q, int pg) {
     GeomBasis gb{};
@@ -35,6 +25,11 @@ GeomBasis make_geom_basis(int Q, int pg) {
     for (int i = 0; i < Q; ++i) gb.w[i] = w[i];
     return gb;
 }
+
+namespace {
+
+constexpr int kBlock = 256;
+inline unsigned nblocks(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
 struct Fourier8 {           // g(x) = sum_m a cos(2 pi k_m . x + phi_m)
     double k[8][3];
@@ -117,6 +112,158 @@ __global__ void k_nodes_curved(int64_t ne, int Dg, const int *__restrict__ topo,
     X[l + nd * (2 + 3 * e)] = zp;
 }
 
+__device__ inline double coeff_value(int kind, double cval, const double *__restrict__ cdata,
+                                     const Fourier8 &fm, int64_t e, int q, int nq,
+                                     const double (&P)[3]) {
+    const double tp = 6.283185307179586476925286766559;
+    switch (kind) {
+        case H1PA_COEFF_SINCOS:
+            return 1.0 + 0.5 * sin(tp * P[0]) * cos(tp * P[1]) * sin(tp * P[2]);
+        case H1PA_COEFF_PER_ELEMENT: return cdata[e];
+        case H1PA_COEFF_QUADRATURE: return cdata[q + (int64_t)nq * e];
+        case H1PA_COEFF_FOURIER: {
+            double g = 0.0;
+            for (int m = 0; m < 8; ++m)
+                g += fm.a * cos(tp * (fm.k[m][0] * P[0] + fm.k[m][1] * P[1] + fm.k[m][2] * P[2]) +
+                                fm.phi[m]);
+            return exp(g);
+        }
+        default: return cval;
+    }
+}
+
+// What the element, the quadrature column (a, b) and the LDS of this thread
+// are.  Straight-sided elements need no barrier and no LDS, so their threads
+// run over (element, column) without a gap; the curved evaluation keeps the
+// Q^2 threads of nb whole elements in a block.
+template <int Q, int DG>
+struct ColumnOf {
+    int64_t e;
+    int a, b, t;
+    bool valid;
+    double *s;
+    __device__ __forceinline__ ColumnOf(int64_t ne, int nb, int Dg, double *smem) {
+        constexpr int QQ = Q * Q;
+        if constexpr (DG != 2) {
+            const int le = threadIdx.x / QQ;
+            t = threadIdx.x - le * QQ;
+            e = (int64_t)blockIdx.x * nb + le;
+            valid = e < ne;
+            s = smem + geom_tab_lds(Q, Dg) + le * geom_lds(Q, Dg);
+        } else {
+            const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+            e = i / QQ;
+            t = (int)(i - e * QQ);
+            valid = e < ne;
+            s = nullptr;
+        }
+        a = t % Q;
+        b = t / Q;
+    }
+};
+
+template <int Q, int DG>
+__global__ void __launch_bounds__(kBlock)
+k_geometric_factors(int64_t ne, int nb, GeomBasis gb, const double *__restrict__ X,
+                    double *__restrict__ Xq, double *__restrict__ Jq, double *__restrict__ detJ) {
+    extern __shared__ double smem[];
+    constexpr int nq = Q * Q * Q;
+    if constexpr (DG != 2) load_geom_tables(gb, Q, smem);
+    const ColumnOf<Q, DG> k(ne, nb, gb.Dg, smem);
+    const int nd = gb.Dg * gb.Dg * gb.Dg;
+    if constexpr (DG != 2) __syncthreads();
+    GeomColumn<Q, true, DG> g;
+    g.eval(gb, X + (int64_t)nd * 3 * k.e, k.a, k.b, k.t, k.valid, k.s, smem);
+    if (!k.valid) return;
+#pragma unroll
+    for (int qz = 0; qz < Q; ++qz) {
+        double J[9], P[3];
+        g.at(gb, qz, J, P);
+        const int q = k.a + Q * (k.b + Q * qz);
+        if (Xq)
+#pragma unroll
+            for (int r = 0; r < 3; ++r) Xq[q + (int64_t)nq * (r + 3 * k.e)] = P[r];
+        if (Jq)
+#pragma unroll
+            for (int c = 0; c < 9; ++c) Jq[q + (int64_t)nq * (c + 9 * k.e)] = J[c];
+        if (detJ) detJ[q + (int64_t)nq * k.e] = det3(J);
+    }
+}
+
+// D = W k adj(J) adj(J)^T / det J and / or W k det J at the Q points of a
+// column.  WP: the coefficient needs the physical point.
+template <int Q, bool WP, int DG>
+__global__ void __launch_bounds__(kBlock)
+k_pa_setup(int64_t ne, int nb, GeomBasis gb, const double *__restrict__ X, int kind,
+           double cval, const double *__restrict__ cdata, Fourier8 fm, double *__restrict__ Dd,
+           double *__restrict__ Mv) {
+    extern __shared__ double smem[];
+    constexpr int nq = Q * Q * Q;
+    if constexpr (DG != 2) load_geom_tables(gb, Q, smem);
+    const ColumnOf<Q, DG> c(ne, nb, gb.Dg, smem);
+    const int nd = gb.Dg * gb.Dg * gb.Dg;
+    if constexpr (DG != 2) __syncthreads();
+    GeomColumn<Q, WP, DG> g;
+    g.eval(gb, X + (int64_t)nd * 3 * c.e, c.a, c.b, c.t, c.valid, c.s, smem);
+    if (!c.valid) return;
+    const double wxy = gb.w[c.a] * gb.w[c.b];
+    double *const dcol = Dd ? Dd + (int64_t)nq * 6 * c.e + c.a + Q * c.b : nullptr;
+    double *const mcol = Mv ? Mv + (int64_t)nq * c.e + c.a + Q * c.b : nullptr;
+    // the curved evaluation holds its Q points in registers: fully unrolled
+    constexpr int UZ = DG != 2 ? Q : 1;
+#pragma unroll UZ
+    for (int qz = 0; qz < Q; ++qz) {
+        double J[9], P[3] = {0.0, 0.0, 0.0};
+        g.at(gb, qz, J, P);
+        const double W = wxy * gb.w[qz];
+        const double k = coeff_value(kind, cval, cdata, fm, c.e, c.a + Q * (c.b + Q * qz), nq, P);
+        const double J11 = J[0], J21 = J[1], J31 = J[2];
+        const double J12 = J[3], J22 = J[4], J32 = J[5];
+        const double J13 = J[6], J23 = J[7], J33 = J[8];
+        const double detJ = det3(J);
+        if (mcol) mcol[Q * Q * qz] = W * k * detJ;
+        if (dcol) {
+            // (1/detJ) adj(J) adj(J)^T, symmetric storage 11,21,31,22,32,33
+            const double A11 = J22 * J33 - J23 * J32, A12 = J32 * J13 - J12 * J33,
+                         A13 = J12 * J23 - J22 * J13;
+            const double A21 = J31 * J23 - J21 * J33, A22 = J11 * J33 - J13 * J31,
+                         A23 = J21 * J13 - J11 * J23;
+            const double A31 = J21 * J32 - J31 * J22, A32 = J31 * J12 - J11 * J32,
+                         A33 = J11 * J22 - J12 * J21;
+            const double s = W / detJ * k;
+            double *d = dcol + Q * Q * qz;
+            d[0 * nq] = s * (A11 * A11 + A12 * A12 + A13 * A13);
+            d[1 * nq] = s * (A11 * A21 + A12 * A22 + A13 * A23);
+            d[2 * nq] = s * (A11 * A31 + A12 * A32 + A13 * A33);
+            d[3 * nq] = s * (A21 * A21 + A22 * A22 + A23 * A23);
+            d[4 * nq] = s * (A21 * A31 + A22 * A32 + A23 * A33);
+            d[5 * nq] = s * (A31 * A31 + A32 * A32 + A33 * A33);
+        }
+    }
+}
+
+// Launch shape of a geometry kernel: blocks, threads and LDS bytes.
+struct GeomLaunch {
+    dim3 grid, block;
+    unsigned lds;
+    int nb;  // elements per block
+};
+GeomLaunch geom_launch(int64_t ne, int Q, int Dg) {
+    GeomLaunch l;
+    if (Dg == 2) {
+        l.nb = 0;
+        l.grid = dim3(nblocks(ne * Q * Q));
+        l.block = dim3(kBlock);
+        l.lds = 0;
+    } else {
+        l.nb = geom_nb(Q, geom_lds(Q, Dg));
+        l.grid = dim3((unsigned)((ne + l.nb - 1) / l.nb));
+        l.block = dim3(l.nb * Q * Q);
+        l.lds = 8 * (geom_tab_lds(Q, Dg) + l.nb * geom_lds(Q, Dg));
+    }
+    return l;
+}
+
 // Jacobian J(r, c) = dx_r / dxi_c and the physical point at quadrature point
 // (qx, qy, qz) of element e, from nodes X[Dg^3][3][ne].
 __device__ inline void eval_geom(const GeomBasis &gb, const double *__restrict__ X, int64_t e,
@@ -144,85 +291,6 @@ __device__ inline void eval_geom(const GeomBasis &gb, const double *__restrict__
                 }
             }
         }
-    }
-}
-
-__device__ inline double coeff_value(int kind, double cval, const double *__restrict__ cdata,
-                                     const Fourier8 &fm, int64_t e, int q, int nq,
-                                     const double P[3]) {
-    const double tp = 6.283185307179586476925286766559;
-    switch (kind) {
-        case H1PA_COEFF_SINCOS:
-            return 1.0 + 0.5 * sin(tp * P[0]) * cos(tp * P[1]) * sin(tp * P[2]);
-        case H1PA_COEFF_PER_ELEMENT: return cdata[e];
-        case H1PA_COEFF_QUADRATURE: return cdata[q + (int64_t)nq * e];
-        case H1PA_COEFF_FOURIER: {
-            double g = 0.0;
-            for (int m = 0; m < 8; ++m)
-                g += fm.a * cos(tp * (fm.k[m][0] * P[0] + fm.k[m][1] * P[1] + fm.k[m][2] * P[2]) +
-                                fm.phi[m]);
-            return exp(g);
-        }
-        default: return cval;
-    }
-}
-
-__global__ void k_geometric_factors(int64_t ne, GeomBasis gb, const double *__restrict__ X,
-                                    double *__restrict__ Xq, double *__restrict__ Jq,
-                                    double *__restrict__ detJ) {
-    const int Q = gb.Q, nq = Q * Q * Q;
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= ne * nq) return;
-    const int64_t e = i / nq;
-    const int q = (int)(i - e * nq);
-    double J[3][3], P[3];
-    eval_geom(gb, X, e, q % Q, (q / Q) % Q, q / (Q * Q), J, P);
-    if (Xq)
-        for (int r = 0; r < 3; ++r) Xq[q + (int64_t)nq * (r + 3 * e)] = P[r];
-    if (Jq)
-        for (int c = 0; c < 3; ++c)
-            for (int r = 0; r < 3; ++r) Jq[q + (int64_t)nq * (r + 3 * (c + 3 * e))] = J[r][c];
-    if (detJ)
-        detJ[q + (int64_t)nq * e] = J[0][0] * (J[1][1] * J[2][2] - J[2][1] * J[1][2]) -
-                                    J[1][0] * (J[0][1] * J[2][2] - J[2][1] * J[0][2]) +
-                                    J[2][0] * (J[0][1] * J[1][2] - J[1][1] * J[0][2]);
-}
-
-__global__ void k_pa_setup(int64_t ne, GeomBasis gb, const double *__restrict__ X, int kind,
-                           double cval, const double *__restrict__ cdata, Fourier8 fm,
-                           double *__restrict__ Dd, double *__restrict__ Mv) {
-    const int Q = gb.Q, nq = Q * Q * Q;
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= ne * nq) return;
-    const int64_t e = i / nq;
-    const int q = (int)(i - e * nq);
-    const int qx = q % Q, qy = (q / Q) % Q, qz = q / (Q * Q);
-    double J[3][3], P[3];
-    eval_geom(gb, X, e, qx, qy, qz, J, P);
-    const double W = gb.w[qx] * gb.w[qy] * gb.w[qz];
-    const double k = coeff_value(kind, cval, cdata, fm, e, q, nq, P);
-    const double J11 = J[0][0], J21 = J[1][0], J31 = J[2][0];
-    const double J12 = J[0][1], J22 = J[1][1], J32 = J[2][1];
-    const double J13 = J[0][2], J23 = J[1][2], J33 = J[2][2];
-    const double detJ = J11 * (J22 * J33 - J32 * J23) - J21 * (J12 * J33 - J32 * J13) +
-                        J31 * (J12 * J23 - J22 * J13);
-    if (Mv) Mv[q + (int64_t)nq * e] = W * k * detJ;
-    if (Dd) {
-        // (1/detJ) adj(J) adj(J)^T, symmetric storage 11,21,31,22,32,33
-        const double A11 = J22 * J33 - J23 * J32, A12 = J32 * J13 - J12 * J33,
-                     A13 = J12 * J23 - J22 * J13;
-        const double A21 = J31 * J23 - J21 * J33, A22 = J11 * J33 - J13 * J31,
-                     A23 = J21 * J13 - J11 * J23;
-        const double A31 = J21 * J32 - J31 * J22, A32 = J31 * J12 - J11 * J32,
-                     A33 = J11 * J22 - J12 * J21;
-        const double s = W / detJ * k;
-        double *d = Dd + (int64_t)nq * 6 * e + q;
-        d[0 * nq] = s * (A11 * A11 + A12 * A12 + A13 * A13);
-        d[1 * nq] = s * (A11 * A21 + A12 * A22 + A13 * A23);
-        d[2 * nq] = s * (A11 * A31 + A12 * A32 + A13 * A33);
-        d[3 * nq] = s * (A21 * A21 + A22 * A22 + A23 * A23);
-        d[4 * nq] = s * (A21 * A31 + A22 * A32 + A23 * A33);
-        d[5 * nq] = s * (A31 * A31 + A32 * A32 + A33 * A33);
     }
 }
 
@@ -281,25 +349,58 @@ void nodes_curved(const Mesh &m, int pg, double amp, double *d_nodes, hipStream_
     H1PA_HIP(hipStreamSynchronize(s));
 }
 
+// q1d -> template argument
+#define H1PA_FOR_EACH_Q(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10)
+
 void geometric_factors(const Mesh &m, int q1d, double *X, double *J, double *detJ,
                        hipStream_t s) {
     H1PA_CHECK(q1d >= 1 && q1d <= 10, H1PA_EUNSUP, "q1d must be in [1,10]");
     const GeomBasis gb = make_geom_basis(q1d, m.node_order);
-    const int64_t n = m.ne * q1d * q1d * q1d;
-    hipLaunchKernelGGL(k_geometric_factors, dim3(nblocks(n)), dim3(kBlock), 0, s, m.ne, gb,
-                       m.d_nodes.p, X, J, detJ);
+    const GeomLaunch l = geom_launch(m.ne, q1d, gb.Dg);
+#define X_(Q)                                                                                 \
+    if (q1d == Q) {                                                                           \
+        if (gb.Dg == 2)                                                                       \
+            hipLaunchKernelGGL((k_geometric_factors<Q, 2>), l.grid, l.block, l.lds, s,        \
+                               m.ne, l.nb, gb, m.d_nodes.p, X, J, detJ);                      \
+        else                                                                                  \
+            hipLaunchKernelGGL((k_geometric_factors<Q, 0>), l.grid, l.block, l.lds, s,        \
+                               m.ne, l.nb, gb, m.d_nodes.p, X, J, detJ);                      \
+    }
+    H1PA_FOR_EACH_Q(X_)
+#undef X_
     H1PA_HIP(hipGetLastError());
 }
 
 void pa_setup(const Mesh &m, const Form &f, hipStream_t s) {
-    const int Q = f.q1d;
-    H1PA_CHECK(Q >= 1 && Q <= 10, H1PA_EUNSUP, "q1d must be in [1,10]");
-    const GeomBasis gb = make_geom_basis(Q, m.node_order);
+    const int q1d = f.q1d;
+    H1PA_CHECK(q1d >= 2 && q1d <= 10, H1PA_EUNSUP, "q1d must be in [2,10]");
+    const GeomBasis gb = make_geom_basis(q1d, m.node_order);
     const Fourier8 fm = make_fourier(f.desc.coeff_seed);
-    const int64_t n = m.ne * Q * Q * Q;
-    hipLaunchKernelGGL(k_pa_setup, dim3(nblocks(n)), dim3(kBlock), 0, s, m.ne, gb, m.d_nodes.p,
-                       f.desc.coeff_kind, f.desc.coeff_value, f.desc.d_coeff, fm, f.pa_diff.p,
-                       f.pa_mass.p);
+    const bool wp = f.desc.coeff_kind == H1PA_COEFF_SINCOS ||
+                    f.desc.coeff_kind == H1PA_COEFF_FOURIER;
+    const GeomLaunch l = geom_launch(m.ne, q1d, gb.Dg);
+#define K_(Q, WP, DG)                                                                         \
+    hipLaunchKernelGGL((k_pa_setup<Q, WP, DG>), l.grid, l.block, l.lds, s, m.ne, l.nb,    \
+                       gb, m.d_nodes.p, f.desc.coeff_kind, f.desc.coeff_value,          \
+                       f.desc.d_coeff, fm, f.pa_diff.p, f.pa_mass.p)
+#define W_(Q, DG)                                                                             \
+    do {                                                                                      \
+        if (wp) K_(Q, true, DG);                                                              \
+        else K_(Q, false, DG);                                                                \
+    } while (0)
+    // geometry of the field's own order (q1d = Dg or Dg + 1) has its node count
+    // compiled in; other curved orders read it at run time
+#define X_(Q)                                                                                 \
+    if (q1d == Q) {                                                                           \
+        if (gb.Dg == 2) W_(Q, 2);                                                             \
+        else if (gb.Dg == Q && Q > 2 && Q < 10) W_(Q, (Q > 2 && Q < 10 ? Q : 0));             \
+        else if (gb.Dg == Q - 1 && Q > 3) W_(Q, (Q > 3 ? Q - 1 : 0));                         \
+        else W_(Q, 0);                                                                        \
+    }
+    X_(2) X_(3) X_(4) X_(5) X_(6) X_(7) X_(8) X_(9) X_(10)
+#undef X_
+#undef W_
+#undef K_
     H1PA_HIP(hipGetLastError());
 }
 

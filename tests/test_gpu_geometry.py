@@ -1,0 +1,68 @@
+"""GPU: the sum-factorized element geometry against the oracle's, at every
+node order (1..8) and number of points (1..10), so at every kernel that is
+chosen by them, with element counts that leave the last block partly filled.
+
+Bar: 1e-13 relative (2-norm).  A Jacobian entry is three nested sums of at most
+nine products with table entries of size at most ~50 (the derivative row of
+order 8), each rounded to 2^-53 of its partial sums: below 27 * 2^-53 * 30 on
+the entries of a mesh whose nodes move by a few percent of h, 9e-14 at worst
+and far less in the mean that the 2-norm takes.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+RTOL = 1e-13
+
+
+def _rel(a, b):
+    return np.linalg.norm(np.ravel(a) - np.ravel(b)) / np.linalg.norm(b)
+
+
+def _nodes(orc, M, torch, dims, g, seed):
+    """A mesh with order-g nodes given by the caller, moved at random by 0.05 h."""
+    mesh = M.Mesh.MakeCartesian3D(*dims)
+    om = orc.CartesianMesh(*dims)
+    X = om.nodes_curved(om.vertices(), g, 0.0).copy()
+    X += np.random.default_rng(seed).uniform(-0.05, 0.05, X.size).reshape(X.shape) / (max(dims) * g * g)
+    mesh.SetNodes(g, torch.from_numpy(np.ravel(X).copy()).cuda())
+    return mesh, X
+
+
+@pytest.mark.parametrize("g", range(1, 9))
+@pytest.mark.parametrize("dims", [(1, 1, 1), (5, 4, 3)])
+def test_geometric_factors_every_order(orc, h1pa, torch_cuda, g, dims):
+    mesh, X = _nodes(orc, h1pa, torch_cuda, dims, g, g)
+    ne = int(np.prod(dims))
+    for q in range(1, 11):
+        J, P = orc.geom(ne, g, q, X)
+        Xq, Jq, dJ = (t.cpu().numpy() for t in mesh.GetGeometricFactors(q))
+        assert _rel(Xq, P) < RTOL and _rel(Jq, J) < RTOL, (g, q)
+        Jr = np.asarray(J).reshape(ne, 3, 3, -1)
+        assert _rel(dJ, np.linalg.det(Jr.transpose(0, 3, 2, 1))) < RTOL, (g, q)
+
+
+@pytest.mark.parametrize("p", range(1, 9))
+@pytest.mark.parametrize("g", range(1, 9))
+def test_pa_data_every_order(orc, h1pa, torch_cuda, p, g):
+    M, dims = h1pa, (5, 3, 3)
+    mesh, X = _nodes(orc, M, torch_cuda, dims, g, 10 * p + g)
+    ne = int(np.prod(dims))
+    fes = M.FiniteElementSpace(mesh, M.H1_FECollection(p, 3))
+    kv = np.random.default_rng(p).uniform(0.5, 2.0, ne)
+    for q in (p + 1, p + 2):
+        J, P = orc.geom(ne, g, q, X)
+        W = orc.tensor_weights(q)
+        for coeff, k in ((M.SinCosCoefficient(), orc.coeff_sincos(q, ne, P)),
+                         (M.PWConstCoefficient(torch_cuda.from_numpy(kv).cuda()),
+                          np.repeat(kv, q ** 3))):
+            a = M.BilinearForm(fes)
+            a.SetAssemblyLevel(M.AssemblyLevel.PARTIAL)
+            a.AddDomainIntegrator(M.DiffusionIntegrator(coeff, q))
+            a.AddDomainIntegrator(M.MassIntegrator(coeff, q))
+            a.Assemble()
+            a.Assemble()  # in place, into the same buffers
+            dd, dm = a.PAData()
+            assert _rel(dd.cpu().numpy(), orc.diffusion_setup(q, ne, W, J, k)) < RTOL
+            assert _rel(dm.cpu().numpy(), orc.mass_setup(q, ne, W, J, k)) < RTOL
