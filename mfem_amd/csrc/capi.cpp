@@ -1036,8 +1036,15 @@ int h1pa_space_domain_lf_qf(h1pa_space *space, double fval, const double *d_fq, 
     hipStream_t s = as_stream(stream);
     sp.mesh->ensure_nodes(s);
     StreamBuf<double> bE(sp.ne * sp.dof, s);
-    kern::domain_lf(*sp.mesh, sp.p, fval, d_fq, bE.p, s);
-    restriction_scatter(sp.restr, true, bE.p, b, 0, s);
+    kern::EOut out;  // the fused layout of the applies: interior DOFs straight to b
+    out.ye = bE.p;
+    out.yL = b;
+    out.bb = sp.restr.bubble_begin;
+    out.l2n = sp.restr.lex2nat.p;
+    kern::domain_lf(*sp.mesh, sp.p, fval, d_fq, out, s);
+    kern::restrict_mult_transpose(sp.restr.bubble_begin, sp.restr.offsets.p,
+                                  sp.restr.indices_nat.p, bE.p, b, 0, sp.restr.perm.p,
+                                  sp.restr.nperm, s);
     H1PA_HIP(hipStreamSynchronize(s));
     API_END
 }

@@ -6,6 +6,7 @@
 // PA data (PADiffusionSetup3D, fem/integ/bilininteg_diffusion_kernels.cpp:
 // 262-386; MassIntegrator::AssemblePA, fem/integ/bilininteg_mass_pa.cpp:76-88).
 // J is never stored: at 32M DOFs and p = 1 it alone would be 61 GB.
+#include <algorithm>
 #include <cmath>
 
 #include "apply_body.hpp"
@@ -264,64 +265,82 @@ GeomLaunch geom_launch(int64_t ne, int Q, int Dg) {
     return l;
 }
 
-// Jacobian J(r, c) = dx_r / dxi_c and the physical point at quadrature point
-// (qx, qy, qz) of element e, from nodes X[Dg^3][3][ne].
-__device__ inline void eval_geom(const GeomBasis &gb, const double *__restrict__ X, int64_t e,
-                                 int qx, int qy, int qz, double J[3][3], double P[3]) {
-    const int Dg = gb.Dg, Q = gb.Q, nd = Dg * Dg * Dg;
-    for (int r = 0; r < 3; ++r) {
-        P[r] = 0.0;
-        for (int c = 0; c < 3; ++c) J[r][c] = 0.0;
-    }
-    for (int k = 0; k < Dg; ++k) {
-        const double bz = gb.B[qz + Q * k], gz = gb.G[qz + Q * k];
-        for (int j = 0; j < Dg; ++j) {
-            const double by = gb.B[qy + Q * j], gy = gb.G[qy + Q * j];
-            for (int i = 0; i < Dg; ++i) {
-                const double bx = gb.B[qx + Q * i], gx = gb.G[qx + Q * i];
-                const int l = i + Dg * (j + Dg * k);
-                const double w0 = gx * by * bz, w1 = bx * gy * bz, w2 = bx * by * gz,
-                             wv = bx * by * bz;
-                for (int r = 0; r < 3; ++r) {
-                    const double xv = X[l + nd * (r + 3 * e)];
-                    J[r][0] += w0 * xv;
-                    J[r][1] += w1 * xv;
-                    J[r][2] += w2 * xv;
-                    P[r] += wv * xv;
-                }
-            }
+// DomainLFIntegrator (fem/lininteg.cpp:51-79) at Q = D points per direction:
+// b_e = (B^T x B^T x B^T) [w det J f], f at quadrature point q of element e:
+// fq[q + nq e] when fq is given (a QuadratureFunction, points x fastest), else
+// the constant f.  The sum over the D^3 points of each of the D^3 rows taken
+// directly cost 2 D^6 operations an element and was all of the time (933 us at
+// p = 5, 23^3 elements); contracted along z, y, x it is 6 D^4 and the kernel
+// takes 19 us: latency, 7 blocks per CU at that size; its 37 MB take 7 us at the
+// rate of a large copy.
+struct LfBasis {
+    double B[81];  // B[q + Q d]
+};
+
+template <int D, int DG>
+__global__ void __launch_bounds__(kBlock)
+k_domain_lf(int64_t ne, int nb, int per, GeomBasis gb, LfBasis lb, const double *__restrict__ X,
+            double f, const double *__restrict__ fq, const EOut out) {
+    extern __shared__ double smem[];
+    constexpr int Q = D, QQ = Q * Q, nq = Q * Q * Q;
+    if constexpr (DG != 2) load_geom_tables(gb, Q, smem);
+    const int le = threadIdx.x / QQ, t = threadIdx.x - le * QQ;
+    const int a = t % Q, b = t / Q;
+    const int64_t e = (int64_t)blockIdx.x * nb + le;
+    const bool valid = e < ne;
+    double *const s = smem + geom_tab_lds(Q, gb.Dg) + le * per;
+    const int nd = gb.Dg * gb.Dg * gb.Dg;
+    double v[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) v[q] = (valid && fq) ? fq[a + Q * b + QQ * q + nq * e] : f;
+    if constexpr (DG != 2) __syncthreads();
+    {
+        GeomColumn<Q, false, DG> g;
+        g.eval(gb, X + (int64_t)nd * 3 * e, a, b, t, valid, s, smem);
+        const double wxy = gb.w[a] * gb.w[b];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            double J[9], P[3];
+            g.at(gb, q, J, P);
+            v[q] *= wxy * gb.w[q] * det3(J);
         }
     }
-}
-
-// DomainLFIntegrator with constant f, Q = p + 1 (fem/lininteg.cpp:51-79):
-// one block per element; detJ at the Q^3 points staged in LDS first.
-// f at quadrature point q of element e: fq[q + nq e] when fq is given (a
-// QuadratureFunction, points x fastest), else the constant f.
-__global__ void k_domain_lf(int64_t ne, int D, GeomBasis gb, const double *__restrict__ Bs,
-                            const double *__restrict__ X, double f,
-                            const double *__restrict__ fq, double *__restrict__ bE) {
-    __shared__ double wdet[1000];
-    const int Q = gb.Q, nq = Q * Q * Q, nd = D * D * D;
-    const int64_t e = blockIdx.x;
-    for (int q = threadIdx.x; q < nq; q += blockDim.x) {
-        const int qx = q % Q, qy = (q / Q) % Q, qz = q / (Q * Q);
-        double J[3][3], P[3];
-        eval_geom(gb, X, e, qx, qy, qz, J, P);
-        const double detJ = J[0][0] * (J[1][1] * J[2][2] - J[2][1] * J[1][2]) -
-                            J[1][0] * (J[0][1] * J[2][2] - J[2][1] * J[0][2]) +
-                            J[2][0] * (J[0][1] * J[1][2] - J[1][1] * J[0][2]);
-        wdet[q] = gb.w[qx] * gb.w[qy] * gb.w[qz] * detJ * (fq ? fq[q + (int64_t)nq * e] : f);
+    if constexpr (DG != 2) __syncthreads();  // the geometry's LDS is free
+    if (valid) {   // z: thread (qx, qy)
+#pragma unroll
+        for (int dz = 0; dz < D; ++dz) {
+            double z = 0.0;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) z = fma(lb.B[q + Q * dz], v[q], z);
+            s[a + Q * (b + Q * dz)] = z;
+        }
     }
     __syncthreads();
-    for (int l = threadIdx.x; l < nd; l += blockDim.x) {
-        const int dx = l % D, dy = (l / D) % D, dz = l / (D * D);
-        double s = 0.0;
-        for (int q = 0; q < nq; ++q) {
-            const int qx = q % Q, qy = (q / Q) % Q, qz = q / (Q * Q);
-            s += wdet[q] * Bs[qx + Q * dx] * Bs[qy + Q * dy] * Bs[qz + Q * dz];
+    if (valid)   // y: thread (qx, dz)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) v[q] = s[a + Q * (q + Q * b)];
+    __syncthreads();
+    if (valid)
+#pragma unroll
+        for (int dy = 0; dy < D; ++dy) {
+            double y = 0.0;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) y = fma(lb.B[q + Q * dy], v[q], y);
+            s[a + Q * (dy + D * b)] = y;
         }
-        bE[l + (int64_t)nd * e] = s;
+    __syncthreads();
+    if (valid) {   // x: thread (dy, dz)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) v[q] = s[q + Q * (a + D * b)];
+        double yv[D];
+#pragma unroll
+        for (int dx = 0; dx < D; ++dx) {
+            double x = 0.0;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) x = fma(lb.B[q + Q * dx], v[q], x);
+            yv[dx] = x;
+        }
+        store_line<D, double>(out, e, a, b, yv, 0);
     }
 }
 
@@ -411,18 +430,31 @@ void randomize(int64_t n, double *x, uint64_t seed, double lo, double hi, hipStr
     H1PA_HIP(hipGetLastError());
 }
 
-void domain_lf(const Mesh &m, int p, double f, const double *fq, double *bE, hipStream_t s) {
-    const int Q = p + 1, D = p + 1;
-    const GeomBasis gb = make_geom_basis(Q, m.node_order);
-    double x[16], w[16], B[256], G[256];
-    gauss_legendre(Q, x, w);
-    lagrange_basis(p, Q, x, B, G);
-    StreamBuf<double> Bs;
-    Bs.upload(B, Q * D, s);
-    hipLaunchKernelGGL(k_domain_lf, dim3((unsigned)m.ne), dim3(256), 0, s, m.ne, D, gb, Bs.p,
-                       m.d_nodes.p, f, fq, bE);
+void domain_lf(const Mesh &m, int p, double f, const double *fq, const EOut &out,
+               hipStream_t s) {
+    const int D = p + 1;
+    const GeomBasis gb = make_geom_basis(D, m.node_order);
+    double x[16], w[16], G[256];
+    LfBasis lb;
+    gauss_legendre(D, x, w);
+    lagrange_basis(p, D, x, lb.B, G);
+    const int per = std::max(geom_lds(D, gb.Dg), D * D * D);
+    const int nb = geom_nb(D, per);
+    const dim3 grid((unsigned)((m.ne + nb - 1) / nb)), block(nb * D * D);
+    const unsigned lds = 8 * (geom_tab_lds(D, gb.Dg) + nb * per);
+#define K_(D_, DG)                                                                            \
+    hipLaunchKernelGGL((k_domain_lf<D_, DG>), grid, block, lds, s, m.ne, nb, per, gb, lb,     \
+                       m.d_nodes.p, f, fq, out)
+#define X_(D_)                                                                                \
+    if (D == D_) {                                                                            \
+        if (gb.Dg == 2) K_(D_, 2);                                                            \
+        else if (gb.Dg == D_) K_(D_, D_);                                                     \
+        else K_(D_, 0);                                                                       \
+    }
+    X_(2) X_(3) X_(4) X_(5) X_(6) X_(7) X_(8) X_(9)
+#undef X_
+#undef K_
     H1PA_HIP(hipGetLastError());
-    H1PA_HIP(hipStreamSynchronize(s));
 }
 
 }  // namespace kern

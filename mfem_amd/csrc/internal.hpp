@@ -319,9 +319,6 @@ void qinterp(Space &sp, int q1d, int vdim, unsigned flags, int by_vdim, const do
 void geometric_factors(const Mesh &m, int q1d, double *X, double *J, double *detJ,
                        hipStream_t s);
 void pa_setup(const Mesh &m, const Form &f, hipStream_t s);
-// DomainLFIntegrator element vectors at q1d = p + 1: constant f, or f given
-// per quadrature point (fq[q + (p+1)^3 e]) when fq is not null.
-void domain_lf(const Mesh &m, int p, double f, const double *fq, double *bE, hipStream_t s);
 void randomize(int64_t n, double *x, uint64_t seed, double lo, double hi, hipStream_t s);
 
 // E->E: ye = A_E xe (overwrite) or += ; x may be gathered from an L-vector
@@ -339,6 +336,9 @@ struct EOutT {
     const int *stop = nullptr;  // device flag: when nonzero the launch does nothing
 };
 using EOut = EOutT<double>;
+// DomainLFIntegrator element vectors at q1d = p + 1: constant f, or f given
+// per quadrature point (fq[q + (p+1)^3 e]) when fq is not null.
+void domain_lf(const Mesh &m, int p, double f, const double *fq, const EOut &out, hipStream_t s);
 // Reduced-precision applies: FP32 vectors/arithmetic, PA data as FP32
 // (pa_kind 0) or BF16 (pa_kind 1, FP32 accumulation).
 void diffusion_apply_lp(int p, int q1d, int64_t ne, const float *basis, const void *pa,

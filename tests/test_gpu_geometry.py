@@ -66,3 +66,24 @@ def test_pa_data_every_order(orc, h1pa, torch_cuda, p, g):
             dd, dm = a.PAData()
             assert _rel(dd.cpu().numpy(), orc.diffusion_setup(q, ne, W, J, k)) < RTOL
             assert _rel(dm.cpu().numpy(), orc.mass_setup(q, ne, W, J, k)) < RTOL
+
+
+@pytest.mark.parametrize("p", range(1, 9))
+@pytest.mark.parametrize("g", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_domain_rhs_every_order(orc, h1pa, torch_cuda, p, g):
+    """b = sum over elements and points of w det J f B: sums of positive weights
+    against basis values below 1 in size, so the same bar holds."""
+    M, dims = h1pa, (5, 3, 3)
+    mesh, X = _nodes(orc, M, torch_cuda, dims, g, 100 * p + g)
+    ne = int(np.prod(dims))
+    fes = M.FiniteElementSpace(mesh, M.H1_FECollection(p, 3))
+    gmap = fes.GetElementRestriction().GatherMap().cpu().numpy()
+    fq = np.random.default_rng(p).uniform(-1, 1, (p + 1) ** 3 * ne)
+    for coeff, kw in ((M.ConstantCoefficient(1.5), dict(f=1.5)),
+                      (M.QuadratureFunctionCoefficient(torch_cuda.from_numpy(fq).cuda()),
+                       dict(fq=fq))):
+        lf = M.LinearForm(fes)
+        lf.AddDomainIntegrator(M.DomainLFIntegrator(coeff))
+        ref = np.zeros(fes.GetNDofs())
+        np.add.at(ref, gmap, np.ravel(orc.domain_lf(p, ne, g, X, **kw)))
+        assert _rel(lf.Assemble().cpu().numpy(), ref) < RTOL
