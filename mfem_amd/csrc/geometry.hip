@@ -163,7 +163,7 @@ struct ColumnOf {
     }
 };
 
-template <int Q, int DG>
+template <int Q, bool WP, int DG>
 __global__ void __launch_bounds__(kBlock)
 k_geometric_factors(int64_t ne, int nb, GeomBasis gb, const double *__restrict__ X,
                     double *__restrict__ Xq, double *__restrict__ Jq, double *__restrict__ detJ) {
@@ -173,7 +173,7 @@ k_geometric_factors(int64_t ne, int nb, GeomBasis gb, const double *__restrict__
     const ColumnOf<Q, DG> k(ne, nb, gb.Dg, smem);
     const int nd = gb.Dg * gb.Dg * gb.Dg;
     if constexpr (DG != 2) __syncthreads();
-    GeomColumn<Q, true, DG> g;
+    GeomColumn<Q, WP, DG> g;
     g.eval(gb, X + (int64_t)nd * 3 * k.e, k.a, k.b, k.t, k.valid, k.s, smem);
     if (!k.valid) return;
 #pragma unroll
@@ -181,7 +181,7 @@ k_geometric_factors(int64_t ne, int nb, GeomBasis gb, const double *__restrict__
         double J[9], P[3];
         g.at(gb, qz, J, P);
         const int q = k.a + Q * (k.b + Q * qz);
-        if (Xq)
+        if constexpr (WP)
 #pragma unroll
             for (int r = 0; r < 3; ++r) Xq[q + (int64_t)nq * (r + 3 * k.e)] = P[r];
         if (Jq)
@@ -368,25 +368,35 @@ void nodes_curved(const Mesh &m, int pg, double amp, double *d_nodes, hipStream_
     H1PA_HIP(hipStreamSynchronize(s));
 }
 
-// q1d -> template argument
-#define H1PA_FOR_EACH_Q(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10)
+// Launches K_(Q, WP, DG) for the number of points and the node count: the field's
+// own order (isoparametric, Q = Dg, Dg + 1 and, for the interpolator, Dg + 2)
+// has its node count compiled in; other curved orders read it at run time.
+#define W_(Q, DG)                                                                             \
+    do {                                                                                      \
+        if (wp) K_(Q, true, DG);                                                              \
+        else K_(Q, false, DG);                                                                \
+    } while (0)
+#define X_(Q)                                                                                 \
+    if (q1d == Q) {                                                                           \
+        if (gb.Dg == 2) W_(Q, 2);                                                             \
+        else if (gb.Dg == Q && Q > 2 && Q < 10) W_(Q, (Q > 2 && Q < 10 ? Q : 0));             \
+        else if (gb.Dg == Q - 1 && Q > 3) W_(Q, (Q > 3 ? Q - 1 : 0));                         \
+        else if (gb.Dg == Q - 2 && Q > 4 && ISO2) W_(Q, (Q > 4 && ISO2 ? Q - 2 : 0));         \
+        else W_(Q, 0);                                                                        \
+    }
 
 void geometric_factors(const Mesh &m, int q1d, double *X, double *J, double *detJ,
                        hipStream_t s) {
     H1PA_CHECK(q1d >= 1 && q1d <= 10, H1PA_EUNSUP, "q1d must be in [1,10]");
     const GeomBasis gb = make_geom_basis(q1d, m.node_order);
     const GeomLaunch l = geom_launch(m.ne, q1d, gb.Dg);
-#define X_(Q)                                                                                 \
-    if (q1d == Q) {                                                                           \
-        if (gb.Dg == 2)                                                                       \
-            hipLaunchKernelGGL((k_geometric_factors<Q, 2>), l.grid, l.block, l.lds, s,        \
-                               m.ne, l.nb, gb, m.d_nodes.p, X, J, detJ);                      \
-        else                                                                                  \
-            hipLaunchKernelGGL((k_geometric_factors<Q, 0>), l.grid, l.block, l.lds, s,        \
-                               m.ne, l.nb, gb, m.d_nodes.p, X, J, detJ);                      \
-    }
-    H1PA_FOR_EACH_Q(X_)
-#undef X_
+    const bool wp = X != nullptr;
+    constexpr bool ISO2 = true;
+#define K_(Q, WP, DG)                                                                         \
+    hipLaunchKernelGGL((k_geometric_factors<Q, WP, DG>), l.grid, l.block, l.lds, s, m.ne,     \
+                       l.nb, gb, m.d_nodes.p, X, J, detJ)
+    X_(1) X_(2) X_(3) X_(4) X_(5) X_(6) X_(7) X_(8) X_(9) X_(10)
+#undef K_
     H1PA_HIP(hipGetLastError());
 }
 
@@ -398,24 +408,11 @@ void pa_setup(const Mesh &m, const Form &f, hipStream_t s) {
     const bool wp = f.desc.coeff_kind == H1PA_COEFF_SINCOS ||
                     f.desc.coeff_kind == H1PA_COEFF_FOURIER;
     const GeomLaunch l = geom_launch(m.ne, q1d, gb.Dg);
+    constexpr bool ISO2 = false;
 #define K_(Q, WP, DG)                                                                         \
     hipLaunchKernelGGL((k_pa_setup<Q, WP, DG>), l.grid, l.block, l.lds, s, m.ne, l.nb,    \
                        gb, m.d_nodes.p, f.desc.coeff_kind, f.desc.coeff_value,          \
                        f.desc.d_coeff, fm, f.pa_diff.p, f.pa_mass.p)
-#define W_(Q, DG)                                                                             \
-    do {                                                                                      \
-        if (wp) K_(Q, true, DG);                                                              \
-        else K_(Q, false, DG);                                                                \
-    } while (0)
-    // geometry of the field's own order (q1d = Dg or Dg + 1) has its node count
-    // compiled in; other curved orders read it at run time
-#define X_(Q)                                                                                 \
-    if (q1d == Q) {                                                                           \
-        if (gb.Dg == 2) W_(Q, 2);                                                             \
-        else if (gb.Dg == Q && Q > 2 && Q < 10) W_(Q, (Q > 2 && Q < 10 ? Q : 0));             \
-        else if (gb.Dg == Q - 1 && Q > 3) W_(Q, (Q > 3 ? Q - 1 : 0));                         \
-        else W_(Q, 0);                                                                        \
-    }
     X_(2) X_(3) X_(4) X_(5) X_(6) X_(7) X_(8) X_(9) X_(10)
 #undef X_
 #undef W_

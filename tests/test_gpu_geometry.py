@@ -87,3 +87,31 @@ def test_domain_rhs_every_order(orc, h1pa, torch_cuda, p, g):
         ref = np.zeros(fes.GetNDofs())
         np.add.at(ref, gmap, np.ravel(orc.domain_lf(p, ne, g, X, **kw)))
         assert _rel(lf.Assemble().cpu().numpy(), ref) < RTOL
+
+
+@pytest.mark.parametrize("p", range(1, 9))
+@pytest.mark.parametrize("g", [1, 0])
+def test_physical_derivatives_every_rule(orc, h1pa, torch_cuda, p, g):
+    """Straight-sided (the Jacobian is formed with the field) and isoparametric
+    meshes, at every rule and both layouts.  The gradient multiplies by J^-T, of
+    condition number below 4 on these meshes: the bar of the factors times 4."""
+    M, dims, g = h1pa, (5, 3, 3), g or p
+    mesh, X = _nodes(orc, M, torch_cuda, dims, g, 1000 * p + g)
+    ne = int(np.prod(dims))
+    fes = M.FiniteElementSpace(mesh, M.H1_FECollection(p, 3))
+    flags = M.QI_VALUES | M.QI_PHYSICAL_DERIVATIVES
+    for q in range(p + 1, min(p + 3, 10) + 1):
+        J, _ = orc.geom(ne, g, q, X)
+        for vdim in (1, 3):
+            xE = np.random.default_rng(q).uniform(-1, 1, (p + 1) ** 3 * vdim * ne)
+            for layout in (0, 1):
+                qi = fes.GetQuadratureInterpolator(q, vdim)
+                qi.SetOutputLayout(layout)
+                val = torch_cuda.full((q ** 3 * vdim * ne,), np.nan, dtype=torch_cuda.float64,
+                                      device="cuda")
+                der = torch_cuda.full((3 * val.numel(),), np.nan, dtype=torch_cuda.float64,
+                                      device="cuda")
+                qi.Mult(torch_cuda.from_numpy(xE).cuda(), flags, val, der, None)
+                ref = orc.qinterp(p, q, vdim, ne, xE, flags, by_vdim=bool(layout), J=J)
+                assert _rel(val.cpu().numpy(), np.ravel(ref[0])) < RTOL
+                assert _rel(der.cpu().numpy(), np.ravel(ref[1])) < 4 * RTOL
