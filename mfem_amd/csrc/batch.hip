@@ -34,7 +34,7 @@
 #include <vector>
 
 #include "apply_body.hpp"
-#include "row_sum.hpp"
+#include "row_table.hpp"
 
 namespace h1pa {
 
@@ -57,14 +57,15 @@ struct SlotState {
 struct SlotDesc {
     const void *pa;        // inner PA data (FP64, FP32 or BF16)
     const double *pa64;    // FP64 PA data (refinement residual)
-    const int *gmap, *offsets, *indices, *perm, *l2n;
+    const int *gmap, *l2n;
+    RowTab rows;           // E -> L rows of the native E-vector
     const uint8_t *mask;
     const double *b;
     double *x;
     void *r, *z, *d, *dinv, *xi, *ye;  // inner vectors (type T of the batch); xi: FP64
                                        // mode the solution x, mixed the update xs
     double *r64, *dinv64, *ye64;       // mixed: FP64 residual, Jacobi, E-vector
-    int64_t ne, n, nperm;
+    int64_t ne, n;
     int64_t bb;                        // first row written directly by the element kernel
                                        // (interior DOFs; n when none)
     int part0, nchunks;
@@ -163,19 +164,47 @@ __device__ __forceinline__ Share share_of(int chunk, int64_t n) {
     return h;
 }
 
-// The DOFs of chunk tk.chunk that this thread owns (kPer of them, kT apart),
-// one after another (kernels whose DOFs branch on their kind).
-#define H1PA_CHUNK_LOOP(i)                                                                 \
-    for (int64_t i = (int64_t)tk.chunk * kChunk + threadIdx.x,                             \
-                 i##_end = min(sd.n, (int64_t)(tk.chunk + 1) * kChunk);                    \
-         i < i##_end; i += kT)
-
 // Descriptor pointer of type T as a global-memory pointer.
 template <typename T>
 __device__ __forceinline__ T *gv(void *p) { return global_ptr(reinterpret_cast<T *>(p)); }
 template <typename T>
 __device__ __forceinline__ const T *gv(const void *p) {
     return global_ptr(reinterpret_cast<const T *>(p));
+}
+
+// The slot's row table with its pointers marked as global memory.
+__device__ __forceinline__ RowTab slot_rows(const SlotDesc &sd) {
+    RowTab t = sd.rows;
+    t.tab = global_ptr(t.tab);
+    t.perm = global_ptr(t.perm);
+    if (t.over) {
+        t.offsets = global_ptr(t.offsets);
+        t.indices = global_ptr(t.indices);
+    }
+    return t;
+}
+
+// E -> L sums of the share's rows: v[k] = the row's sum for a position below
+// bb, z[ii[k]] (written by the element kernel) for an interior DOF.
+template <typename T>
+__device__ __forceinline__ void share_rows(const RowTab &tb, int64_t bb, const Share &h,
+                                           const int (&ii)[kPer], const T *ye, const T *z,
+                                           T (&v)[kPer]) {
+    const bool rows = __ballot(h.lt[0] < bb), inner = __ballot(h.lt[kPer - 1] >= bb);
+    T vz[kPer];
+    if (inner)
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) vz[k] = z[ii[k]];
+    if (rows) {
+        int t[kPer];
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) t[k] = (int)(h.lt[k] < bb ? h.lt[k] : bb - 1);
+        rows_sum<kPer>(tb, t, ye, v);
+    }
+    if (inner)
+#pragma unroll
+        for (int k = 0; k < kPer; ++k)
+            if (h.lt[k] >= bb) v[k] = vz[k];
 }
 
 // Producer kernels run one block per (slot, chunk) work item and skip the
@@ -335,18 +364,18 @@ kb_diffusion(const ElemTask *__restrict__ tasks, const SlotDesc *__restrict__ de
     __shared__ T smem[NB * diffusion_buf<D, Q>()];
     EOutT<T> out;
     out.l2n = global_ptr(sd.l2n);
-    if (sd.bb < sd.n) {  // interior DOFs straight to the L-vector (z, or r64 for RU)
-        out.yL = RU ? gv<T>(sd.r64) : gv<T>(sd.z);
-        out.bb = sd.bb;
-    }
+    out.ye = RU ? gv<T>(sd.ye64) : gv<T>(sd.ye);
+    // interior DOFs straight to the L-vector (z, or r64 for RU), or after the
+    // surface entries
+    const bool direct = sd.bb < sd.n;
+    out.yL = !direct ? out.ye : RU ? gv<T>(sd.r64) : gv<T>(sd.z);
+    out.bb = direct ? sd.bb : sd.rows.ebub;
     const int *gmap = global_ptr(sd.gmap);
     const uint8_t *mask = sd.mask ? global_ptr(sd.mask) : nullptr;
     if constexpr (RU) {
-        out.ye = gv<T>(sd.ye64);
         diffusion_elements<T, TP, D, Q, NB, U, K>(tk.e0, sd.ne, basis, gv<TP>(sd.pa64), gmap, mask,
                                                   gv<T>(sd.x), out, 0, smem);
     } else {
-        out.ye = gv<T>(sd.ye);
         diffusion_elements<T, TP, D, Q, NB, U, K>(tk.e0, sd.ne, basis, gv<TP>(sd.pa), gmap, mask,
                                                   gv<T>(sd.d), out, 0, smem);
     }
@@ -361,36 +390,28 @@ kb_scatter(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
     H1PA_TASK_PROLOGUE(ph_ == PH_INNER)
     const T *ye = gv<const T>(sd.ye), *d = gv<const T>(sd.d);
     T *z = gv<T>(sd.z);
-    const int *perm = sd.perm ? global_ptr(sd.perm) : nullptr;
-    const int *off = global_ptr(sd.offsets), *ind = global_ptr(sd.indices);
     const uint8_t *mask = sd.mask ? global_ptr(sd.mask) : nullptr;
-    // the share's rows, then their offsets, masks and d values, as batches
+    const RowTab tb = slot_rows(sd);
     const Share h = share_of(tk.chunk, sd.n);
-    int64_t ii[kPer];
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) ii[k] = h.lt[k] < sd.nperm ? perm[h.lt[k]] : h.lt[k];
-    T vd[kPer];
-    int ob[kPer], oe[kPer];
+    int ii[kPer];
+    T vd[kPer], v[kPer];
     bool m[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
+        ii[k] = row_dof(tb, (int)h.lt[k]);
         vd[k] = d[ii[k]];
-        ob[k] = off[ii[k]];
-        oe[k] = off[ii[k] + 1];
         m[k] = mask && mask[ii[k]];
     }
+    share_rows(tb, sd.bb, h, ii, ye, z, v);
     double acc[1] = {0.0};
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
         if (!h.ok[k]) continue;
-        T v;
-        if (h.t[k] >= sd.bb) {  // interior DOF: written by the element kernel
-            v = z[ii[k]];
-        } else {
-            v = m[k] ? vd[k] : row_sum(ind, ob[k], oe[k], ye);
-            z[ii[k]] = v;
+        if (h.t[k] < sd.bb) {
+            v[k] = m[k] ? vd[k] : v[k];
+            z[ii[k]] = v[k];
         }
-        acc[0] += (double)vd[k] * (double)v;
+        acc[0] += (double)vd[k] * (double)v[k];
     }
     store_chunk<1>(acc, sd, tk.chunk, partials, sh);
 }
@@ -604,25 +625,31 @@ kbm_ru_res(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
     H1PA_TASK_PROLOGUE(ph_ == PH_RU)
     float *r = vp<float>(sd.r), *z = vp<float>(sd.z);
     const float *dinv = vp<float>(sd.dinv);
+    const double *b = sd.b, *x = sd.x, *dinv64 = sd.dinv64, *ye64 = sd.ye64;
+    double *r64 = sd.r64;
+    const uint8_t *mask = sd.mask;
+    const RowTab tb = slot_rows(sd);
+    const Share h = share_of(tk.chunk, sd.n);
+    int ii[kPer];
+    double v[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) ii[k] = row_dof(tb, (int)h.lt[k]);
+    // interior DOFs: (A x)_i was written into r64 by the element kernel
+    share_rows(tb, sd.bb, h, ii, ye64, r64, v);
     double acc[3] = {0.0, 0.0, 0.0};
-    H1PA_CHUNK_LOOP(t) {
-        const int64_t i = t < sd.nperm ? sd.perm[t] : t;
-        double y;
-        if (t >= sd.bb) {  // interior DOF: (A x)_i written into r64 by the element kernel
-            y = sd.r64[i];
-        } else if (sd.mask && sd.mask[i]) {
-            y = sd.x[i];
-        } else {
-            y = row_sum(sd.indices, sd.offsets[i], sd.offsets[i + 1], sd.ye64);
-        }
-        const double ri = sd.b[i] - y;
-        sd.r64[i] = ri;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        if (!h.ok[k]) continue;
+        const int64_t i = ii[k];
+        const double y = (h.t[k] < sd.bb && mask && mask[i]) ? x[i] : v[k];
+        const double ri = b[i] - y;
+        r64[i] = ri;
         const float rf = (float)ri;
         const float zf = dinv[i] * rf;
         r[i] = rf;
         z[i] = zf;
         acc[0] += (double)rf * (double)zf;
-        acc[1] += ri * sd.dinv64[i] * ri;
+        acc[1] += ri * dinv64[i] * ri;
         acc[2] += ri * ri;
     }
     store_chunk<3>(acc, sd, tk.chunk, partials, sh);
@@ -1130,10 +1157,7 @@ int batch_add(Batch &B, h1pa_form *form, const uint8_t *mask_src, const double *
     }
     SlotDesc &d = sl->desc;
     d.gmap = sp.restr.gather_map.p;
-    d.offsets = sp.restr.offsets.p;
-    d.indices = sp.restr.indices_nat.p;
-    d.perm = sp.restr.perm.p;
-    d.nperm = sp.restr.nperm;
+    d.rows = sp.restr.rows();
     d.l2n = sp.restr.lex2nat.p;
     d.mask = sl->mask.p;
     d.b = b;

@@ -268,10 +268,8 @@ int h1pa_space_create(h1pa_mesh *mesh, int order, h1pa_space **space) {
             std::vector<int> dm(s.dof);
             h1_dof_map(order, dm.data());  // lex -> native
             r.lex2nat.upload(dm.data(), dm.size(), st);
-            r.indices_nat.alloc(s.ne * s.dof);
-            kern::native_indices(s.ne * s.dof, (int)s.dof, r.indices.p, r.lex2nat.p,
-                                 r.indices_nat.p, st);
-            H1PA_HIP(hipStreamSynchronize(st));
+            r.nedofs = s.nedofs;
+            kern::build_row_table(r, st);
         }
         auto *rh = new h1pa_restriction();
         rh->owned_by_space = true;
@@ -524,10 +522,8 @@ void autotune_diffusion(Form &f, hipStream_t s) {
     kern::EOut out;
     out.ye = f.ework0.p;
     out.l2n = sp.restr.lex2nat.p;
-    if (sp.restr.bubble_begin < sp.ndofs) {
-        out.yL = x.p + sp.ndofs;
-        out.bb = sp.restr.bubble_begin;
-    }
+    out.yL = x.p + sp.ndofs;
+    out.bb = sp.restr.bubble_begin;
     // three interleaved rounds (1 warm-up + 4 timed launches per variant each),
     // so that a drift of the clock or of the other work on the device does
     // not pick the variant that happened to run in a quiet moment
@@ -608,7 +604,7 @@ void require_assembled(const Form &f) {
 // E-part of the operator: ework0 = sum of integrators applied to x.  `gmap`
 // null means x is already an E-vector.
 // yL != nullptr selects the fused layout: bubble DOFs straight into yL and
-// the other E-entries in native order (read back through indices_nat).
+// the other E-entries in native order (read back through the row table).
 void element_apply(Form &f, const int *gmap, const uint8_t *mask, const double *x, double *ye,
                    double *yL, bool accumulate, hipStream_t s) {
     kern::EOut out;
@@ -745,9 +741,7 @@ void h1pa::operator_diagonal(Form &f, double *diag, hipStream_t s) {
     out.l2n = sp.restr.lex2nat.p;
     if (diff) kern::diffusion_diagonal(sp.p, f.q1d, sp.ne, f.basis.p, f.pa_diff.p, out, false, s);
     if (mass) kern::mass_diagonal(sp.p, f.q1d, sp.ne, f.basis.p, f.pa_mass.p, out, diff, s);
-    kern::restrict_mult_transpose(sp.restr.bubble_begin, sp.restr.offsets.p,
-                                  sp.restr.indices_nat.p, f.ework0.p, diag, 2, sp.restr.perm.p,
-                                  sp.restr.nperm, s);
+    kern::scatter_rows(sp.restr, sp.restr.bubble_begin, f.ework0.p, nullptr, nullptr, diag, s);
 }
 
 int64_t h1pa::form_device_bytes(const Form &f) {
@@ -759,7 +753,7 @@ int64_t h1pa::form_device_bytes(const Form &f) {
     b += f.pa_diff_lp.n * 4 + f.pa_mass_lp.n * 4 + f.ework32.n * 4;
     const Restriction &r = sp.restr;
     b += (r.gather_map.n + r.offsets.n + r.indices.n + r.perm.n + r.perm_lex.n + r.lex2nat.n +
-          r.indices_nat.n) * 4;
+          r.indices_nat.n + r.row_tab.n) * 4;
     b += (sp.elem_dof.n + sp.ess.n) * 4 + sp.ess_mask.n;
     b += m.d_nodes.n * 8 + m.d_topo.n * 4 + m.d_ori.n + m.d_elem_at.n * 4;
     return b;
@@ -782,9 +776,7 @@ int h1pa_form_mult(h1pa_form *form, const double *x, double *y, void *stream) {
                                 f.iface.p, 3, s);
     } else {
         element_apply(f, sp.restr.gather_map.p, nullptr, x, f.ework0.p, y, false, s);
-        kern::restrict_mult_transpose(sp.restr.bubble_begin, sp.restr.offsets.p,
-                                      sp.restr.indices_nat.p, f.ework0.p, y, 0, sp.restr.perm.p,
-                                      sp.restr.nperm, s);
+        kern::scatter_rows(sp.restr, sp.restr.bubble_begin, f.ework0.p, nullptr, nullptr, y, s);
     }
     API_END
 }
@@ -802,9 +794,7 @@ int h1pa_form_add_mult(h1pa_form *form, const double *x, double *y, double a, vo
                                 f.lwork0.p, f.iface.p, 3, s);
     } else {
         element_apply(f, sp.restr.gather_map.p, nullptr, x, f.ework0.p, f.lwork0.p, false, s);
-        kern::restrict_mult_transpose(sp.restr.bubble_begin, sp.restr.offsets.p,
-                                      sp.restr.indices_nat.p, f.ework0.p, f.lwork0.p, 0,
-                                      sp.restr.perm.p, sp.restr.nperm, s);
+        kern::scatter_rows(sp.restr, sp.restr.bubble_begin, f.ework0.p, nullptr, nullptr, f.lwork0.p, s);
     }
     kern::axpy(sp.ndofs, a, f.lwork0.p, y, s);
     API_END
@@ -859,9 +849,7 @@ int h1pa_form_mult_noalloc(h1pa_form *form, const double *x, double *y, void *st
     // the element path of h1pa_form_mult, with its E-vector in the scratch:
     // every E-entry the scatter reads is written first (accumulate = false)
     element_apply(f, sp.restr.gather_map.p, nullptr, x, ye, y, false, s);
-    kern::restrict_mult_transpose(sp.restr.bubble_begin, sp.restr.offsets.p,
-                                  sp.restr.indices_nat.p, ye, y, 0, sp.restr.perm.p,
-                                  sp.restr.nperm, s);
+    kern::scatter_rows(sp.restr, sp.restr.bubble_begin, ye, nullptr, nullptr, y, s);
     API_END
 }
 
@@ -889,9 +877,7 @@ int h1pa_form_mult_timed(h1pa_form *form, const double *x, double *y, int steps,
                 kern::diffusion_columns(sp.p, f.cols, f.basis.p, f.pa_diff.p,
                                         sp.restr.gather_map.p, x, y, f.iface.p, 2, s);
             else
-                kern::restrict_mult_transpose(sp.restr.bubble_begin, sp.restr.offsets.p,
-                                              sp.restr.indices_nat.p, f.ework0.p, y, 0,
-                                              sp.restr.perm.p, sp.restr.nperm, s);
+                kern::scatter_rows(sp.restr, sp.restr.bubble_begin, f.ework0.p, nullptr, nullptr, y, s);
             H1PA_HIP(hipEventRecord(ev[3 * k + 2], s));
         }
         H1PA_HIP(hipEventSynchronize(ev.back()));
@@ -974,10 +960,11 @@ int h1pa_form_constrained_mult(h1pa_form *form, const int *d_ess, int64_t n_ess,
     // interior DOFs go straight to y unless the constraint list may hold some
     const bool direct = !mask || mask == sp.ess_mask.p;
     element_apply(f, sp.restr.gather_map.p, mask, x, f.ework0.p, direct ? y : nullptr, false, s);
-    kern::scatter_constrained(direct ? sp.restr.bubble_begin : sp.ndofs, sp.restr.offsets.p,
-                              direct ? sp.restr.indices_nat.p : sp.restr.indices.p, f.ework0.p,
-                              mask, x, y, direct ? sp.restr.perm.p : sp.restr.perm_lex.p,
-                              direct ? sp.restr.nperm : sp.restr.nperm_lex, s);
+    if (direct)
+        kern::scatter_rows(sp.restr, sp.restr.bubble_begin, f.ework0.p, mask, x, y, s);
+    else
+        kern::scatter_constrained(sp.ndofs, sp.restr.offsets.p, sp.restr.indices.p, f.ework0.p,
+                                  mask, x, y, sp.restr.perm_lex.p, sp.restr.nperm_lex, s);
     API_END
 }
 
@@ -1001,9 +988,7 @@ int h1pa_form_linear_system(h1pa_form *form, const int *d_ess, int64_t n_ess, co
     StreamBuf<double> z(sp.ndofs, s);
     kern::form_x(sp.ndofs, mask, x, X, s);  // X = x on ess, 0 elsewhere (= w)
     element_apply(f, sp.restr.gather_map.p, nullptr, X, f.ework0.p, z.p, false, s);
-    kern::restrict_mult_transpose(sp.restr.bubble_begin, sp.restr.offsets.p,
-                                  sp.restr.indices_nat.p, f.ework0.p, z.p, 0, sp.restr.perm.p,
-                                  sp.restr.nperm, s);
+    kern::scatter_rows(sp.restr, sp.restr.bubble_begin, f.ework0.p, nullptr, nullptr, z.p, s);
     kern::form_b(sp.ndofs, mask, X, b, z.p, B, s);
     H1PA_HIP(hipStreamSynchronize(s));
     API_END
@@ -1042,9 +1027,7 @@ int h1pa_space_domain_lf_qf(h1pa_space *space, double fval, const double *d_fq, 
     out.bb = sp.restr.bubble_begin;
     out.l2n = sp.restr.lex2nat.p;
     kern::domain_lf(*sp.mesh, sp.p, fval, d_fq, out, s);
-    kern::restrict_mult_transpose(sp.restr.bubble_begin, sp.restr.offsets.p,
-                                  sp.restr.indices_nat.p, bE.p, b, 0, sp.restr.perm.p,
-                                  sp.restr.nperm, s);
+    kern::scatter_rows(sp.restr, sp.restr.bubble_begin, bE.p, nullptr, nullptr, b, s);
     H1PA_HIP(hipStreamSynchronize(s));
     API_END
 }

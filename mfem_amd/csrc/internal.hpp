@@ -190,6 +190,19 @@ struct ColumnGrid {
 };
 
 // ---- restriction -----------------------------------------------------------
+// Device view of an H1 space's E -> L rows on native-order E-vectors
+// (row_table.hpp): positions [0, ebeg) vertex DOFs in the order perm, [ebeg,
+// fbeg) edge DOFs, [fbeg, bbeg) face DOFs, from bbeg on the nb interior DOFs of
+// each element.  tab: 8, 4 and 2 native E-indices a row, -1 past its entries.
+struct RowTab {
+    const int *tab = nullptr, *perm = nullptr;
+    int ebeg = 0, fbeg = 0, bbeg = 0;  // a space has below 2^31 DOFs and E-entries
+    int es = 0, nb = 0;  // surface entries and interior DOFs of an element
+    int64_t ebub = 0;    // interior entries of a native E-vector that holds them
+    int over = 0;  // some rows are wider than their kind: offsets, indices (native)
+    const int *offsets = nullptr, *indices = nullptr;
+};
+
 struct Restriction {
     int64_t ne = 0, dof = 0, ndofs = 0;
     DevBuf<int> gather_map, offsets, indices;
@@ -210,8 +223,19 @@ struct Restriction {
     // Internal E-vector layout of the fused operator: per element in native
     // (vertex, edge, face, bubble) order, so the entries of one edge or face
     // are contiguous for the E->L pass.  lex2nat[lex] = native position;
-    // indices_nat = indices re-addressed to that layout (same order).
-    DevBuf<int> lex2nat, indices_nat;
+    // row_tab: the rows' indices into that layout (row_table.hpp);
+    // indices_nat = indices re-addressed to that layout (same order), kept
+    // when the table leaves rows to it (row_over).
+    DevBuf<int> lex2nat, indices_nat, row_tab;
+    int64_t nedofs = 0;  // edge DOFs, after the nperm vertex DOFs
+    // Native layout: the surface entries of all elements, then (only where the
+    // element kernels do not write them to an L-vector) the interior entries.
+    int64_t interior() const {
+        return ne > 0 && ndofs > bubble_begin ? (ndofs - bubble_begin) / ne : 0;
+    }
+    int64_t native_bubble() const { return ne * (dof - interior()); }
+    int row_over = 0;
+    RowTab rows() const;
 };
 
 struct Space {
@@ -272,8 +296,18 @@ void list_to_mask(const int *list, int64_t nlist, uint8_t *mask, int64_t n, hipS
 
 void restrict_mult(int64_t nE, const int *gmap, const double *x, double *y, bool abs_,
                    hipStream_t s);
-// indices_nat[j] = indices[j] with E-index e*dof + lex moved to e*dof + lex2nat[lex].
-void native_indices(int64_t nE, int dof, const int *indices, const int *lex2nat, int *out,
+// Fills r.row_tab (and r.indices_nat, r.row_over) of an H1 space's restriction
+// from its CSR table, lex2nat, perm and nedofs.
+void build_row_table(Restriction &r, hipStream_t s);
+// E -> L on a native-order E-vector over row positions [0, nrows): y = sum of
+// the row, or with a mask y[i] = mask[i] ? xin[i] : sum (DIAG_ONE).
+void scatter_rows(const Restriction &r, int64_t nrows, const double *ye, const uint8_t *mask,
+                  const double *xin, double *y, hipStream_t s);
+void scatter_rows(const Restriction &r, int64_t nrows, const float *ye, const uint8_t *mask,
+                  const float *xin, float *y, hipStream_t s);
+// indices_nat[j] = indices[j] with E-index e*dof + lex moved to its place in the
+// native layout (surface entries; es of them an element).
+void native_indices(int64_t nE, int dof, int es, const int *indices, const int *lex2nat, int *out,
                     hipStream_t s);
 // First-contribution order of the L-DOFs [0, nv): perm[k] = k-th vertex DOF.
 void first_contribution_order(int64_t nE, const int *gmap, const int *offsets,
@@ -324,8 +358,8 @@ void randomize(int64_t n, double *x, uint64_t seed, double lo, double hi, hipStr
 // E->E: ye = A_E xe (overwrite) or += ; x may be gathered from an L-vector
 // through gmap (gmap != nullptr) with constrained entries masked to zero.
 // basis = [B q-fastest | G q-fastest | B d-fastest | G d-fastest], 4*Q*D doubles.
-// Output of an element kernel: the E-vector ye (lexicographic, or native
-// order when l2n != nullptr) and, when yL != nullptr, interior (bubble) DOFs
+// Output of an element kernel: the E-vector ye (lexicographic, or the surface
+// entries in native order when l2n != nullptr) and, when yL != nullptr, interior (bubble) DOFs
 // written straight to the L-vector yL at MFEM's bubble block starting at bb.
 template <typename T>
 struct EOutT {

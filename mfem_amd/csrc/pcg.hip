@@ -28,7 +28,7 @@
 #include <stdlib.h>
 
 #include "internal.hpp"
-#include "row_sum.hpp"
+#include "row_table.hpp"
 
 namespace h1pa {
 
@@ -97,6 +97,42 @@ __device__ __forceinline__ Grp grp_of(int64_t b, int64_t end) {
                  g##_e = min((int64_t)(n), (int64_t)(blockIdx.x + 1) * kThreads * per);        \
          g##_b < g##_e; g##_b += (int64_t)kGrp * kThreads)                                     \
         for (const Grp g = grp_of(g##_b, g##_e), *g##_1 = &g; g##_1; g##_1 = nullptr)
+
+// E -> L sums of the group's rows (positions g.lt): v[k] = the row's sum for a
+// position below bb, z[ii[k]] (written by the element kernel) for an interior
+// DOF.  A wave of interior DOFs alone reads no row.
+template <typename T>
+__device__ __forceinline__ void group_rows(const RowTab &tb, int64_t bb, int per, const Grp &g,
+                                           const int (&ii)[kGrp], const T *__restrict__ ye,
+                                           const T *z, T (&v)[kGrp]) {
+    const bool rows = __ballot(g.lt[0] < bb), inner = __ballot(g.lt[kGrp - 1] >= bb);
+    T vz[kGrp];
+    if (inner)
+#pragma unroll
+        for (int k = 0; k < kGrp; ++k)
+            if (k < per) vz[k] = z[ii[k]];
+    if (rows) {
+        int t[kGrp];
+#pragma unroll
+        for (int k = 0; k < kGrp; ++k) t[k] = (int)(g.lt[k] < bb ? g.lt[k] : bb - 1);
+        if (per >= kGrp) {
+            rows_sum<kGrp>(tb, t, ye, v);
+        } else {
+#pragma unroll
+            for (int k = 0; k < kGrp; ++k) {
+                if (k >= per) break;
+                const int t1[1] = {t[k]};
+                T v1[1];
+                rows_sum<1>(tb, t1, ye, v1);
+                v[k] = v1[0];
+            }
+        }
+    }
+    if (inner)
+#pragma unroll
+        for (int k = 0; k < kGrp; ++k)
+            if (k < per && g.lt[k] >= bb) v[k] = vz[k];
+}
 
 // Block sum in a fixed tree order, returned to every thread.
 __device__ inline double block_sum(double v, double *sh) {
@@ -218,44 +254,32 @@ k_pcg_fin_init(int nb, const double *__restrict__ partials, PcgState *st, double
 // z = A d from the element output, DIAG_ONE rows copy d; partials of (d, z).
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
-k_pcg_scatter(int64_t n, int per, int64_t bb, const int *__restrict__ offsets,
-              const int *__restrict__ indices, const T *__restrict__ ye,
+k_pcg_scatter(int64_t n, int per, int64_t bb, RowTab tb, const T *__restrict__ ye,
               const uint8_t *__restrict__ mask, const T *__restrict__ d, T *__restrict__ z,
-              double *__restrict__ partials, const PcgState *st, const int *__restrict__ perm,
-              int64_t nperm) {
+              double *__restrict__ partials, const PcgState *st) {
     __shared__ double sh[kThreads];
     if (st->done) return;
     double acc[1] = {0.0};
     H1PA_GROUPS(g, n) {
-        // the group's rows, then their offsets, masks and d values, as batches
-        int64_t ii[kGrp];
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (k >= per) break;  // past this thread's entries
-            ii[k] = g.lt[k] < nperm ? perm[g.lt[k]] : g.lt[k];
-        }
-        T vd[kGrp];
-        int ob[kGrp], oe[kGrp];
+        int ii[kGrp];
+        T vd[kGrp], v[kGrp];
         bool m[kGrp];
 #pragma unroll
         for (int k = 0; k < kGrp; ++k) {
             if (k >= per) break;  // past this thread's entries
+            ii[k] = row_dof(tb, (int)g.lt[k]);
             vd[k] = d[ii[k]];
-            ob[k] = offsets[ii[k]];
-            oe[k] = offsets[ii[k] + 1];
             m[k] = mask && mask[ii[k]];
         }
+        group_rows(tb, bb, per, g, ii, ye, z, v);
 #pragma unroll
         for (int k = 0; k < kGrp; ++k) {
             if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
-            T v;
-            if (g.t[k] >= bb) {  // interior DOF: written by the element kernel
-                v = z[ii[k]];
-            } else {
-                v = m[k] ? vd[k] : row_sum(indices, ob[k], oe[k], ye);
+            if (g.t[k] < bb) {
+                v[k] = m[k] ? vd[k] : v[k];
+                z[ii[k]] = v[k];
             }
-            if (g.t[k] < bb) z[ii[k]] = v;
-            acc[0] += (double)vd[k] * (double)v;
+            acc[0] += (double)vd[k] * (double)v[k];
         }
     }
     store_partials<1>(acc, partials, sh);
@@ -386,17 +410,6 @@ __global__ void k_to_bf16(int64_t n, const double *__restrict__ a, uint16_t *__r
     b[i] = h;
 }
 
-// E->L set over all rows in reduced precision (no constraints).
-template <typename T>
-__global__ void k_scatter_set(int64_t n, const int *__restrict__ offsets,
-                              const int *__restrict__ indices, const T *__restrict__ ye,
-                              T *__restrict__ y, const int *__restrict__ perm, int64_t nperm) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int64_t i = t < nperm ? perm[t] : t;
-    y[i] = row_sum(indices, offsets[i], offsets[i + 1], ye);
-}
-
 // ---- mixed precision: CG with reliable updates -----------------------------
 // The FP32 inner CG runs on its recursive residual r and accumulates its
 // solution in xs.  Whenever the preconditioned norm (r, z) has fallen by
@@ -470,43 +483,32 @@ k_ir_fin_init(int nb, const double *__restrict__ partials, IrState *st) {
 
 // q = A d (FP32; DIAG_ONE rows copy d), partials of (d, q).
 __global__ void __launch_bounds__(kThreads)
-k_ir_scatter(int64_t n, int per, int64_t bb, const int *__restrict__ offsets,
-             const int *__restrict__ indices, const float *__restrict__ ye,
+k_ir_scatter(int64_t n, int per, int64_t bb, RowTab tb, const float *__restrict__ ye,
              const uint8_t *__restrict__ mask, const float *__restrict__ d,
-             float *__restrict__ q, double *__restrict__ partials, const IrState *st,
-             const int *__restrict__ perm, int64_t nperm) {
+             float *__restrict__ q, double *__restrict__ partials, const IrState *st) {
     __shared__ double sh[kThreads];
     if (st->done) return;
     double acc[1] = {0.0};
     H1PA_GROUPS(g, n) {
-        int64_t ii[kGrp];
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (k >= per) break;  // past this thread's entries
-            ii[k] = g.lt[k] < nperm ? perm[g.lt[k]] : g.lt[k];
-        }
-        float vd[kGrp];
-        int ob[kGrp], oe[kGrp];
+        int ii[kGrp];
+        float vd[kGrp], v[kGrp];
         bool m[kGrp];
 #pragma unroll
         for (int k = 0; k < kGrp; ++k) {
             if (k >= per) break;  // past this thread's entries
+            ii[k] = row_dof(tb, (int)g.lt[k]);
             vd[k] = d[ii[k]];
-            ob[k] = offsets[ii[k]];
-            oe[k] = offsets[ii[k] + 1];
             m[k] = mask && mask[ii[k]];
         }
+        group_rows(tb, bb, per, g, ii, ye, q, v);
 #pragma unroll
         for (int k = 0; k < kGrp; ++k) {
             if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
-            float v;
-            if (g.t[k] >= bb) {  // interior DOF: written by the element kernel
-                v = q[ii[k]];
-            } else {
-                v = m[k] ? vd[k] : row_sum(indices, ob[k], oe[k], ye);
+            if (g.t[k] < bb) {
+                v[k] = m[k] ? vd[k] : v[k];
+                q[ii[k]] = v[k];
             }
-            if (g.t[k] < bb) q[ii[k]] = v;
-            acc[0] += (double)vd[k] * (double)v;
+            acc[0] += (double)vd[k] * (double)v[k];
         }
     }
     store_partials<1>(acc, partials, sh);
@@ -606,36 +608,39 @@ k_ir_ru_x(int64_t n, float *__restrict__ xs, double *__restrict__ x, const IrSta
 // r64 = b - A x; partials of (B r64, r64), ||r64||^2 and, with
 // r = (float) r64, z = dinv r, of (r, z).
 __global__ void __launch_bounds__(kThreads)
-k_ir_ru_res(int64_t n, int per, int64_t bb, const int *__restrict__ offsets,
-            const int *__restrict__ indices, const double *__restrict__ ye64,
-            const uint8_t *__restrict__ mask,
-            const double *__restrict__ b, const double *__restrict__ x,
-            const double *__restrict__ dinv64, const float *__restrict__ dinv,
-            double *__restrict__ r64, float *__restrict__ r, float *__restrict__ z,
-            double *__restrict__ partials, const IrState *st, const int *__restrict__ perm,
-            int64_t nperm) {
+k_ir_ru_res(int64_t n, int per, int64_t bb, RowTab tb, const double *__restrict__ ye64,
+            const uint8_t *__restrict__ mask, const double *__restrict__ b,
+            const double *__restrict__ x, const double *__restrict__ dinv64,
+            const float *__restrict__ dinv, double *__restrict__ r64, float *__restrict__ r,
+            float *__restrict__ z, double *__restrict__ partials, const IrState *st) {
     __shared__ double sh[kThreads];
     if (!st->ru) return;
     double acc[3] = {0.0, 0.0, 0.0};
-    H1PA_CHUNK(t, n) {
-        const int64_t i = t < nperm ? perm[t] : t;
-        double y;
-        if (t >= bb) {  // interior DOF: (A x)_i written into r64 by the element kernel
-            y = r64[i];
-        } else if (mask && mask[i]) {
-            y = x[i];
-        } else {
-            y = row_sum(indices, offsets[i], offsets[i + 1], ye64);
+    H1PA_GROUPS(g, n) {
+        int ii[kGrp];
+        double v[kGrp];
+#pragma unroll
+        for (int k = 0; k < kGrp; ++k) {
+            if (k >= per) break;  // past this thread's entries
+            ii[k] = row_dof(tb, (int)g.lt[k]);
         }
-        const double ri = b[i] - y;
-        r64[i] = ri;
-        const float rf = (float)ri;
-        const float zf = dinv[i] * rf;
-        r[i] = rf;
-        z[i] = zf;
-        acc[0] += (double)rf * (double)zf;
-        acc[1] += ri * dinv64[i] * ri;
-        acc[2] += ri * ri;
+        // interior DOFs: (A x)_i was written into r64 by the element kernel
+        group_rows(tb, bb, per, g, ii, ye64, r64, v);
+#pragma unroll
+        for (int k = 0; k < kGrp; ++k) {
+            if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
+            const int64_t i = ii[k];
+            const double y = (g.t[k] < bb && mask && mask[i]) ? x[i] : v[k];
+            const double ri = b[i] - y;
+            r64[i] = ri;
+            const float rf = (float)ri;
+            const float zf = dinv[i] * rf;
+            r[i] = rf;
+            z[i] = zf;
+            acc[0] += (double)rf * (double)zf;
+            acc[1] += ri * dinv64[i] * ri;
+            acc[2] += ri * ri;
+        }
     }
     store_partials<3>(acc, partials, sh);
 }
@@ -717,39 +722,30 @@ k_cheb_first(int64_t n, int per, const double *__restrict__ dinv, const double *
 // k >= 1: u = A t (constrained: interior rows written by the element kernel
 // into u, DIAG_ONE rows copy t); t = u * dinv; y += ck t
 __global__ void __launch_bounds__(kThreads)
-k_cheb_scatter(int64_t n, int per, int64_t bb, const int *__restrict__ offsets,
-               const int *__restrict__ indices, const double *__restrict__ ye,
+k_cheb_scatter(int64_t n, int per, int64_t bb, RowTab tb, const double *__restrict__ ye,
                const uint8_t *__restrict__ mask, const double *__restrict__ dinv,
                const double *__restrict__ u, double *__restrict__ t, double *__restrict__ y,
-               double ck, const int *stop, const int *__restrict__ perm, int64_t nperm) {
+               double ck, const int *stop) {
     if (stop && *stop) return;
     H1PA_GROUPS(g, n) {
-        int64_t ii[kGrp];
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (k >= per) break;  // past this thread's entries
-            ii[k] = g.lt[k] < nperm ? perm[g.lt[k]] : g.lt[k];
-        }
-        double vi[kGrp], vy[kGrp], vt[kGrp];
-        int ob[kGrp], oe[kGrp];
+        int ii[kGrp];
+        double vi[kGrp], vy[kGrp], vt[kGrp], v[kGrp];
         bool m[kGrp];
 #pragma unroll
         for (int k = 0; k < kGrp; ++k) {
             if (k >= per) break;  // past this thread's entries
+            ii[k] = row_dof(tb, (int)g.lt[k]);
             vi[k] = dinv[ii[k]];
             vy[k] = y[ii[k]];
             vt[k] = t[ii[k]];
-            ob[k] = offsets[ii[k]];
-            oe[k] = offsets[ii[k] + 1];
             m[k] = mask && mask[ii[k]];
         }
+        group_rows(tb, bb, per, g, ii, ye, u, v);
 #pragma unroll
         for (int k = 0; k < kGrp; ++k) {
             if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
-            double v;
-            if (g.t[k] >= bb) v = u[ii[k]];
-            else v = m[k] ? vt[k] : row_sum(indices, ob[k], oe[k], ye);
-            const double ti = v * vi[k];
+            if (g.t[k] < bb && m[k]) v[k] = vt[k];
+            const double ti = v[k] * vi[k];
             t[ii[k]] = ti;
             y[ii[k]] = vy[k] + ck * ti;
         }
@@ -945,7 +941,7 @@ void form_b(int64_t n, const uint8_t *mask, const double *X, const double *b, co
 namespace {
 
 // Element part of the constrained apply, d -> A_E d, E-vector in native
-// order (read back through indices_nat); with yL, the interior DOFs go
+// order (read back through the row table); with yL, the interior DOFs go
 // straight to yL.  Stops early once `stop` is set.
 
 // Interior DOFs may bypass the E-vector when no constrained DOF is interior:
@@ -963,10 +959,9 @@ void pcg_element_apply(Form &f, int prec, const uint8_t *mask, const T *d, T *ye
     out.ye = ye;
     out.l2n = sp.restr.lex2nat.p;
     out.stop = stop;
-    if (yL) {  // interior DOFs straight to the L-vector
-        out.yL = yL;
-        out.bb = sp.restr.bubble_begin;
-    }
+    // interior DOFs straight to the L-vector, or after the surface entries
+    out.yL = yL ? yL : ye;
+    out.bb = yL ? sp.restr.bubble_begin : sp.restr.native_bubble();
     if constexpr (sizeof(T) == 8) {
         // FP64 vectors; prec = BF16_PA takes the diffusion PA data from the
         // form's BF16 shadow (the applies of a mixed-precision cycle)
@@ -1053,9 +1048,8 @@ void pcg_run(Form &f, int prec, const uint8_t *mask, const T *dinv, const T *b, 
     const int64_t bb = direct_rows(sp, mask);
     auto apply = [&]() {
         pcg_element_apply<T>(f, prec, mask, d, ye, bb < n ? z : nullptr, stop, s);
-        hipLaunchKernelGGL(kern::k_pcg_scatter<T>, grid, blk, 0, s, n, per, bb, sp.restr.offsets.p,
-                           sp.restr.indices_nat.p, ye, mask, d, z, partials, st,
-                           sp.restr.perm.p, sp.restr.nperm);
+        hipLaunchKernelGGL(kern::k_pcg_scatter<T>, grid, blk, 0, s, n, per, bb, sp.restr.rows(), ye,
+                           mask, d, z, partials, st);
         hipLaunchKernelGGL(kern::k_pcg_fin_den, one, blk, 0, s, (int)nb, partials, st);
     };
     apply();
@@ -1117,6 +1111,8 @@ void autotune_lp(Form &f, int kind, hipStream_t s) {
     kern::EOutT<float> out;
     out.ye = f.ework32.p;
     out.l2n = sp.restr.lex2nat.p;
+    out.yL = f.ework32.p;
+    out.bb = sp.restr.native_bubble();
     int best = 0;
     float best_ms = 1e30f;
     for (int v : {0, 1, 4, 5, 6, 7, 8}) {
@@ -1192,11 +1188,8 @@ void ensure_low_precision(Form &f, int precision, hipStream_t s) {
 void form_mult_lp(Form &f, int precision, const float *x, float *y, hipStream_t s) {
     ensure_low_precision(f, precision, s);
     Space &sp = *f.space;
-    pcg_element_apply<float>(f, precision, nullptr, x, f.ework32.p, nullptr, nullptr, s);
-    hipLaunchKernelGGL(kern::k_scatter_set<float>, dim3((unsigned)((sp.ndofs + 255) / 256)),
-                       dim3(256), 0, s, sp.ndofs, sp.restr.offsets.p, sp.restr.indices_nat.p,
-                       f.ework32.p, y, sp.restr.perm.p, sp.restr.nperm);
-    H1PA_HIP(hipGetLastError());
+    pcg_element_apply<float>(f, precision, nullptr, x, f.ework32.p, y, nullptr, s);
+    kern::scatter_rows(sp.restr, sp.restr.bubble_begin, f.ework32.p, nullptr, nullptr, y, s);
 }
 
 void pcg_solve(Form &f, const uint8_t *mask, const double *diag, const double *b, double *x,
@@ -1221,8 +1214,7 @@ void constrained_apply(Form &f, const uint8_t *mask, const double *v, double *u,
     const int64_t bb = direct_rows(sp, mask);
     pcg_element_apply<double>(f, prec, mask, v, f.ework0.p, bb < sp.ndofs ? u : nullptr, stop,
                               s);
-    kern::scatter_constrained(bb, sp.restr.offsets.p, sp.restr.indices_nat.p, f.ework0.p, mask,
-                              v, u, sp.restr.perm.p, sp.restr.nperm, s);
+    kern::scatter_rows(sp.restr, bb, f.ework0.p, mask, v, u, s);
 }
 
 // ---- OperatorChebyshevSmoother ----------------------------------------------
@@ -1375,9 +1367,8 @@ void chebyshev_apply(Chebyshev &c, const double *x, double *y, const int *stop, 
         pcg_element_apply<double>(f, c.prec, c.mask, c.t.p, f.ework0.p,
                                   bb < n ? c.u.p : nullptr, stop, s);
         hipLaunchKernelGGL(kern::k_cheb_scatter, dim3(ch.blocks), dim3(kern::kThreads), 0, s, n,
-                           ch.per, bb, sp.restr.offsets.p, sp.restr.indices_nat.p, f.ework0.p,
-                           c.mask, c.dinv.p, c.u.p, c.t.p, y, c.coeffs[k], stop, sp.restr.perm.p,
-                           sp.restr.nperm);
+                           ch.per, bb, sp.restr.rows(), f.ework0.p, c.mask, c.dinv.p, c.u.p,
+                           c.t.p, y, c.coeffs[k], stop);
     }
     H1PA_HIP(hipGetLastError());
 }
@@ -1490,8 +1481,7 @@ void pcg_preconditioned(Form &f, const uint8_t *mask, const Precond &M, const do
         pcg_element_apply<double>(f, H1PA_PREC_FP64, mask, d, f.ework0.p,
                                   bb < n ? q : nullptr, stop, s);
         hipLaunchKernelGGL(kern::k_pcg_scatter<double>, grid, blk, 0, s, n, per, bb,
-                           sp.restr.offsets.p, sp.restr.indices_nat.p, f.ework0.p, mask, d,
-                           q, partials, st, sp.restr.perm.p, sp.restr.nperm);
+                           sp.restr.rows(), f.ework0.p, mask, d, q, partials, st);
         hipLaunchKernelGGL(kern::k_pcg_fin_den, one, blk, 0, s, (int)nb, partials, st);
     };
     apply();
@@ -1569,9 +1559,8 @@ void ir_solve(Form &f, const uint8_t *mask, const double *diag, const double *b,
         // q = A d with the reduced-precision operator
         pcg_element_apply<float>(f, o.inner_precision, mask, d.p, f.ework32.p,
                                  bb < n ? q.p : nullptr, done, s);
-        hipLaunchKernelGGL(kern::k_ir_scatter, grid, blk, 0, s, n, per, bb, sp.restr.offsets.p,
-                           sp.restr.indices_nat.p, f.ework32.p, mask, d.p, q.p, partials.p, st.p,
-                           sp.restr.perm.p, sp.restr.nperm);
+        hipLaunchKernelGGL(kern::k_ir_scatter, grid, blk, 0, s, n, per, bb, sp.restr.rows(),
+                           f.ework32.p, mask, d.p, q.p, partials.p, st.p);
         hipLaunchKernelGGL(kern::k_ir_fin_den, one, blk, 0, s, (int)nb, partials.p, st.p);
         hipLaunchKernelGGL(kern::k_ir_update, grid, blk, 0, s, n, per, dinv.p, xs.p, r.p, z.p, q.p,
                            d.p, partials.p, st.p);
@@ -1579,9 +1568,9 @@ void ir_solve(Form &f, const uint8_t *mask, const double *diag, const double *b,
         hipLaunchKernelGGL(kern::k_ir_ru_x, dim3(nbx), blk, 0, s, n, xs.p, x, st.p);
         pcg_element_apply<double>(f, H1PA_PREC_FP64, mask, x, f.ework0.p,
                                   bb < n ? r64.p : nullptr, nru, s);
-        hipLaunchKernelGGL(kern::k_ir_ru_res, grid, blk, 0, s, n, per, bb, sp.restr.offsets.p,
-                           sp.restr.indices_nat.p, f.ework0.p, mask, b, x, dinv64.p, dinv.p,
-                           r64.p, r.p, z.p, partials.p, st.p, sp.restr.perm.p, sp.restr.nperm);
+        hipLaunchKernelGGL(kern::k_ir_ru_res, grid, blk, 0, s, n, per, bb, sp.restr.rows(),
+                           f.ework0.p, mask, b, x, dinv64.p, dinv.p, r64.p, r.p, z.p, partials.p,
+                           st.p);
         hipLaunchKernelGGL(kern::k_ir_fin_ru, one, blk, 0, s, (int)nb, partials.p, st.p);
         hipLaunchKernelGGL(kern::k_ir_dir, grid, blk, 0, s, n, per, z.p, d.p, st.p);
         H1PA_HIP(hipGetLastError());

@@ -12,8 +12,11 @@
 //    bit-identical to MFEM's sequential build (restriction.cpp:73-113).
 //  * E->L: one thread per L-DOF sums its E-entries in table order -- no
 //    floating-point atomics, deterministic (restriction.cpp:159-228).
+#include <algorithm>
+
 #include "internal.hpp"
 #include "row_sum.hpp"
+#include "row_table.hpp"
 
 
 namespace h1pa {
@@ -384,14 +387,69 @@ __global__ void k_scatter_constrained(int64_t nrows, const int *__restrict__ off
     y[i] = row_sum(indices, b, e, xe);
 }
 
-__global__ void k_native_indices(int64_t nE, int dof, const int *__restrict__ indices,
+// One row of the table per thread; over[0] is set when a row does not fit.
+__global__ void k_build_row_table(RowTab tb, int dof, const int *__restrict__ offsets,
+                                  const int *__restrict__ indices, const int *__restrict__ l2n,
+                                  int *__restrict__ tab, int *__restrict__ over) {
+    const int64_t tl = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (tl >= tb.bbeg) return;
+    const int t = (int)tl, i = row_dof(tb, t);
+    int w;
+    int *p;
+    if (t < tb.ebeg) {
+        w = 8;
+        p = tab + 8 * tl;
+    } else if (t < tb.fbeg) {
+        w = 4;
+        p = tab + 8 * (int64_t)tb.ebeg + 4 * (tl - tb.ebeg);
+    } else {
+        w = 2;
+        p = tab + 8 * (int64_t)tb.ebeg + 4 * (int64_t)(tb.fbeg - tb.ebeg) + 2 * (tl - tb.fbeg);
+    }
+    const int b = offsets[i], n = offsets[i + 1] - b;
+    for (int k = 0; k < w; ++k) {
+        int v = -1;
+        if (k < n && n <= w) {
+            const int l = indices[b + k], e = l / dof;
+            v = e * tb.es + l2n[l - e * dof];
+        }
+        p[k] = v;
+    }
+    if (n > w) {
+        p[0] = kRowOver;
+        over[0] = 1;
+    }
+}
+
+// E -> L from the row table, R rows per thread kBlock apart.
+template <int R, bool NT, typename T>
+__global__ void __launch_bounds__(kBlock)
+k_scatter_rows(int64_t nrows, RowTab tb, const T *__restrict__ ye,
+               const uint8_t *__restrict__ mask, const T *__restrict__ xin, T *__restrict__ y) {
+    const int64_t t0 = (int64_t)blockIdx.x * (R * kBlock) + threadIdx.x;
+    if (t0 >= nrows) return;
+    int t[R], i[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int64_t q = t0 + r * kBlock;
+        t[r] = (int)(q < nrows ? q : nrows - 1);
+        i[r] = row_dof(tb, t[r]);
+    }
+    T s[R];
+    rows_sum<R, NT>(tb, t, ye, s);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (t0 + r * kBlock < nrows) y[i[r]] = (mask && mask[i[r]]) ? xin[i[r]] : s[r];
+}
+
+__global__ void k_native_indices(int64_t nE, int dof, int es, const int *__restrict__ indices,
                                  const int *__restrict__ l2n, int *__restrict__ out) {
     const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (j >= nE) return;
     const int v = indices[j];
     const int lid = v >= 0 ? v : -1 - v;
     const int e = lid / dof, l = lid - e * dof;
-    const int n = e * dof + l2n[l];
+    const int n = e * es + l2n[l];  // interior entries (l2n >= es) are not read from here
     out[j] = v >= 0 ? n : -1 - n;
 }
 
@@ -506,10 +564,10 @@ void restrict_mult(int64_t nE, const int *gmap, const double *x, double *y, bool
     H1PA_HIP(hipGetLastError());
 }
 
-void native_indices(int64_t nE, int dof, const int *indices, const int *lex2nat, int *out,
+void native_indices(int64_t nE, int dof, int es, const int *indices, const int *lex2nat, int *out,
                     hipStream_t s) {
-    hipLaunchKernelGGL(k_native_indices, dim3(nblocks(nE)), dim3(kBlock), 0, s, nE, dof, indices,
-                       lex2nat, out);
+    hipLaunchKernelGGL(k_native_indices, dim3(nblocks(nE)), dim3(kBlock), 0, s, nE, dof, es,
+                       indices, lex2nat, out);
     H1PA_HIP(hipGetLastError());
 }
 
@@ -552,6 +610,62 @@ void bubble_mult_transpose(int64_t ne, int D, int64_t bb, const double *xe, doub
     H1PA_HIP(hipGetLastError());
 }
 
+void build_row_table(Restriction &r, hipStream_t s) {
+    const int64_t nv = r.nperm, nf = r.bubble_begin - nv - r.nedofs;
+    r.row_tab.alloc(std::max<size_t>((size_t)(8 * nv + 4 * r.nedofs + 2 * nf), 1));
+    r.row_over = 0;
+    StreamBuf<int> over(1, s);
+    H1PA_HIP(hipMemsetAsync(over.p, 0, sizeof(int), s));
+    const RowTab tb = r.rows();
+    hipLaunchKernelGGL(k_build_row_table, dim3(nblocks(r.bubble_begin)), dim3(kBlock), 0, s, tb,
+                       (int)r.dof, r.offsets.p, r.indices.p, r.lex2nat.p, r.row_tab.p, over.p);
+    H1PA_HIP(hipGetLastError());
+    int h = 0;
+    H1PA_HIP(hipMemcpyAsync(&h, over.p, sizeof(int), hipMemcpyDeviceToHost, s));
+    H1PA_HIP(hipStreamSynchronize(s));
+    if (h) {  // the wide rows are read from the native CSR table
+        r.indices_nat.alloc((size_t)(r.ne * r.dof));
+        native_indices(r.ne * r.dof, (int)r.dof, tb.es, r.indices.p, r.lex2nat.p, r.indices_nat.p, s);
+        H1PA_HIP(hipStreamSynchronize(s));
+        r.row_over = 1;
+    }
+}
+
+namespace {
+template <typename T>
+void launch_scatter_rows(const Restriction &r, int64_t nrows, const T *ye, const uint8_t *mask,
+                         const T *xin, T *y, hipStream_t s) {
+    if (nrows <= 0) return;
+    // Rows per thread.  Below a block per CU of two-row threads one row each
+    // (p = 3, 16^3 elements, 86k rows: 7.05 -> 6.27 us between events); from 6M
+    // rows on, where the E-vector and the table no longer stay in the caches,
+    // four with the table streamed (p = 4, 79^3, 18.6M rows: 174 -> 165 us; p = 2, 100^3: 154 ->
+    // 145; at 4M rows, p = 8: 30.9 -> 31.7 us); two between.
+    const RowTab tb = r.rows();
+    auto grid = [&](int R) { return dim3(nblocks((nrows + R - 1) / R)); };
+    if (nrows <= 256 * 2 * kBlock)
+        hipLaunchKernelGGL((k_scatter_rows<1, false, T>), grid(1), dim3(kBlock), 0, s, nrows, tb,
+                           ye, mask, xin, y);
+    else if (nrows < (int64_t)6 << 20)
+        hipLaunchKernelGGL((k_scatter_rows<2, false, T>), grid(2), dim3(kBlock), 0, s, nrows, tb,
+                           ye, mask, xin, y);
+    else
+        hipLaunchKernelGGL((k_scatter_rows<4, true, T>), grid(4), dim3(kBlock), 0, s, nrows, tb,
+                           ye, mask, xin, y);
+    H1PA_HIP(hipGetLastError());
+}
+}  // namespace
+
+void scatter_rows(const Restriction &r, int64_t nrows, const double *ye, const uint8_t *mask,
+                  const double *xin, double *y, hipStream_t s) {
+    launch_scatter_rows(r, nrows, ye, mask, xin, y, s);
+}
+
+void scatter_rows(const Restriction &r, int64_t nrows, const float *ye, const uint8_t *mask,
+                  const float *xin, float *y, hipStream_t s) {
+    launch_scatter_rows(r, nrows, ye, mask, xin, y, s);
+}
+
 void boolean_mask(int64_t nrows, const int *offsets, const int *indices, double *ye,
                   hipStream_t s) {
     if (nrows <= 0) return;
@@ -570,4 +684,20 @@ void scatter_constrained(int64_t nrows, const int *offsets, const int *indices, 
 }
 
 }  // namespace kern
+
+RowTab Restriction::rows() const {
+    RowTab t;
+    t.tab = row_tab.p;
+    t.perm = perm.p;
+    t.ebeg = (int)nperm;
+    t.fbeg = (int)(nperm + nedofs);
+    t.bbeg = (int)bubble_begin;
+    t.es = (int)(dof - interior());
+    t.nb = (int)interior();
+    t.ebub = native_bubble();
+    t.over = row_over;
+    t.offsets = offsets.p;
+    t.indices = indices_nat.p;
+    return t;
+}
 }  // namespace h1pa
