@@ -72,8 +72,11 @@ struct SlotDesc {
     double rel_tol, abs_tol;           // CGSolver settings (mixed: rel_tol on the FP64 measure)
     double delta;                      // mixed: refinement trigger
     int max_outer;
-    int pad_;
+    int p;                             // order (the merged element kernel)
 };
+
+// (D, Q) of a batch's forms: q1d = p + 2.
+#define H1PA_BATCH_DQ(X) X(2, 3) X(3, 4) X(4, 5) X(5, 6) X(6, 7) X(7, 8) X(8, 9) X(9, 10)
 
 struct VecTask {
     int slot, chunk;
@@ -138,6 +141,29 @@ __device__ inline void slot_totals(const SlotDesc &sd, const double *partials, d
         for (int u = 0; u < U8; ++u) w += v[u];
         tot[k] = bsum(w, sh);
     }
+}
+
+// The same total, bit for bit, for a slot of at most 4 kT chunks, in the two
+// halves of a folded step: the loads go out with the step's other ones.
+struct FoldSum {
+    double v[4];
+};
+__device__ __forceinline__ FoldSum fold_load(const double *__restrict__ partials, int part0,
+                                             int nchunks) {
+    FoldSum f;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int i = u * kT + threadIdx.x;
+        const double v = partials[part0 + (i < nchunks ? i : nchunks - 1)];
+        f.v[u] = i < nchunks ? 0.0 + v : 0.0;
+    }
+    return f;
+}
+__device__ __forceinline__ double fold_total(const FoldSum &f, double *sh) {
+    double w = 0.0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) w += f.v[u];
+    return bsum(w, sh);
 }
 
 template <typename T>
@@ -221,6 +247,81 @@ __device__ __forceinline__ void share_rows(const RowTab &tb, int64_t bb, const S
     SlotState *st = states + slot;                                                \
     const int ph_ = st->phase;                                                    \
     if (!(PHASE_OK)) return;
+
+// The scalar logic of an iteration, in and out of plain values: after the
+// (A d, d) product and after the (B r, r) product of the update.
+struct StepOut {
+    int phase, nonfinite;
+};
+template <bool MIXED>
+__device__ __forceinline__ StepOut after_den(double den) {
+    if (!isfinite(den)) return {PH_DONE, 1};  // MFEM_VERIFY(IsFinite(den))
+    if (den == 0.0)  // mixed: the inner residual is zero, check the true one
+        return {MIXED ? PH_RU : PH_DONE, 0};
+    return {PH_INNER, 0};
+}
+// iter: the iteration that rho belongs to (FP64 mode: MFEM's i; mixed: counted
+// from 1); thresh: the stop level (FP64 mode) or the level that asks for a
+// refinement step (mixed).
+template <bool MIXED>
+__device__ __forceinline__ StepOut after_update(double rho, double thresh, int iter,
+                                                int max_iter) {
+    if (!isfinite(rho)) return {PH_DONE, 1};  // MFEM_VERIFY(IsFinite(betanom))
+    if (rho < 0.0) return {PH_DONE, 0};       // the preconditioner is not positive definite
+    if (MIXED) return {rho <= thresh || iter >= max_iter ? PH_RU : PH_INNER, 0};
+    return {rho <= thresh || iter + 1 > max_iter ? PH_DONE : PH_INNER, 0};
+}
+template <bool MIXED>
+__device__ __forceinline__ double update_thresh(const SlotState &st, const SlotDesc &sd) {
+    if (!MIXED) return st.r0;
+    const double a = sd.delta * sd.delta * st.rho_ref, b = sd.rel_tol * sd.rel_tol * st.rho64_0;
+    return a > b ? a : b;
+}
+template <bool MIXED>
+__device__ __forceinline__ void write_den(SlotState *st, double den) {
+    const StepOut u = after_den<MIXED>(den);
+    st->den = den;
+    if (u.phase == PH_INNER) return;
+    if (u.nonfinite) st->nonfinite = 1;
+    if (u.phase == PH_DONE) st->final_iter = st->in_loop ? st->iter : 0;
+    st->phase = u.phase;
+}
+// o = the state after the update's product rho of a slot in PH_INNER
+template <bool MIXED>
+__device__ __forceinline__ void write_update(const SlotState &st, SlotState *o, double rho,
+                                             double thresh, const StepOut &u) {
+    const int i = MIXED ? st.iter + 1 : st.iter;
+    const bool on = u.phase == PH_INNER;
+    const int converged = st.converged, max_iter = st.max_iter, final_iter = st.final_iter;
+    const double nom = st.nom, beta = st.beta;
+    o->nom0 = st.nom0;
+    o->den = st.den;
+    o->r0 = st.r0;
+    o->rho_ref = st.rho_ref;
+    o->rho64 = st.rho64;
+    o->rho64_0 = st.rho64_0;
+    o->r2 = st.r2;
+    o->b2 = st.b2;
+    o->outer = st.outer;
+    o->max_iter = max_iter;
+    o->betanom = MIXED ? st.betanom : rho;
+    o->in_loop = MIXED ? st.in_loop : 1;
+    o->beta = on ? rho / nom : beta;
+    o->nom = on ? rho : nom;
+    o->nonfinite = st.nonfinite | u.nonfinite;
+    o->phase = u.phase;
+    if (MIXED) {
+        o->iter = i;
+        o->converged = converged;
+        o->final_iter = final_iter;
+    } else {
+        o->iter = on ? i + 1 : i;
+        const bool conv = !u.nonfinite && rho >= 0.0 && rho <= thresh;
+        o->converged = conv ? 1 : converged;
+        o->final_iter = on ? final_iter
+                        : (!u.nonfinite && rho >= 0.0 && !conv) ? max_iter : i;
+    }
+}
 
 // ---- FP64 mode: CGSolver on each slot ---------------------------------------
 __global__ void __launch_bounds__(kT)
@@ -381,6 +482,68 @@ kb_diffusion(const ElemTask *__restrict__ tasks, const SlotDesc *__restrict__ de
     }
 }
 
+// The element kernel over slots of any order in one launch: the block takes its
+// task's order.  A batch of small problems has a few hundred blocks per order,
+// each launch of which leaves most of the chip idle for its whole latency: 24
+// problems of 729 to 117,649 DOFs, p = 2..6, BF16 data: five launches of 3.8 to
+// 10.7 us (39 us an iteration), 20 us merged, near the element kernels' own
+// rate.  256 threads, two PA planes requested ahead; the registers are those of
+// the widest order (up to p = 6, or all), so a group that fills the chip by
+// itself keeps its own tuned launch (rebuild).  Waves per SIMD: 5 and 4 for
+// FP32 (6 spills: 21.5 us; 4 at p <= 6: 24.5), 2 for FP64 (3 spills: 28 against
+// 19 us).
+template <typename T>
+struct BasisOf {
+    const T *b[9] = {};  // by order
+};
+template <int Q>
+constexpr int nb_any() { return 256 / (Q * Q); }
+template <typename T, int PMAX>
+constexpr int any_lds() {
+    int m = 0;
+#define X(DD, QQ)                                                                   \
+    if (DD <= PMAX + 1 && nb_any<QQ>() * diffusion_buf<DD, QQ>() > m)               \
+        m = nb_any<QQ>() * diffusion_buf<DD, QQ>();
+    H1PA_BATCH_DQ(X)
+#undef X
+    return m;
+}
+template <typename T, int PMAX>
+constexpr int any_waves() { return sizeof(T) == 8 ? 2 : PMAX <= 6 ? 5 : 4; }
+template <typename T, typename TP, bool RU, int PMAX, int W>
+__global__ void __launch_bounds__(256, W)
+kb_diffusion_any(const ElemTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
+                 const SlotState *__restrict__ states, const BasisOf<T> basis) {
+    const ElemTask tk = tasks[blockIdx.x];
+    const SlotDesc &sd = desc[tk.slot];
+    if (states[tk.slot].phase != (RU ? PH_RU : PH_INNER)) return;
+    __shared__ T smem[any_lds<T, PMAX>()];
+    EOutT<T> out;
+    out.l2n = global_ptr(sd.l2n);
+    out.ye = RU ? gv<T>(sd.ye64) : gv<T>(sd.ye);
+    const bool direct = sd.bb < sd.n;
+    out.yL = !direct ? out.ye : RU ? gv<T>(sd.r64) : gv<T>(sd.z);
+    out.bb = direct ? sd.bb : sd.rows.ebub;
+    const int *gmap = global_ptr(sd.gmap);
+    const uint8_t *mask = sd.mask ? global_ptr(sd.mask) : nullptr;
+    const TP *pa = RU ? gv<TP>(sd.pa64) : gv<TP>(sd.pa);
+    const T *x = RU ? gv<T>(sd.x) : gv<T>(sd.d);
+    const T *bs = basis.b[sd.p];
+    // threads past the block's whole elements are past the last valid one
+#define X(DD, QQ)                                                                              \
+    case DD - 1:                                                                               \
+        if constexpr (DD <= PMAX + 1)                                                          \
+            diffusion_elements<T, TP, DD, QQ, nb_any<QQ>(), 1, 2>(                             \
+                tk.e0, min(sd.ne, (int64_t)tk.e0 + nb_any<QQ>()), bs, pa, gmap, mask, x, out,  \
+                0, smem);                                                                      \
+        break;
+    switch (sd.p) {
+        H1PA_BATCH_DQ(X)
+        default: break;
+    }
+#undef X
+}
+
 // z = A d for PH_INNER slots (DIAG_ONE rows copy d); partials of (d, z).
 template <typename T>
 __global__ void __launch_bounds__(kT)
@@ -425,32 +588,27 @@ kb_fin_den(const int *__restrict__ runlist, const SlotDesc *__restrict__ desc,
     double tot[1];
     slot_totals<1>(sd, partials, sh, tot);
     if (threadIdx.x != 0) return;
-    st->den = tot[0];
-    if (!isfinite(tot[0])) {  // MFEM_VERIFY(IsFinite(den))
-        st->nonfinite = 1;
-        st->final_iter = st->in_loop ? st->iter : 0;
-        st->phase = PH_DONE;
-    } else if (tot[0] == 0.0) {
-        if (MIXED) {
-            st->phase = PH_RU;  // inner residual is zero: check the true one
-        } else {            // CGSolver: den == 0 ends the loop
-            st->final_iter = st->in_loop ? st->iter : 0;
-            st->phase = PH_DONE;
-        }
-    }
+    write_den<MIXED>(st, tot[0]);
 }
 
+// x += alpha d, r -= alpha z, z = dinv r, partials of (r, z); x is the
+// solution (FP64 mode) or the FP32 update xs (mixed).  FOLD: the slot's
+// (A d, d) is summed here, by every block from the partials pden, and the
+// block of chunk 0 applies the step's scalar logic (a block that reads the
+// phase it writes stops either way: it finds the same total).
+template <typename T, bool MIXED, bool FOLD>
 __global__ void __launch_bounds__(kT)
 kb_update(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
-          const SlotState *__restrict__ states, double *__restrict__ partials) {
+          SlotState *states, const double *__restrict__ pden, double *__restrict__ partials) {
     __shared__ double sh[kT];
     H1PA_TASK_PROLOGUE(ph_ == PH_INNER)
-    const SlotState *st = states + tk.slot;
-    const double alpha = st->nom / st->den;
-    double *x = global_ptr(sd.x), *r = gv<double>(sd.r), *z = gv<double>(sd.z);
-    const double *d = gv<double>(sd.d), *dinv = gv<double>(sd.dinv);
+    double nom = states[tk.slot].nom, den;
+    FoldSum fs;
+    if constexpr (FOLD) fs = fold_load(pden, sd.part0, sd.nchunks);
+    T *x = gv<T>(sd.xi), *r = gv<T>(sd.r), *z = gv<T>(sd.z);
+    const T *d = gv<T>(sd.d), *dinv = gv<T>(sd.dinv);
     const Share h = share_of(tk.chunk, sd.n);
-    double vx[kPer], vd[kPer], vr[kPer], vz[kPer], vi[kPer];
+    T vx[kPer], vd[kPer], vr[kPer], vz[kPer], vi[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
         const int64_t j = h.lt[k];
@@ -460,21 +618,30 @@ kb_update(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
         vz[k] = z[j];
         vi[k] = dinv[j];
     }
+    if constexpr (FOLD) {
+        den = fold_total(fs, sh);
+        if (tk.chunk == 0 && threadIdx.x == 0) write_den<MIXED>(states + tk.slot, den);
+        if (after_den<MIXED>(den).phase != PH_INNER) return;
+    } else {
+        den = states[tk.slot].den;
+    }
+    const T alpha = (T)(nom / den);
     double acc[1] = {0.0};
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
         if (!h.ok[k]) continue;
         const int64_t i = h.t[k];
         x[i] = vx[k] + alpha * vd[k];
-        const double ri = vr[k] - alpha * vz[k];
+        const T ri = vr[k] - alpha * vz[k];
         r[i] = ri;
-        const double zi = vi[k] * ri;
+        const T zi = vi[k] * ri;
         z[i] = zi;
-        acc[0] += ri * zi;
+        acc[0] += (double)ri * (double)zi;
     }
     store_chunk<1>(acc, sd, tk.chunk, partials, sh);
 }
 
+template <bool MIXED>
 __global__ void __launch_bounds__(kT)
 kb_fin_update(const int *__restrict__ runlist, const SlotDesc *__restrict__ desc,
               SlotState *__restrict__ states, const double *__restrict__ partials) {
@@ -483,93 +650,10 @@ kb_fin_update(const int *__restrict__ runlist, const SlotDesc *__restrict__ desc
     double tot[1];
     slot_totals<1>(sd, partials, sh, tot);
     if (threadIdx.x != 0) return;
-    const double betanom = tot[0];
-    const int i = st->iter;
-    st->in_loop = 1;
-    st->betanom = betanom;
-    if (!isfinite(betanom)) {  // MFEM_VERIFY(IsFinite(betanom))
-        st->nonfinite = 1;
-        st->final_iter = i;
-        st->phase = PH_DONE;
-    } else if (betanom < 0.0) {
-        st->final_iter = i;
-        st->phase = PH_DONE;
-    } else if (betanom <= st->r0) {
-        st->converged = 1;
-        st->final_iter = i;
-        st->phase = PH_DONE;
-    } else if (i + 1 > st->max_iter) {
-        st->final_iter = st->max_iter;
-        st->phase = PH_DONE;
-    } else {
-        st->beta = betanom / st->nom;
-        st->nom = betanom;
-        st->iter = i + 1;
-    }
-}
-
-__global__ void __launch_bounds__(kT)
-kbm_update(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
-           const SlotState *__restrict__ states, double *__restrict__ partials) {
-    __shared__ double sh[kT];
-    H1PA_TASK_PROLOGUE(ph_ == PH_INNER)
-    const SlotState *st = states + tk.slot;
-    const float alpha = (float)(st->nom / st->den);
-    float *xs = gv<float>(sd.xi), *r = gv<float>(sd.r), *z = gv<float>(sd.z);
-    const float *d = gv<float>(sd.d), *dinv = gv<float>(sd.dinv);
-    const Share h = share_of(tk.chunk, sd.n);
-    float vx[kPer], vd[kPer], vr[kPer], vz[kPer], vi[kPer];
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        const int64_t j = h.lt[k];
-        vx[k] = xs[j];
-        vd[k] = d[j];
-        vr[k] = r[j];
-        vz[k] = z[j];
-        vi[k] = dinv[j];
-    }
-    double acc[1] = {0.0};
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        if (!h.ok[k]) continue;
-        const int64_t i = h.t[k];
-        xs[i] = vx[k] + alpha * vd[k];
-        const float ri = vr[k] - alpha * vz[k];
-        r[i] = ri;
-        const float zi = vi[k] * ri;
-        z[i] = zi;
-        acc[0] += (double)ri * (double)zi;
-    }
-    store_chunk<1>(acc, sd, tk.chunk, partials, sh);
-}
-
-__global__ void __launch_bounds__(kT)
-kbm_fin_update(const int *__restrict__ runlist, const SlotDesc *__restrict__ desc,
-               SlotState *__restrict__ states, const double *__restrict__ partials) {
-    __shared__ double sh[kT];
-    H1PA_FIN_PROLOGUE(ph_ == PH_INNER)
-    double tot[1];
-    slot_totals<1>(sd, partials, sh, tot);
-    if (threadIdx.x != 0) return;
-    const double rho = tot[0];
-    st->iter += 1;
-    if (!isfinite(rho)) {
-        st->nonfinite = 1;
-        st->phase = PH_DONE;
-        return;
-    }
-    if (rho < 0.0) {  // the preconditioner is not positive definite
-        st->phase = PH_DONE;
-        return;
-    }
-    const double tol2 = sd.rel_tol * sd.rel_tol;
-    if (rho <= sd.delta * sd.delta * st->rho_ref || rho <= tol2 * st->rho64_0 ||
-        st->iter >= st->max_iter) {
-        st->phase = PH_RU;
-    } else {
-        st->beta = rho / st->nom;
-        st->nom = rho;
-    }
+    const double thresh = update_thresh<MIXED>(*st, sd);
+    write_update<MIXED>(*st, st, tot[0], thresh,
+                        after_update<MIXED>(tot[0], thresh, MIXED ? st->iter + 1 : st->iter,
+                                            st->max_iter));
 }
 
 template <typename T>
@@ -587,6 +671,47 @@ kb_dir(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
         vz[k] = z[h.lt[k]];
         vd[k] = d[h.lt[k]];
     }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+        if (h.ok[k]) d[h.t[k]] = vz[k] + beta * vd[k];
+}
+
+// The same with the update's scalar step folded in (a launch less, of 4 us and
+// the gap before it, for up to 8 KB of partials per block): every block sums the slot's
+// (r, z) from the partials and finds the iteration's outcome; the block of
+// chunk 0 writes the state to `next`, which the kernels after this one read
+// (no block reads what another of this launch writes).
+template <typename T, bool MIXED>
+__global__ void __launch_bounds__(kT)
+kb_dir_fold(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
+            const SlotState *__restrict__ states, SlotState *__restrict__ next,
+            const double *__restrict__ partials) {
+    __shared__ double sh[kT];
+    const VecTask tk = tasks[blockIdx.x];
+    const SlotDesc &sd = desc[tk.slot];
+    const SlotState &st = states[tk.slot];
+    const bool writer = tk.chunk == 0 && threadIdx.x == 0;
+    if (st.phase != PH_INNER) {
+        if (writer) next[tk.slot] = st;
+        return;
+    }
+    const FoldSum fs = fold_load(partials, sd.part0, sd.nchunks);
+    const double nom = st.nom, thresh = update_thresh<MIXED>(st, sd);
+    const int iter = MIXED ? st.iter + 1 : st.iter, max_iter = st.max_iter;
+    const T *z = gv<T>(sd.z);
+    T *d = gv<T>(sd.d);
+    const Share h = share_of(tk.chunk, sd.n);
+    T vz[kPer], vd[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        vz[k] = z[h.lt[k]];
+        vd[k] = d[h.lt[k]];
+    }
+    const double rho = fold_total(fs, sh);
+    const StepOut u = after_update<MIXED>(rho, thresh, iter, max_iter);
+    if (writer) write_update<MIXED>(st, next + tk.slot, rho, thresh, u);
+    if (u.phase != PH_INNER) return;
+    const T beta = (T)(rho / nom);
 #pragma unroll
     for (int k = 0; k < kPer; ++k)
         if (h.ok[k]) d[h.t[k]] = vz[k] + beta * vd[k];
@@ -745,8 +870,6 @@ bool variant_ok(int prec, int v) {
     return prec == H1PA_PREC_FP64 ? (v >= 0 && v < 9) : (v == 0 || v == 1 || (v >= 4 && v < 9));
 }
 
-#define H1PA_BATCH_DQ(X) X(2, 3) X(3, 4) X(4, 5) X(5, 6) X(6, 7) X(7, 8) X(8, 9) X(9, 10)
-
 // Elements per block of variant v: FP64 kernels (fp64 = true) or FP32 ones.
 int nb_of_dq(int D, int Q, int v, bool fp64) {
 #define X(DD, QQ) \
@@ -785,6 +908,43 @@ void launch_group(int prec, bool ru, int D, int Q, int v, const ElemTask *tasks,
     throw Error{H1PA_EUNSUP, "batch: unsupported (p, q1d)"};
 }
 
+template <int PMAX>
+void launch_any_pmax(int prec, bool ru, const ElemTask *tasks, int ntasks, const SlotDesc *desc,
+                     const SlotState *st, const void *const *basis, hipStream_t s) {
+    constexpr int W64 = kern::any_waves<double, PMAX>(), W32 = kern::any_waves<float, PMAX>();
+    const dim3 grid((unsigned)ntasks), blk(256);
+    if (ru || prec == H1PA_PREC_FP64) {
+        kern::BasisOf<double> b;
+        for (int p = 1; p <= 8; ++p) b.b[p] = (const double *)basis[p];
+        if (ru)
+            hipLaunchKernelGGL((kern::kb_diffusion_any<double, double, true, PMAX, W64>), grid, blk, 0,
+                               s, tasks, desc, st, b);
+        else
+            hipLaunchKernelGGL((kern::kb_diffusion_any<double, double, false, PMAX, W64>), grid, blk, 0,
+                               s, tasks, desc, st, b);
+    } else {
+        kern::BasisOf<float> b;
+        for (int p = 1; p <= 8; ++p) b.b[p] = (const float *)basis[p];
+        if (prec == H1PA_PREC_FP32)
+            hipLaunchKernelGGL((kern::kb_diffusion_any<float, float, false, PMAX, W32>), grid, blk, 0,
+                               s, tasks, desc, st, b);
+        else
+            hipLaunchKernelGGL((kern::kb_diffusion_any<float, bf16_t, false, PMAX, W32>), grid, blk, 0,
+                               s, tasks, desc, st, b);
+    }
+    H1PA_HIP(hipGetLastError());
+}
+// pmax: the highest order in the work list.
+void launch_any(int prec, bool ru, int pmax, const ElemTask *tasks, int ntasks,
+                const SlotDesc *desc, const SlotState *st, const void *const *basis,
+                hipStream_t s) {
+    if (ntasks <= 0) return;
+    if (pmax <= 6) launch_any_pmax<6>(prec, ru, tasks, ntasks, desc, st, basis, s);
+    else launch_any_pmax<8>(prec, ru, tasks, ntasks, desc, st, basis, s);
+}
+// Elements per block of the merged kernel.
+int nb_merged(int q1d) { return 256 / (q1d * q1d); }
+
 }  // namespace
 
 struct BatchSlot {
@@ -820,6 +980,7 @@ struct BatchGroup {
     DevBuf<ElemTask> tasks64;  // mixed: work list of the FP64 refinement kernels
     int ntasks64 = 0;
     bool tuned = false;
+    bool merged = false;  // its slots are in the batch's merged work list
 };
 
 }  // namespace h1pa
@@ -830,9 +991,14 @@ struct h1pa_batch {
     std::vector<std::unique_ptr<h1pa::BatchSlot>> slots;
     std::vector<h1pa::BatchGroup> groups;
     h1pa::DevBuf<h1pa::SlotDesc> d_desc;
-    h1pa::DevBuf<h1pa::SlotState> d_state;
+    // The states, and the copy that the folded direction updates write: a
+    // replay swaps the two an even number of times.
+    h1pa::DevBuf<h1pa::SlotState> d_state, d_next;
     std::vector<h1pa::SlotState> h_state;
-    h1pa::DevBuf<double> partials;
+    h1pa::DevBuf<double> partials, pden;  // pden: of (A d, d) when the scalar steps are folded
+    bool fold = false;
+    h1pa::DevBuf<h1pa::ElemTask> any_tasks;  // merged element work list (groups with `merged`)
+    int n_any = 0, any_pmax = 0;
     h1pa::DevBuf<h1pa::VecTask> vtasks;
     int nvtasks = 0;
     h1pa::DevBuf<int> runlist;  // slots with work items, one finalize block each
@@ -906,8 +1072,9 @@ void drop_graph(Batch &B) {
 
 // Work list of group g: (slot, first element) per block, in slot and element
 // order (consecutive blocks take neighbouring elements of one slot).
-void element_tasks(const Batch &B, int g, int nb, std::vector<ElemTask> &out) {
-    out.clear();
+void element_tasks(const Batch &B, int g, int nb, std::vector<ElemTask> &out,
+                   bool append = false) {
+    if (!append) out.clear();
     for (size_t k = 0; k < B.slots.size(); ++k) {
         const BatchSlot &sl = *B.slots[k];
         if (sl.group != g || !sl.live || !running_phase(B.h_state[k].phase)) continue;
@@ -947,9 +1114,28 @@ void rebuild(Batch &B) {
     B.nrun = (int)run.size();
     if (B.runlist.n < run.size()) B.runlist.alloc(run.size());
     B.runlist.upload(run.data(), run.size(), B.stream);
-    std::vector<ElemTask> et;
+    // Folded scalar steps make every vector block sum its slot's partials: for
+    // slots of up to 1024 chunks (1M DOFs), four values a thread.
+    B.fold = true;
+    for (int k : run) B.fold = B.fold && desc[k].nchunks <= 1024;
+    if (B.fold && B.pden.n < (size_t)part + 1) B.pden.alloc((size_t)part + 1);
+    if (B.fold && B.d_next.n < B.d_state.n) B.d_next.alloc(B.d_state.n);
+    // Groups below four merged blocks per CU share one launch, when there are
+    // at least two of them.
+    std::vector<ElemTask> et, any;
+    int small = 0;
+    for (size_t g = 0; g < B.groups.size(); ++g) {
+        element_tasks(B, (int)g, nb_merged(B.groups[g].q1d), et);
+        B.groups[g].merged = !et.empty() && et.size() < 1024;
+        small += B.groups[g].merged ? 1 : 0;
+    }
     for (size_t g = 0; g < B.groups.size(); ++g) {
         BatchGroup &G = B.groups[g];
+        if (small < 2) G.merged = false;
+        if (G.merged) {
+            G.ntasks = G.ntasks64 = 0;
+            continue;
+        }
         element_tasks(B, (int)g, G.nb, et);
         G.ntasks = (int)et.size();
         if (G.tasks.n < et.size()) G.tasks.alloc(et.size());
@@ -961,6 +1147,17 @@ void rebuild(Batch &B) {
             G.tasks64.upload(et.data(), et.size(), B.stream);
         }
     }
+    // the highest orders' blocks, which run longest, first
+    B.any_pmax = 0;
+    for (int p = 8; p >= 1; --p)
+        for (size_t g = 0; g < B.groups.size(); ++g)
+            if (B.groups[g].merged && B.groups[g].p == p) {
+                element_tasks(B, (int)g, nb_merged(B.groups[g].q1d), any, true);
+                B.any_pmax = std::max(B.any_pmax, p);
+            }
+    B.n_any = (int)any.size();
+    if (B.any_tasks.n < any.size()) B.any_tasks.alloc(any.size());
+    B.any_tasks.upload(any.data(), any.size(), B.stream);
     H1PA_HIP(hipStreamSynchronize(B.stream));
     B.dirty = false;
 }
@@ -978,7 +1175,7 @@ void autotune(Batch &B) {
     try {
         for (size_t g = 0; g < B.groups.size(); ++g) {
             BatchGroup &G = B.groups[g];
-            if (G.tuned || G.ntasks < 256) continue;
+            if (G.tuned || G.merged || G.ntasks < 256) continue;
             G.tuned = true;
             float best = 1e30f;
             int bestv = G.variant;
@@ -1025,7 +1222,10 @@ void autotune(Batch &B) {
 std::vector<uintptr_t> replay_arguments(const Batch &B) {
     std::vector<uintptr_t> a{(uintptr_t)B.vtasks.p, (uintptr_t)B.runlist.p,
                              (uintptr_t)B.d_desc.p, (uintptr_t)B.d_state.p,
-                             (uintptr_t)B.partials.p, (uintptr_t)B.nvtasks, (uintptr_t)B.nrun};
+                             (uintptr_t)B.partials.p, (uintptr_t)B.nvtasks, (uintptr_t)B.nrun,
+                             (uintptr_t)B.d_next.p,   (uintptr_t)B.pden.p,  (uintptr_t)B.fold,
+                             (uintptr_t)B.any_tasks.p, (uintptr_t)B.n_any,
+                             (uintptr_t)B.any_pmax};
     for (const BatchGroup &G : B.groups) {
         a.push_back((uintptr_t)G.tasks.p);
         a.push_back((uintptr_t)G.ntasks);
@@ -1038,18 +1238,23 @@ std::vector<uintptr_t> replay_arguments(const Batch &B) {
     return a;
 }
 
-void enqueue_replay(Batch &B, hipStream_t s) {
-    const unsigned nv = (unsigned)B.nvtasks;
-    if (nv == 0) return;
-    const int prec = B.o.precision;
-    const dim3 grid(nv), blk(kern::kT), fin((unsigned)B.nrun);
+template <typename T, bool MIXED>
+void enqueue_iterations(Batch &B, hipStream_t s) {
+    const int prec = B.o.precision, K = B.o.iters_per_replay;
+    const dim3 grid((unsigned)B.nvtasks), blk(kern::kT), fin((unsigned)B.nrun);
     const VecTask *vt = B.vtasks.p;
     const int *rl = B.runlist.p;
     const SlotDesc *ds = B.d_desc.p;
-    SlotState *st = B.d_state.p;
+    SlotState *st = B.d_state.p, *next = B.d_next.p;
     double *pt = B.partials.p;
+    const void *basis[9] = {}, *basis64[9] = {};
+    for (const BatchGroup &G : B.groups) {
+        basis[G.p] = G.basis;
+        basis64[G.p] = G.basis64;
+    }
     auto elements = [&](bool ru) {
         for (BatchGroup &G : B.groups) {
+            if (G.merged) continue;
             if (ru)
                 launch_group(prec, true, G.p + 1, G.q1d, G.variant, G.tasks64.p, G.ntasks64, ds,
                              st, G.basis64, 0, s);
@@ -1057,39 +1262,63 @@ void enqueue_replay(Batch &B, hipStream_t s) {
                 launch_group(prec, false, G.p + 1, G.q1d, G.variant, G.tasks.p, G.ntasks, ds, st,
                              G.basis, 0, s);
         }
+        launch_any(prec, ru, B.any_pmax, B.any_tasks.p, B.n_any, ds, st, ru ? basis64 : basis, s);
     };
+    // Direction updates with the scalar step folded in swap the states; their
+    // number in a replay is even.  The last iteration of a mixed replay keeps
+    // the separate step, since the refinement follows it.
+    const int last = MIXED ? 1 : 0;
+    const int folded = B.fold ? (K - last) / 2 * 2 : 0;
+    for (int it = 0; it < K; ++it) {
+        elements(false);
+        hipLaunchKernelGGL(kern::kb_scatter<T>, grid, blk, 0, s, vt, ds, st,
+                           B.fold ? B.pden.p : pt);
+        if (B.fold) {
+            hipLaunchKernelGGL((kern::kb_update<T, MIXED, true>), grid, blk, 0, s, vt, ds, st,
+                               B.pden.p, pt);
+        } else {
+            hipLaunchKernelGGL(kern::kb_fin_den<MIXED>, fin, blk, 0, s, rl, ds, st, pt);
+            hipLaunchKernelGGL((kern::kb_update<T, MIXED, false>), grid, blk, 0, s, vt, ds, st,
+                               pt, pt);
+        }
+        if (it >= K - last - folded && it < K - last) {
+            hipLaunchKernelGGL((kern::kb_dir_fold<T, MIXED>), grid, blk, 0, s, vt, ds, st, next,
+                               pt);
+            std::swap(st, next);
+            continue;
+        }
+        hipLaunchKernelGGL(kern::kb_fin_update<MIXED>, fin, blk, 0, s, rl, ds, st, pt);
+        if (MIXED && it == K - 1) {
+            // refinement steps once per replay: a slot whose inner residual
+            // fell by delta waits in PH_RU (skipped by the inner kernels)
+            // until here, instead of every iteration launching the
+            // refinement kernels over all slots
+            hipLaunchKernelGGL(kern::kbm_ru_x, grid, blk, 0, s, vt, ds, st);
+            elements(true);
+            hipLaunchKernelGGL(kern::kbm_ru_res, grid, blk, 0, s, vt, ds, st, pt);
+            hipLaunchKernelGGL(kern::kbm_fin_ru, fin, blk, 0, s, rl, ds, st, pt);
+        }
+        hipLaunchKernelGGL(kern::kb_dir<T>, grid, blk, 0, s, vt, ds, st);
+    }
+}
+
+void enqueue_replay(Batch &B, hipStream_t s) {
+    const unsigned nv = (unsigned)B.nvtasks;
+    if (nv == 0) return;
+    const dim3 grid(nv), blk(kern::kT), fin((unsigned)B.nrun);
+    const VecTask *vt = B.vtasks.p;
+    const int *rl = B.runlist.p;
+    const SlotDesc *ds = B.d_desc.p;
+    SlotState *st = B.d_state.p;
+    double *pt = B.partials.p;
     if (!mixed_mode(B)) {
         hipLaunchKernelGGL(kern::kb_init, grid, blk, 0, s, vt, ds, st, pt);
         hipLaunchKernelGGL(kern::kb_fin_init, fin, blk, 0, s, rl, ds, st, pt);
-        for (int it = 0; it < B.o.iters_per_replay; ++it) {
-            elements(false);
-            hipLaunchKernelGGL(kern::kb_scatter<double>, grid, blk, 0, s, vt, ds, st, pt);
-            hipLaunchKernelGGL(kern::kb_fin_den<false>, fin, blk, 0, s, rl, ds, st, pt);
-            hipLaunchKernelGGL(kern::kb_update, grid, blk, 0, s, vt, ds, st, pt);
-            hipLaunchKernelGGL(kern::kb_fin_update, fin, blk, 0, s, rl, ds, st, pt);
-            hipLaunchKernelGGL(kern::kb_dir<double>, grid, blk, 0, s, vt, ds, st);
-        }
+        enqueue_iterations<double, false>(B, s);
     } else {
         hipLaunchKernelGGL(kern::kbm_init, grid, blk, 0, s, vt, ds, st, pt);
         hipLaunchKernelGGL(kern::kbm_fin_init, fin, blk, 0, s, rl, ds, st, pt);
-        for (int it = 0; it < B.o.iters_per_replay; ++it) {
-            elements(false);
-            hipLaunchKernelGGL(kern::kb_scatter<float>, grid, blk, 0, s, vt, ds, st, pt);
-            hipLaunchKernelGGL(kern::kb_fin_den<true>, fin, blk, 0, s, rl, ds, st, pt);
-            hipLaunchKernelGGL(kern::kbm_update, grid, blk, 0, s, vt, ds, st, pt);
-            hipLaunchKernelGGL(kern::kbm_fin_update, fin, blk, 0, s, rl, ds, st, pt);
-            if (it == B.o.iters_per_replay - 1) {
-                // refinement steps once per replay: a slot whose inner residual
-                // fell by delta waits in PH_RU (skipped by the inner kernels)
-                // until here, instead of every iteration launching the
-                // refinement kernels over all slots
-                hipLaunchKernelGGL(kern::kbm_ru_x, grid, blk, 0, s, vt, ds, st);
-                elements(true);
-                hipLaunchKernelGGL(kern::kbm_ru_res, grid, blk, 0, s, vt, ds, st, pt);
-                hipLaunchKernelGGL(kern::kbm_fin_ru, fin, blk, 0, s, rl, ds, st, pt);
-            }
-            hipLaunchKernelGGL(kern::kb_dir<float>, grid, blk, 0, s, vt, ds, st);
-        }
+        enqueue_iterations<float, true>(B, s);
     }
     H1PA_HIP(hipGetLastError());
 }
@@ -1164,6 +1393,7 @@ int batch_add(Batch &B, h1pa_form *form, const uint8_t *mask_src, const double *
     d.x = x;
     d.ne = sp.ne;
     d.n = n;
+    d.p = sp.p;
     // interior DOFs bypass the E-vector unless a constrained DOF may be interior
     d.bb = (!mask_src || mask_src == sp.ess_mask.p) ? sp.restr.bubble_begin : n;
     d.pa64 = f.pa_diff.p;

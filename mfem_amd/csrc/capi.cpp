@@ -269,7 +269,7 @@ int h1pa_space_create(h1pa_mesh *mesh, int order, h1pa_space **space) {
             h1_dof_map(order, dm.data());  // lex -> native
             r.lex2nat.upload(dm.data(), dm.size(), st);
             r.nedofs = s.nedofs;
-            kern::build_row_table(r, st);
+            kern::build_row_table(r, m.from_file, st);
         }
         auto *rh = new h1pa_restriction();
         rh->owned_by_space = true;

@@ -297,8 +297,9 @@ void list_to_mask(const int *list, int64_t nlist, uint8_t *mask, int64_t n, hipS
 void restrict_mult(int64_t nE, const int *gmap, const double *x, double *y, bool abs_,
                    hipStream_t s);
 // Fills r.row_tab (and r.indices_nat, r.row_over) of an H1 space's restriction
-// from its CSR table, lex2nat, perm and nedofs.
-void build_row_table(Restriction &r, hipStream_t s);
+// from its CSR table, lex2nat, perm and nedofs.  wide: the mesh may have rows
+// wider than their kind (every mesh but a Cartesian one).
+void build_row_table(Restriction &r, bool wide, hipStream_t s);
 // E -> L on a native-order E-vector over row positions [0, nrows): y = sum of
 // the row, or with a mask y[i] = mask[i] ? xin[i] : sum (DIAG_ONE).
 void scatter_rows(const Restriction &r, int64_t nrows, const double *ye, const uint8_t *mask,

@@ -417,7 +417,7 @@ __global__ void k_build_row_table(RowTab tb, int dof, const int *__restrict__ of
     }
     if (n > w) {
         p[0] = kRowOver;
-        over[0] = 1;
+        if (over) over[0] = 1;
     }
 }
 
@@ -610,18 +610,21 @@ void bubble_mult_transpose(int64_t ne, int D, int64_t bb, const double *xe, doub
     H1PA_HIP(hipGetLastError());
 }
 
-void build_row_table(Restriction &r, hipStream_t s) {
+void build_row_table(Restriction &r, bool wide, hipStream_t s) {
     const int64_t nv = r.nperm, nf = r.bubble_begin - nv - r.nedofs;
     r.row_tab.alloc(std::max<size_t>((size_t)(8 * nv + 4 * r.nedofs + 2 * nf), 1));
     r.row_over = 0;
-    StreamBuf<int> over(1, s);
-    H1PA_HIP(hipMemsetAsync(over.p, 0, sizeof(int), s));
+    StreamBuf<int> over;
+    if (wide) {
+        over.alloc(1, s);
+        H1PA_HIP(hipMemsetAsync(over.p, 0, sizeof(int), s));
+    }
     const RowTab tb = r.rows();
     hipLaunchKernelGGL(k_build_row_table, dim3(nblocks(r.bubble_begin)), dim3(kBlock), 0, s, tb,
                        (int)r.dof, r.offsets.p, r.indices.p, r.lex2nat.p, r.row_tab.p, over.p);
     H1PA_HIP(hipGetLastError());
     int h = 0;
-    H1PA_HIP(hipMemcpyAsync(&h, over.p, sizeof(int), hipMemcpyDeviceToHost, s));
+    if (wide) H1PA_HIP(hipMemcpyAsync(&h, over.p, sizeof(int), hipMemcpyDeviceToHost, s));
     H1PA_HIP(hipStreamSynchronize(s));
     if (h) {  // the wide rows are read from the native CSR table
         r.indices_nat.alloc((size_t)(r.ne * r.dof));
