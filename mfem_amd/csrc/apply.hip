@@ -39,7 +39,6 @@ __global__ void __launch_bounds__(NB * Q * Q, W)
 k_diffusion_apply(int64_t ne, const T *__restrict__ basis, const TP *__restrict__ pa,
                   const int *__restrict__ gmap, const uint8_t *__restrict__ mask,
                   const T *__restrict__ x, const EOutT<T> out, int accumulate) {
-    if (out.stop && *out.stop) return;  // solver already finished (block-uniform)
     __shared__ T smem[NB * diffusion_buf<D, Q>()];
     diffusion_elements<T, TP, D, Q, NB, U, K>((int64_t)blockIdx.x * NB, ne, basis, pa,
                                               gmap, mask, x, out, accumulate, smem);
@@ -50,7 +49,6 @@ __global__ void __launch_bounds__(NB * Q * Q)
 k_mass_apply(int64_t ne, const T *__restrict__ basis, const TP *__restrict__ pa,
              const int *__restrict__ gmap, const uint8_t *__restrict__ mask,
              const T *__restrict__ x, const EOutT<T> out, int accumulate) {
-    if (out.stop && *out.stop) return;
     __shared__ T smem[NB * D * Q * Q];
     mass_elements<T, TP, D, Q, NB>((int64_t)blockIdx.x * NB, ne, basis, pa, gmap, mask,
                                    x, out, accumulate, smem);

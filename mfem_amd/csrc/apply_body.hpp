@@ -244,6 +244,11 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
     const int64_t e = OM ? e0 : e0 + le;
     const bool valid = OM ? ne != 0 : e < ne;
     T *s = smem + le * BUF;
+    // Solver already finished: nothing is done; or (stop_late, small systems) the
+    // flag is tested after the first stage, so that its round trip is not ahead
+    // of all others.
+    const int stopped = out.stop ? *out.stop : 0;
+    if (!out.stop_late && stopped) return;  // block-uniform
     constexpr int KP = K > 0 ? ((K + 1) / 2 < R ? (K + 1) / 2 : R) : 0;  // pairs ahead
     const TP *pcol = pa + (int64_t)QQQ * 6 * (valid ? e : 0) + a + Q * b;
     // the 12 PA values of plane pair j: planes j and Q-1-j (the same plane
@@ -300,6 +305,7 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
         }
     }
     __syncthreads();
+    if (out.stop_late && stopped) return;
 
     // ---- forward y: thread (qx, dz) = (a, b); lines r0 = B_x u, r1 = G_x u
     {
@@ -607,6 +613,11 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
     const int64_t e = e0 + le;
     const bool valid = e < ne;
     T *s = smem + le * BUF;
+    // Solver already finished: nothing is done; or (stop_late, small systems) the
+    // flag is tested after the first stage, so that its round trip is not ahead
+    // of all others.
+    const int stopped = out.stop ? *out.stop : 0;
+    if (!out.stop_late && stopped) return;  // block-uniform
     // the column's Q PA values are loaded first, so that their round trip
     // overlaps the gather and the x and y stages instead of the z stage
     T pz[Q];
@@ -651,6 +662,7 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
         }
     }
     __syncthreads();
+    if (out.stop_late && stopped) return;
     // y: thread (qx, dz)
     {
         T re[HD > 0 ? HD : 1], ro[HD > 0 ? HD : 1], rm = T(0);
@@ -825,6 +837,11 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
     const int64_t e = OM ? e0 : e0 + le;
     const bool valid = OM ? ne != 0 : e < ne;
     T *s = smem + le * BUF;
+    // Solver already finished: nothing is done; or (stop_late, small systems) the
+    // flag is tested after the first stage, so that its round trip is not ahead
+    // of all others.
+    const int stopped = out.stop ? *out.stop : 0;
+    if (!out.stop_late && stopped) return;  // block-uniform
     constexpr int KK = K < Q ? K : Q;
     const TP *pcol = pa + (int64_t)QQQ * 6 * (valid ? e : 0) + a + Q * b;
     T ring[KK > 0 ? KK : 1][6];
@@ -858,6 +875,7 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
         }
     }
     __syncthreads();
+    if (out.stop_late && stopped) return;
 
     // ---- forward y: thread (qx, dz) = (a, b)
     {
@@ -1068,6 +1086,11 @@ mass_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, const 
     const int64_t e = e0 + le;
     const bool valid = e < ne;
     T *s = smem + le * BUF;
+    // Solver already finished: nothing is done; or (stop_late, small systems) the
+    // flag is tested after the first stage, so that its round trip is not ahead
+    // of all others.
+    const int stopped = out.stop ? *out.stop : 0;
+    if (!out.stop_late && stopped) return;  // block-uniform
     // the column's Q PA values first (their round trip overlaps the gather
     // and the x and y stages)
     T pz[Q];
@@ -1090,6 +1113,7 @@ mass_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, const 
         }
     }
     __syncthreads();
+    if (out.stop_late && stopped) return;
     {
         T r[D];
         const bool act = valid && b < D;

@@ -368,7 +368,8 @@ struct EOutT {
     T *yL = nullptr;
     int64_t bb = 0;
     const int *l2n = nullptr;
-    const int *stop = nullptr;  // device flag: when nonzero the launch does nothing
+    const int *stop = nullptr;  // device flag: when nonzero the launch stores nothing
+    int stop_late = 0;          // test it after the first stage, not before the first load
 };
 using EOut = EOutT<double>;
 // DomainLFIntegrator element vectors at q1d = p + 1: constant f, or f given
@@ -462,6 +463,7 @@ void pcg_solve(Form &f, const uint8_t *mask, const double *diag, const double *b
 struct PcgWork {
     DevBuf<double> r, z, d, q, partials;
     DevBuf<uint8_t> state;
+    std::shared_ptr<void> reader;  // of the state on the host, one look late (pcg.hip)
 };
 // Jacobi-PCG with the inverse diagonal given and the caller's work vectors.
 // prec = H1PA_PREC_BF16_PA applies the operator with the form's BF16 PA shadow

@@ -182,6 +182,44 @@ __device__ inline void sum_partials(const double *partials, int nb, double *sh,
     }
 }
 
+// Small systems: up to kFoldBlocks blocks of one entry per thread.  The blocks of
+// the kernel that needs a product sum its partials themselves -- four loads a
+// thread that go out with the kernel's other ones -- instead of a one-block
+// kernel of 3-4 us in between, and every load is issued before the first wait,
+// the test of `done` included.  Every block gets the same bits (same loads,
+// same order).  p = 3, 16^3 elements (117,649 DOFs), an iteration: six launches
+// of 29 us together -> four
+// of 22 (6.98 instead of 9.25 ms for a solve of 296 iterations).
+constexpr int kFoldBlocks = 4 * kThreads;
+inline bool small_system(const Chunks &c) { return c.per == 1 && c.blocks <= (unsigned)kFoldBlocks; }
+struct FoldSum {
+    double v[4];
+};
+__device__ __forceinline__ FoldSum fold_load(const double *__restrict__ partials, int nb) {
+    FoldSum f;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int i = u * kThreads + threadIdx.x;
+        const double v = partials[i < nb ? i : nb - 1];
+        f.v[u] = i < nb ? v : 0.0;
+    }
+    return f;
+}
+// Block sum: a butterfly within each wave, then the four wave totals in order.
+__device__ __forceinline__ double wave_block_sum(double v, double *sh) {
+    static_assert(kThreads == 256, "four 64-lane waves");
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    const double r = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+    __syncthreads();
+    return r;
+}
+__device__ __forceinline__ double fold_total(const FoldSum &f, double *sh) {
+    return wave_block_sum((f.v[0] + f.v[1]) + (f.v[2] + f.v[3]), sh);
+}
+
 template <typename T>
 __global__ void k_jacobi_dinv(int64_t n, const double *__restrict__ diag,
                               const uint8_t *__restrict__ mask, T *__restrict__ dinv) {
@@ -285,22 +323,23 @@ k_pcg_scatter(int64_t n, int per, int64_t bb, RowTab tb, const T *__restrict__ y
     store_partials<1>(acc, partials, sh);
 }
 
+// CGSolver's step after (A d, d): den = 0 or not finite ends the loop.
+__device__ __forceinline__ bool den_ends(double den) { return !isfinite(den) || den == 0.0; }
+__device__ __forceinline__ void write_den(PcgState *st, double den) {
+    st->den = den;
+    if (!den_ends(den)) return;
+    if (!isfinite(den)) st->nonfinite = 1;  // MFEM_VERIFY(IsFinite(den))
+    st->final_iter = st->in_loop ? st->iter : 0;
+    st->done = 1;
+}
+
 __global__ void __launch_bounds__(kThreads)
 k_pcg_fin_den(int nb, const double *__restrict__ partials, PcgState *st) {
     __shared__ double sh[kThreads];
     if (st->done) return;
     double tot[1];
     sum_partials<1>(partials, nb, sh, tot);
-    if (threadIdx.x != 0) return;
-    st->den = tot[0];
-    if (!isfinite(tot[0])) {  // MFEM_VERIFY(IsFinite(den))
-        st->done = 1;
-        st->nonfinite = 1;
-        st->final_iter = st->in_loop ? st->iter : 0;
-    } else if (tot[0] == 0.0) {  // CGSolver: den <= 0 and den == 0 ends the loop
-        st->done = 1;
-        st->final_iter = st->in_loop ? st->iter : 0;
-    }
+    if (threadIdx.x == 0) write_den(st, tot[0]);
 }
 
 template <typename T>
@@ -339,6 +378,96 @@ k_pcg_update(int64_t n, int per, const T *__restrict__ dinv, T *__restrict__ x, 
     store_partials<1>(acc, partials, sh);
 }
 
+// Small systems: the same three vector kernels, one entry a thread.
+// z = A d, DIAG_ONE rows copy d; partials of (d, z).
+template <typename T>
+__global__ void __launch_bounds__(kThreads)
+k_small_scatter(int n, int bb, RowTab tb, const T *__restrict__ ye,
+                const uint8_t *__restrict__ mask, const T *__restrict__ d, T *__restrict__ z,
+                double *__restrict__ pden, const PcgState *__restrict__ st) {
+    __shared__ double sh[4];
+    const int t = blockIdx.x * kThreads + threadIdx.x;
+    const int lt = t < n ? t : n - 1;
+    const int done = st->done;
+    const int i = row_dof(tb, lt);
+    const T vd = d[i];
+    const bool m = mask && mask[i];
+    T v = T(0);
+    if (lt < bb) {
+        const int t1[1] = {lt};
+        T v1[1];
+        rows_sum<1>(tb, t1, ye, v1);
+        v = m ? vd : v1[0];
+    } else {
+        v = z[i];  // interior DOF: written by the element kernel
+    }
+    if (done) return;
+    if (t < n && lt < bb) z[i] = v;
+    const double p = wave_block_sum(t < n ? (double)vd * (double)v : 0.0, sh);
+    if (threadIdx.x == 0) pden[blockIdx.x] = p;
+}
+
+// x += alpha d, r -= alpha z, z = dinv r; partials of (r, z).  Block 0 records
+// (A d, d); a block that finds `done` already set by it stops as it would on its
+// own total.
+template <typename T>
+__global__ void __launch_bounds__(kThreads)
+k_small_update(int n, const T *__restrict__ dinv, T *__restrict__ x, T *__restrict__ r,
+               T *__restrict__ z, const T *__restrict__ d, const double *__restrict__ pden,
+               double *__restrict__ prho, PcgState *st) {
+    __shared__ double sh[4];
+    const int t = blockIdx.x * kThreads + threadIdx.x;
+    const int j = t < n ? t : n - 1;
+    const int done = st->done;
+    const double nom = st->nom;
+    const FoldSum fs = fold_load(pden, gridDim.x);
+    const T vd = d[j], vx = x[j], vr = r[j], vz = z[j], vi = dinv[j];
+    if (done) return;
+    const double den = fold_total(fs, sh);
+    if (blockIdx.x == 0 && threadIdx.x == 0) write_den(st, den);
+    if (den_ends(den)) return;
+    const T alpha = (T)(nom / den);
+    const T ri = vr - alpha * vz, zi = vi * ri;
+    if (t < n) {
+        x[t] = vx + alpha * vd;
+        r[t] = ri;
+        z[t] = zi;
+    }
+    const double p = wave_block_sum(t < n ? (double)ri * (double)zi : 0.0, sh);
+    if (threadIdx.x == 0) prho[blockIdx.x] = p;
+}
+
+// CGSolver's step after betanom = (B r, r) of iteration `iter`.
+struct PcgStep {
+    int done, converged, nonfinite;
+};
+__device__ __forceinline__ PcgStep pcg_step(double betanom, double r0, int iter, int max_iter) {
+    if (!isfinite(betanom)) return {1, 0, 1};  // MFEM_VERIFY(IsFinite(betanom))
+    if (betanom < 0.0) return {1, 0, 0};
+    if (betanom <= r0) return {1, 1, 0};
+    return {iter + 1 > max_iter ? 1 : 0, 0, 0};
+}
+// o = the state after that step (o may be st)
+__device__ __forceinline__ void write_step(const PcgState &st, PcgState *o, double betanom,
+                                           const PcgStep &u) {
+    const int i = st.iter, max_iter = st.max_iter, final_iter = st.final_iter;
+    const double nom = st.nom, beta = st.beta;
+    o->nom0 = st.nom0;
+    o->den = st.den;
+    o->r0 = st.r0;
+    o->max_iter = max_iter;
+    o->in_loop = 1;
+    o->betanom = betanom;
+    o->converged = st.converged | u.converged;
+    o->nonfinite = st.nonfinite | u.nonfinite;
+    o->done = u.done;
+    o->beta = u.done ? beta : betanom / nom;
+    o->nom = u.done ? nom : betanom;
+    o->iter = u.done ? i : i + 1;
+    const bool limit = u.done && !u.nonfinite && !u.converged && !(betanom < 0.0);
+    o->final_iter = !u.done ? final_iter : limit ? max_iter : i;
+}
+
 __global__ void __launch_bounds__(kThreads)
 k_pcg_fin_update(int nb, const double *__restrict__ partials, PcgState *st) {
     __shared__ double sh[kThreads];
@@ -346,29 +475,34 @@ k_pcg_fin_update(int nb, const double *__restrict__ partials, PcgState *st) {
     double tot[1];
     sum_partials<1>(partials, nb, sh, tot);
     if (threadIdx.x != 0) return;
-    const double betanom = tot[0];
-    const int i = st->iter;
-    st->in_loop = 1;
-    st->betanom = betanom;
-    if (!isfinite(betanom)) {  // MFEM_VERIFY(IsFinite(betanom))
-        st->done = 1;
-        st->nonfinite = 1;
-        st->final_iter = i;
-    } else if (betanom < 0.0) {
-        st->done = 1;
-        st->final_iter = i;
-    } else if (betanom <= st->r0) {
-        st->done = 1;
-        st->converged = 1;
-        st->final_iter = i;
-    } else if (i + 1 > st->max_iter) {
-        st->done = 1;
-        st->final_iter = st->max_iter;
-    } else {
-        st->beta = betanom / st->nom;
-        st->nom = betanom;
-        st->iter = i + 1;
+    write_step(*st, st, tot[0], pcg_step(tot[0], st->r0, st->iter, st->max_iter));
+}
+
+// Small systems: d = z + beta d with the step after (B r, r); every block finds
+// beta, block 0 writes the new state to `next`, which the launches after this
+// one take (no block reads what another of this launch writes).
+template <typename T>
+__global__ void __launch_bounds__(kThreads)
+k_small_dir(int n, const T *__restrict__ z, T *__restrict__ d, const double *__restrict__ prho,
+            const PcgState *__restrict__ st, PcgState *__restrict__ next) {
+    __shared__ double sh[4];
+    const int t = blockIdx.x * kThreads + threadIdx.x;
+    const int j = t < n ? t : n - 1;
+    const int done = st->done, iter = st->iter, max_iter = st->max_iter;
+    const double nom = st->nom, r0 = st->r0;
+    const FoldSum fs = fold_load(prho, gridDim.x);
+    const T vz = z[j], vd = d[j];
+    const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+    if (done) {
+        if (writer) *next = *st;
+        return;
     }
+    const double rho = fold_total(fs, sh);
+    const PcgStep u = pcg_step(rho, r0, iter, max_iter);
+    if (writer) write_step(*st, next, rho, u);
+    if (u.done) return;
+    const T beta = (T)(rho / nom);
+    if (t < n) d[t] = vz + beta * vd;
 }
 
 template <typename T>
@@ -951,7 +1085,7 @@ int64_t direct_rows(const Space &sp, const uint8_t *mask) {
 }
 template <typename T>
 void pcg_element_apply(Form &f, int prec, const uint8_t *mask, const T *d, T *ye, T *yL,
-                       const int *stop, hipStream_t s) {
+                       const int *stop, hipStream_t s, bool stop_late = false) {
     Space &sp = *f.space;
     const bool diff = f.desc.integrators & H1PA_INTEG_DIFFUSION;
     const bool mass = f.desc.integrators & H1PA_INTEG_MASS;
@@ -959,6 +1093,7 @@ void pcg_element_apply(Form &f, int prec, const uint8_t *mask, const T *d, T *ye
     out.ye = ye;
     out.l2n = sp.restr.lex2nat.p;
     out.stop = stop;
+    out.stop_late = stop_late;
     // interior DOFs straight to the L-vector, or after the surface entries
     out.yL = yL ? yL : ye;
     out.bb = yL ? sp.restr.bubble_begin : sp.restr.native_bubble();
@@ -988,6 +1123,98 @@ void pcg_element_apply(Form &f, int prec, const uint8_t *mask, const T *d, T *ye
     }
 }
 
+// Reads a solve's state one exchange late: exchange() starts a copy of the
+// state into pinned memory and returns the one before it (a state that is not
+// done at first).  Each solve takes a pinned block and two events from a pool
+// of at most kKept idle ones per device, and gives them back when its copies
+// have ended.
+class StateReader {
+    struct Block {
+        PcgState *host = nullptr;  // two states, pinned
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        int dev = 0;
+        void release() {
+            for (hipEvent_t e : ev)
+                if (e) (void)hipEventDestroy(e);
+            if (host) (void)hipHostFree(host);
+        }
+    };
+    static constexpr size_t kKept = 64;
+    static std::mutex &mu() {
+        static std::mutex *m = new std::mutex;
+        return *m;
+    }
+    static std::vector<Block> &kept() {  // not destroyed at exit: the runtime may be gone
+        static std::vector<Block> *v = new std::vector<Block>;
+        return *v;
+    }
+    Block b_;
+    bool busy_[2] = {false, false};
+    int k_ = 0;
+    hipStream_t s_ = nullptr;
+    bool used_[2] = {false, false};  // a copy was issued (its event recorded)
+
+  public:
+    StateReader() {
+        int dev = 0;
+        H1PA_HIP(hipGetDevice(&dev));
+        {
+            std::lock_guard<std::mutex> g(mu());
+            std::vector<Block> &v = kept();
+            for (size_t i = v.size(); i-- > 0;)
+                if (v[i].dev == dev) {
+                    b_ = v[i];
+                    v.erase(v.begin() + (long)i);
+                    return;
+                }
+        }
+        b_.dev = dev;
+        hipError_t e = hipHostMalloc((void **)&b_.host, 2 * sizeof(PcgState), hipHostMallocDefault);
+        for (int k = 0; k < 2 && e == hipSuccess; ++k)
+            e = hipEventCreateWithFlags(&b_.ev[k], hipEventDisableTiming);
+        if (e != hipSuccess) {
+            b_.release();
+            H1PA_HIP(e);
+        }
+    }
+    StateReader(const StateReader &) = delete;
+    StateReader &operator=(const StateReader &) = delete;
+    ~StateReader() {
+        idle();
+        std::lock_guard<std::mutex> g(mu());
+        if (kept().size() < kKept) kept().push_back(b_);
+        else b_.release();
+    }
+    // A new solve on stream s: copies of the last one that are still under way
+    // come first on the same stream, and are waited for on another.
+    void begin(hipStream_t s) {
+        if (s != s_) idle();
+        busy_[0] = busy_[1] = false;
+        s_ = s;
+    }
+    PcgState exchange(const PcgState *st, hipStream_t s) {
+        PcgState h{};
+        H1PA_HIP(hipMemcpyAsync(b_.host + k_, st, sizeof(PcgState), hipMemcpyDeviceToHost, s));
+        H1PA_HIP(hipEventRecord(b_.ev[k_], s));
+        busy_[k_] = used_[k_] = true;
+        k_ ^= 1;
+        if (busy_[k_]) {
+            H1PA_HIP(hipEventSynchronize(b_.ev[k_]));
+            busy_[k_] = false;
+            h = b_.host[k_];
+        }
+        return h;
+    }
+    // Waits for the copies still under way.
+    void idle() {
+        for (int k = 0; k < 2; ++k)
+            if (used_[k]) {
+                (void)hipEventSynchronize(b_.ev[k]);
+                busy_[k] = used_[k] = false;
+            }
+    }
+};
+
 // Jacobi-PCG on the constrained operator with vectors of type T; dinv in T.
 template <typename T>
 void pcg_run(Form &f, int prec, const uint8_t *mask, const T *dinv, const T *b, T *x, T *ye,
@@ -1012,8 +1239,8 @@ void pcg_run(Form &f, int prec, const uint8_t *mask, const T *dinv, const T *b, 
                 ws->z.alloc(n);
                 ws->d.alloc(n);
             }
-            if (ws->partials.n < nb) ws->partials.alloc(nb);
-            if (ws->state.n < sizeof(PcgState)) ws->state.alloc(sizeof(PcgState));
+            if (ws->partials.n < 2 * nb) ws->partials.alloc(2 * nb);
+            if (ws->state.n < 2 * sizeof(PcgState)) ws->state.alloc(2 * sizeof(PcgState));
             r = ws->r.p;
             z = ws->z.p;
             d = ws->d.p;
@@ -1025,8 +1252,8 @@ void pcg_run(Form &f, int prec, const uint8_t *mask, const T *dinv, const T *b, 
         r_own.alloc(n, s);
         z_own.alloc(n, s);
         d_own.alloc(n, s);
-        part_own.alloc(nb, s);
-        st_own.alloc(1, s);
+        part_own.alloc(2 * (size_t)nb, s);
+        st_own.alloc(2, s);
         r = r_own.p;
         z = z_own.p;
         d = d_own.p;
@@ -1037,8 +1264,17 @@ void pcg_run(Form &f, int prec, const uint8_t *mask, const T *dinv, const T *b, 
     h.max_iter = o.max_iter;
     H1PA_HIP(hipMemcpyAsync(st, &h, sizeof(h), hipMemcpyHostToDevice, s));
     const int check = o.check_every > 0 ? o.check_every : 8;
-    const int *stop = &st->done;
     const dim3 grid(nb), blk(kern::kThreads), one(1);
+    const bool fold = kern::small_system(ch);
+    double *const pden = fold ? partials + nb : partials;
+    PcgState *next = st + 1;
+    std::shared_ptr<StateReader> reader;
+    if (fold) {
+        if (ws && ws->reader) reader = std::static_pointer_cast<StateReader>(ws->reader);
+        else reader = std::make_shared<StateReader>();
+        if (ws) ws->reader = reader;
+        reader->begin(s);
+    }
 
     auto t0 = std::chrono::steady_clock::now();
     hipLaunchKernelGGL(kern::k_pcg_init<T>, grid, blk, 0, s, n, per, b, dinv, x, r, z, d,
@@ -1046,29 +1282,55 @@ void pcg_run(Form &f, int prec, const uint8_t *mask, const T *dinv, const T *b, 
     hipLaunchKernelGGL(kern::k_pcg_fin_init, one, blk, 0, s, (int)nb, partials, st,
                        o.rel_tol, o.abs_tol);
     const int64_t bb = direct_rows(sp, mask);
+    const RowTab rows = sp.restr.rows();
     auto apply = [&]() {
-        pcg_element_apply<T>(f, prec, mask, d, ye, bb < n ? z : nullptr, stop, s);
-        hipLaunchKernelGGL(kern::k_pcg_scatter<T>, grid, blk, 0, s, n, per, bb, sp.restr.rows(), ye,
-                           mask, d, z, partials, st);
-        hipLaunchKernelGGL(kern::k_pcg_fin_den, one, blk, 0, s, (int)nb, partials, st);
+        pcg_element_apply<T>(f, prec, mask, d, ye, bb < n ? z : nullptr, &st->done, s, fold);
+        if (fold) {
+            hipLaunchKernelGGL(kern::k_small_scatter<T>, grid, blk, 0, s, (int)n, (int)bb, rows,
+                               ye, mask, d, z, pden, st);
+        } else {
+            hipLaunchKernelGGL(kern::k_pcg_scatter<T>, grid, blk, 0, s, n, per, bb, rows, ye,
+                               mask, d, z, pden, st);
+            hipLaunchKernelGGL(kern::k_pcg_fin_den, one, blk, 0, s, (int)nb, pden, st);
+        }
     };
     apply();
     H1PA_HIP(hipGetLastError());
     for (int it = 1; it <= o.max_iter; ++it) {
-        hipLaunchKernelGGL(kern::k_pcg_update<T>, grid, blk, 0, s, n, per, dinv, x, r, z, d,
-                           partials, st);
-        hipLaunchKernelGGL(kern::k_pcg_fin_update, one, blk, 0, s, (int)nb, partials, st);
-        hipLaunchKernelGGL(kern::k_pcg_dir<T>, grid, blk, 0, s, n, per, z, d, st);
+        if (fold) {
+            hipLaunchKernelGGL(kern::k_small_update<T>, grid, blk, 0, s, (int)n, dinv, x, r, z, d,
+                               pden, partials, st);
+            hipLaunchKernelGGL(kern::k_small_dir<T>, grid, blk, 0, s, (int)n, z, d, partials, st,
+                               next);
+            std::swap(st, next);
+        } else {
+            hipLaunchKernelGGL(kern::k_pcg_update<T>, grid, blk, 0, s, n, per, dinv, x, r, z, d,
+                               partials, st);
+            hipLaunchKernelGGL(kern::k_pcg_fin_update, one, blk, 0, s, (int)nb, partials, st);
+            hipLaunchKernelGGL(kern::k_pcg_dir<T>, grid, blk, 0, s, n, per, z, d, st);
+        }
         apply();
         H1PA_HIP(hipGetLastError());
         if (it % check == 0 || it == o.max_iter) {
-            H1PA_HIP(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
-            H1PA_HIP(hipStreamSynchronize(s));
+            if (!fold) {
+                H1PA_HIP(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
+                H1PA_HIP(hipStreamSynchronize(s));
+            } else {
+                // the state of `check` iterations ago is read while the last
+                // ones run, so the stream does not drain at every look; once
+                // it says done, what is queued behind it does nothing
+                h = reader->exchange(st, s);
+            }
             if (h.done) break;
         }
     }
-    H1PA_HIP(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
-    H1PA_HIP(hipStreamSynchronize(s));
+    if (!h.done) {
+        H1PA_HIP(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
+        H1PA_HIP(hipStreamSynchronize(s));
+    } else if (fold && !ws) {
+        // the caller may release the form's and its own memory after this
+        H1PA_HIP(hipStreamSynchronize(s));
+    }
     auto t1 = std::chrono::steady_clock::now();
     stats.converged = h.converged;
     stats.iterations = h.done ? h.final_iter : o.max_iter;
