@@ -329,11 +329,6 @@ void bubble_mult_transpose(int64_t ne, int D, int64_t bb, const double *xe, doub
 // basis at the order-ph GLL nodes.
 void first_entry_mask(int64_t nE, const int *gmap, const int *offsets, const int *indices,
                       uint8_t *emask, hipStream_t s);
-void transfer_prolong(int64_t ne, int pl, int ph, const double *B, const int *gmap_l,
-                      const int *gmap_h, const uint8_t *emask_h, const double *xl, double *yh,
-                      hipStream_t s);
-void transfer_restrict_e(int64_t ne, int pl, int ph, const double *B, const int *gmap_h,
-                         const uint8_t *emask_h, const double *xh, double *yle, hipStream_t s);
 // BooleanMask: ye[first E-entry of each row] = 1, every other E-entry 0.
 void boolean_mask(int64_t nrows, const int *offsets, const int *indices, double *ye,
                   hipStream_t s);
@@ -372,6 +367,13 @@ struct EOutT {
     int stop_late = 0;          // test it after the first stage, not before the first load
 };
 using EOut = EOutT<double>;
+// add: yh += the prolonged values, else set.
+void transfer_prolong(int64_t ne, int pl, int ph, const double *B, const int *gmap_l,
+                      const int *gmap_h, const uint8_t *emask_h, const double *xl, double *yh,
+                      bool add, hipStream_t s);
+void transfer_restrict_e(int64_t ne, int pl, int ph, const double *B, const int *gmap_h,
+                         const uint8_t *emask_h, const double *xh, const EOut &out,
+                         hipStream_t s);
 // DomainLFIntegrator element vectors at q1d = p + 1: constant f, or f given
 // per quadrature point (fq[q + (p+1)^3 e]) when fq is not null.
 void domain_lf(const Mesh &m, int p, double f, const double *fq, const EOut &out, hipStream_t s);
@@ -453,6 +455,11 @@ struct Chebyshev {
 void chebyshev_setup(Chebyshev &c, const double *d_diag, double max_eig, int power_iterations,
                      double power_tolerance, int power_seed, hipStream_t s);
 void chebyshev_mult(Chebyshev &c, const double *x, double *y, hipStream_t s);
+// y += S (x - A y) with the smoother's operator; z: scratch of its size.
+void chebyshev_smooth(Chebyshev &c, const double *x, double *y, double *z, hipStream_t s);
+// r = x - A y on f's DIAG_ONE constrained operator (prec as constrained_apply).
+void constrained_residual(Form &f, const uint8_t *mask, const double *x, const double *y,
+                          double *r, hipStream_t s, int prec);
 void pcg_chebyshev(Chebyshev &c, const double *b, double *x, const h1pa_pcg_opts &o,
                    h1pa_pcg_stats &stats, hipStream_t s);
 
@@ -507,7 +514,7 @@ struct Transfer {
     DevBuf<uint8_t> emask_h;  // BooleanMask of the high restriction, one byte per E-entry
     DevBuf<double> eL;        // low E-vector of the restriction
     Transfer(Space &lo, Space &hi, hipStream_t s);
-    void mult(const double *xl, double *yh, hipStream_t s);             // prolongation
+    void mult(const double *xl, double *yh, hipStream_t s, bool add = false);  // prolongation
     void mult_transpose(const double *xh, double *yl, hipStream_t s);   // restriction
 };
 struct MgLevel {

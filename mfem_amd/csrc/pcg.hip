@@ -854,16 +854,19 @@ k_cheb_first(int64_t n, int per, const double *__restrict__ dinv, const double *
 }
 
 // k >= 1: u = A t (constrained: interior rows written by the element kernel
-// into u, DIAG_ONE rows copy t); t = u * dinv; y += ck t
+// into u, DIAG_ONE rows copy t); t = u * dinv; y += ck t.  The last step (to
+// != null) stores no t, and its result goes to `to`: set, or with ADD added (a
+// smoothing step's correction, without a pass of its own).
+template <bool ADD>
 __global__ void __launch_bounds__(kThreads)
 k_cheb_scatter(int64_t n, int per, int64_t bb, RowTab tb, const double *__restrict__ ye,
                const uint8_t *__restrict__ mask, const double *__restrict__ dinv,
-               const double *__restrict__ u, double *__restrict__ t, double *__restrict__ y,
+               const double *__restrict__ u, double *__restrict__ t, double *y, double *to,
                double ck, const int *stop) {
     if (stop && *stop) return;
     H1PA_GROUPS(g, n) {
         int ii[kGrp];
-        double vi[kGrp], vy[kGrp], vt[kGrp], v[kGrp];
+        double vi[kGrp], vy[kGrp], vt[kGrp], vo[kGrp], v[kGrp];
         bool m[kGrp];
 #pragma unroll
         for (int k = 0; k < kGrp; ++k) {
@@ -872,6 +875,7 @@ k_cheb_scatter(int64_t n, int per, int64_t bb, RowTab tb, const double *__restri
             vi[k] = dinv[ii[k]];
             vy[k] = y[ii[k]];
             vt[k] = t[ii[k]];
+            if constexpr (ADD) vo[k] = to[ii[k]];
             m[k] = mask && mask[ii[k]];
         }
         group_rows(tb, bb, per, g, ii, ye, u, v);
@@ -880,8 +884,54 @@ k_cheb_scatter(int64_t n, int per, int64_t bb, RowTab tb, const double *__restri
             if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
             if (g.t[k] < bb && m[k]) v[k] = vt[k];
             const double ti = v[k] * vi[k];
-            t[ii[k]] = ti;
-            y[ii[k]] = vy[k] + ck * ti;
+            const double yi = vy[k] + ck * ti;
+            if (!to) {
+                t[ii[k]] = ti;
+                y[ii[k]] = yi;
+            } else if constexpr (ADD) {
+                to[ii[k]] = vo[k] + yi;
+            } else {
+                to[ii[k]] = yi;
+            }
+        }
+    }
+}
+
+// r = x - A y (A y from the element output, interior rows in u, DIAG_ONE rows
+// y).  FIRST: the smoother's first step on it, t = r * dinv and z = 0 + c0 t, and
+// r is not stored; else r is stored (it may be u).
+template <bool FIRST>
+__global__ void __launch_bounds__(kThreads)
+k_residual(int64_t n, int per, int64_t bb, RowTab tb, const double *__restrict__ ye,
+           const uint8_t *__restrict__ mask, const double *__restrict__ x,
+           const double *__restrict__ y, const double *u, const double *__restrict__ dinv,
+           double *r, double *__restrict__ z, double c0) {
+    H1PA_GROUPS(g, n) {
+        int ii[kGrp];
+        double vx[kGrp], vy[kGrp], vi[kGrp], v[kGrp];
+        bool m[kGrp];
+#pragma unroll
+        for (int k = 0; k < kGrp; ++k) {
+            if (k >= per) break;  // past this thread's entries
+            ii[k] = row_dof(tb, (int)g.lt[k]);
+            vx[k] = x[ii[k]];
+            vy[k] = y[ii[k]];
+            if constexpr (FIRST) vi[k] = dinv[ii[k]];
+            m[k] = mask && mask[ii[k]];
+        }
+        group_rows(tb, bb, per, g, ii, ye, u, v);
+#pragma unroll
+        for (int k = 0; k < kGrp; ++k) {
+            if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
+            if (g.t[k] < bb && m[k]) v[k] = vy[k];
+            const double ri = vx[k] - v[k];
+            if constexpr (FIRST) {
+                const double ti = ri * vi[k];
+                r[ii[k]] = ti;
+                z[ii[k]] = 0.0 + c0 * ti;
+            } else {
+                r[ii[k]] = ri;
+            }
         }
     }
 }
@@ -1616,23 +1666,39 @@ void chebyshev_coeffs(int order, double max_eig, double *c) {
     }
 }
 
-// y = sum_k c_k (D^-1 A)^k D^-1 x
-void chebyshev_apply(Chebyshev &c, const double *x, double *y, const int *stop, hipStream_t s) {
+// Steps 1 .. order-1 after the first (t in c.t, the sum so far in y): the last
+// one writes to `to`, added when `add`.
+void chebyshev_steps(Chebyshev &c, double *y, double *to, bool add, const int *stop,
+                     hipStream_t s) {
     Form &f = *c.f;
     Space &sp = *f.space;
     const int64_t n = sp.ndofs;
     const kern::Chunks ch = kern::chunks(n);
     const int64_t bb = direct_rows(sp, c.mask);
-    hipLaunchKernelGGL(kern::k_cheb_first, dim3(ch.blocks), dim3(kern::kThreads), 0, s, n, ch.per,
-                       c.dinv.p, x, c.t.p, y, c.coeffs[0], stop);
+    const RowTab rows = sp.restr.rows();
     for (int k = 1; k < c.order; ++k) {
+        const bool last = k == c.order - 1;
         pcg_element_apply<double>(f, c.prec, c.mask, c.t.p, f.ework0.p,
                                   bb < n ? c.u.p : nullptr, stop, s);
-        hipLaunchKernelGGL(kern::k_cheb_scatter, dim3(ch.blocks), dim3(kern::kThreads), 0, s, n,
-                           ch.per, bb, sp.restr.rows(), f.ework0.p, c.mask, c.dinv.p, c.u.p,
-                           c.t.p, y, c.coeffs[k], stop);
+        if (last && add)
+            hipLaunchKernelGGL(kern::k_cheb_scatter<true>, dim3(ch.blocks), dim3(kern::kThreads),
+                               0, s, n, ch.per, bb, rows, f.ework0.p, c.mask, c.dinv.p, c.u.p,
+                               c.t.p, y, to, c.coeffs[k], stop);
+        else
+            hipLaunchKernelGGL(kern::k_cheb_scatter<false>, dim3(ch.blocks), dim3(kern::kThreads),
+                               0, s, n, ch.per, bb, rows, f.ework0.p, c.mask, c.dinv.p, c.u.p,
+                               c.t.p, y, last ? to : nullptr, c.coeffs[k], stop);
     }
     H1PA_HIP(hipGetLastError());
+}
+
+// y = sum_k c_k (D^-1 A)^k D^-1 x
+void chebyshev_apply(Chebyshev &c, const double *x, double *y, const int *stop, hipStream_t s) {
+    const int64_t n = c.f->space->ndofs;
+    const kern::Chunks ch = kern::chunks(n);
+    hipLaunchKernelGGL(kern::k_cheb_first, dim3(ch.blocks), dim3(kern::kThreads), 0, s, n, ch.per,
+                       c.dinv.p, x, c.t.p, y, c.coeffs[0], stop);
+    chebyshev_steps(c, y, y, false, stop, s);
 }
 
 }  // namespace
@@ -1697,6 +1763,35 @@ void chebyshev_setup(Chebyshev &c, const double *d_diag, double max_eig, int pow
 
 void chebyshev_mult(Chebyshev &c, const double *x, double *y, hipStream_t s) {
     chebyshev_apply(c, x, y, nullptr, s);
+}
+
+// r = x - A y; interior rows of A y pass through r.
+void constrained_residual(Form &f, const uint8_t *mask, const double *x, const double *y,
+                          double *r, hipStream_t s, int prec) {
+    Space &sp = *f.space;
+    const int64_t n = sp.ndofs, bb = direct_rows(sp, mask);
+    const kern::Chunks ch = kern::chunks(n);
+    pcg_element_apply<double>(f, prec, mask, y, f.ework0.p, bb < n ? r : nullptr, nullptr, s);
+    hipLaunchKernelGGL(kern::k_residual<false>, dim3(ch.blocks), dim3(kern::kThreads), 0, s, n,
+                       ch.per, bb, sp.restr.rows(), f.ework0.p, mask, x, y, r, nullptr, r, nullptr,
+                       0.0);
+    H1PA_HIP(hipGetLastError());
+}
+
+// y += S (x - A y), S the smoother; z: scratch L-vector.
+void chebyshev_smooth(Chebyshev &c, const double *x, double *y, double *z, hipStream_t s) {
+    Form &f = *c.f;
+    Space &sp = *f.space;
+    const int64_t n = sp.ndofs, bb = direct_rows(sp, c.mask);
+    const kern::Chunks ch = kern::chunks(n);
+    pcg_element_apply<double>(f, c.prec, c.mask, y, f.ework0.p, bb < n ? c.u.p : nullptr, nullptr,
+                              s);
+    hipLaunchKernelGGL(kern::k_residual<true>, dim3(ch.blocks), dim3(kern::kThreads), 0, s, n,
+                       ch.per, bb, sp.restr.rows(), f.ework0.p, c.mask, x, y, c.u.p, c.dinv.p,
+                       c.t.p, z, c.coeffs[0]);
+    if (c.order == 1) kern::axpy(n, 1.0, z, y, s);
+    else chebyshev_steps(c, z, y, true, nullptr, s);
+    H1PA_HIP(hipGetLastError());
 }
 
 // CGSolver::Mult (solvers.cpp:869-1050, iterative_mode = false) with a

@@ -9,22 +9,20 @@
 // backwards.  Here the mask is a byte per E-entry, and since exactly one
 // masked entry of each high L-DOF is nonzero, the prolongation writes that
 // entry's value straight to the L-vector (no high E-vector, no sum: the sum
-// of one value and zeros is that value).  The restriction gathers the masked
-// high values, contracts them with B^T into the low E-vector (lexicographic)
-// and the low restriction's deterministic E->L sum finishes it.
+// of one value and zeros is that value), or adds it there (a cycle's
+// correction).  The restriction gathers the masked high values, contracts them
+// with B^T into the low E-vector (native layout, interior DOFs straight to the
+// result) and the low space's deterministic E->L sum finishes it.
 //
-// The contractions keep MFEM's association (x first, then y, then z, each an
-// ascending sum), so results differ from MFEM's only by fused multiply-add
-// rounding.
+// Each contraction is an ascending sum; the prolongation contracts x, y, z as
+// MFEM does, the restriction z, y, x, so results differ from MFEM's by rounding.
+#include "apply_body.hpp"
 #include "internal.hpp"
 
 namespace h1pa {
 namespace kern {
 
 namespace {
-
-constexpr int kThreads = 128;
-constexpr int kMaxD = 9;
 
 // emask[E] = 1 when E-index E is the first entry (indices order) of its
 // L-DOF's row: ElementRestriction::BooleanMask (fem/restriction.cpp:255-290)
@@ -40,89 +38,133 @@ __global__ void k_first_entry_mask(int64_t nE, const int *__restrict__ gmap,
     emask[i] = (first >= 0 ? first : -1 - first) == i ? 1 : 0;
 }
 
-// One work-group per element: low E-values (gathered) -> high node values.
-__global__ void __launch_bounds__(kThreads)
-k_prolong(int64_t ne, int Dl, int Dh, const double *__restrict__ B, const int *__restrict__ gmap_l,
+// Several elements per work-group, a Dh x Dh thread plane each, the orders
+// compiled in: x through LDS, y and z in registers of the thread's own column.
+// What bounds them is latency at the sizes of a cycle: 4913 elements, the three
+// transfers between orders 1, 2, 3 and 6 on average, prolongation 13.1 -> 6.3 us,
+// restriction 11.8 -> 4.8 us against one element of 128 threads per work-group
+// with run-time orders.
+template <int DL, int DH>
+constexpr int tr_nb() { return 256 / (DH * DH); }
+
+template <int DL, int DH>
+__global__ void __launch_bounds__(256)
+k_prolong(int64_t ne, const double *__restrict__ B, const int *__restrict__ gmap_l,
           const int *__restrict__ gmap_h, const uint8_t *__restrict__ emask_h,
-          const double *__restrict__ xl, double *__restrict__ yh) {
-    __shared__ double u[kMaxD * kMaxD * kMaxD];   // low values      [dz][dy][dx]
-    __shared__ double t1[kMaxD * kMaxD * kMaxD];  // x contracted    [dz][dy][qx]
-    __shared__ double t2[kMaxD * kMaxD * kMaxD];  // x, y contracted [dz][qy][qx]
-    __shared__ double Bs[kMaxD * kMaxD];          // B[qh + Dh dl]
-    const int64_t e = blockIdx.x;
-    if (e >= ne) return;
-    const int nl = Dl * Dl * Dl, nh = Dh * Dh * Dh;
-    for (int i = threadIdx.x; i < Dh * Dl; i += blockDim.x) Bs[i] = B[i];
-    for (int i = threadIdx.x; i < nl; i += blockDim.x) {
-        const int g = gmap_l[e * nl + i];
-        u[i] = g >= 0 ? xl[g] : -xl[-1 - g];
+          const double *__restrict__ xl, double *__restrict__ yh, int add) {
+    constexpr int NB = tr_nb<DL, DH>(), PL = DH * DH, NL = DL * DL * DL, NH = DH * DH * DH;
+    __shared__ double sB[DH * DL];                 // B[qh + Dh dl]
+    __shared__ double su[NB][NL], st[NB][DH * DL * DL];  // low values, x contracted
+    const int le = threadIdx.x / PL, t = threadIdx.x - le * PL;
+    const int a = t % DH, b = t / DH;
+    const int64_t e = (int64_t)blockIdx.x * NB + le;
+    const bool valid = le < NB && e < ne;
+    for (int i = threadIdx.x; i < DH * DL; i += blockDim.x) sB[i] = B[i];
+    int g[DH];
+    uint8_t m[DH];
+    if (valid) {
+#pragma unroll
+        for (int q = 0; q < DH; ++q) {
+            const int64_t E = e * NH + t + PL * q;
+            g[q] = gmap_h[E];
+            m[q] = emask_h[E];
+        }
+        for (int i = t; i < NL; i += PL) su[le][i] = xl[gmap_l[e * NL + i]];
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < Dh * Dl * Dl; i += blockDim.x) {
-        const int qx = i % Dh, r = i / Dh;  // r = dy + Dl dz
-        double v = 0.0;
-        for (int dx = 0; dx < Dl; ++dx) v += Bs[qx + Dh * dx] * u[dx + Dl * r];
-        t1[i] = v;
-    }
+    if (valid)
+        for (int r = b; r < DL * DL; r += DH) {  // r = dy + Dl dz
+            double v = 0.0;
+#pragma unroll
+            for (int d = 0; d < DL; ++d) v = fma(sB[a + DH * d], su[le][d + DL * r], v);
+            st[le][a + DH * r] = v;
+        }
     __syncthreads();
-    for (int i = threadIdx.x; i < Dh * Dh * Dl; i += blockDim.x) {
-        const int qx = i % Dh, qy = (i / Dh) % Dh, dz = i / (Dh * Dh);
-        double v = 0.0;
-        for (int dy = 0; dy < Dl; ++dy) v += Bs[qy + Dh * dy] * t1[qx + Dh * (dy + Dl * dz)];
-        t2[i] = v;
+    if (!valid) return;
+    double v[DH];
+#pragma unroll
+    for (int q = 0; q < DH; ++q) v[q] = 0.0;
+#pragma unroll
+    for (int dz = 0; dz < DL; ++dz) {
+        double c = 0.0;
+#pragma unroll
+        for (int dy = 0; dy < DL; ++dy)
+            c = fma(sB[b + DH * dy], st[le][a + DH * (dy + DL * dz)], c);
+#pragma unroll
+        for (int q = 0; q < DH; ++q) v[q] = fma(B[q + DH * dz], c, v[q]);
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < nh; i += blockDim.x) {
-        const int64_t E = e * nh + i;
-        if (!emask_h[E]) continue;
-        const int qxy = i % (Dh * Dh), qz = i / (Dh * Dh);
-        double v = 0.0;
-        for (int dz = 0; dz < Dl; ++dz) v += Bs[qz + Dh * dz] * t2[qxy + Dh * Dh * dz];
-        const int g = gmap_h[E];
-        if (g >= 0) yh[g] = v;
-        else yh[-1 - g] = -v;
+    if (add) {
+        double o[DH];
+#pragma unroll
+        for (int q = 0; q < DH; ++q) o[q] = m[q] ? yh[g[q]] : 0.0;
+#pragma unroll
+        for (int q = 0; q < DH; ++q)
+            if (m[q]) yh[g[q]] = o[q] + v[q];
+    } else {
+#pragma unroll
+        for (int q = 0; q < DH; ++q)
+            if (m[q]) yh[g[q]] = v[q];
     }
 }
 
-// One work-group per element: masked high values (gathered) -> low E-vector.
-__global__ void __launch_bounds__(kThreads)
-k_restrict(int64_t ne, int Dl, int Dh, const double *__restrict__ B, const int *__restrict__ gmap_h,
-           const uint8_t *__restrict__ emask_h, const double *__restrict__ xh,
-           double *__restrict__ yle) {
-    __shared__ double u[kMaxD * kMaxD * kMaxD];   // masked high values [qz][qy][qx]
-    __shared__ double t1[kMaxD * kMaxD * kMaxD];  // x contracted       [qz][qy][dx]
-    __shared__ double t2[kMaxD * kMaxD * kMaxD];  // x, y contracted    [qz][dy][dx]
-    __shared__ double Bs[kMaxD * kMaxD];
-    const int64_t e = blockIdx.x;
-    if (e >= ne) return;
-    const int nl = Dl * Dl * Dl, nh = Dh * Dh * Dh;
-    for (int i = threadIdx.x; i < Dh * Dl; i += blockDim.x) Bs[i] = B[i];
-    for (int i = threadIdx.x; i < nh; i += blockDim.x) {
-        const int64_t E = e * nh + i;
-        const int g = gmap_h[E];
-        const double v = g >= 0 ? xh[g] : -xh[-1 - g];
-        u[i] = emask_h[E] ? v : 0.0;
+template <int DL, int DH>
+__global__ void __launch_bounds__(256)
+k_restrict(int64_t ne, const double *__restrict__ B, const int *__restrict__ gmap_h,
+           const uint8_t *__restrict__ emask_h, const double *__restrict__ xh, const EOut out) {
+    constexpr int NB = tr_nb<DL, DH>(), PL = DH * DH, NH = DH * DH * DH;
+    __shared__ double ss[NB][DH * DH * DL];
+    const int le = threadIdx.x / PL, t = threadIdx.x - le * PL;
+    const int a = t % DH, b = t / DH;
+    const int64_t e = (int64_t)blockIdx.x * NB + le;
+    const bool valid = le < NB && e < ne;
+    if (valid) {  // z: thread (qx, qy)
+        int g[DH];
+        uint8_t m[DH];
+#pragma unroll
+        for (int q = 0; q < DH; ++q) {
+            const int64_t E = e * NH + t + PL * q;
+            g[q] = gmap_h[E];
+            m[q] = emask_h[E];
+        }
+        double u[DH];
+#pragma unroll
+        for (int q = 0; q < DH; ++q) u[q] = m[q] ? xh[g[q]] : 0.0;
+#pragma unroll
+        for (int dz = 0; dz < DL; ++dz) {
+            double c = 0.0;
+#pragma unroll
+            for (int q = 0; q < DH; ++q) c = fma(B[q + DH * dz], u[q], c);
+            ss[le][a + DH * (b + DH * dz)] = c;
+        }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < Dl * Dh * Dh; i += blockDim.x) {
-        const int dx = i % Dl, r = i / Dl;  // r = qy + Dh qz
-        double v = 0.0;
-        for (int qx = 0; qx < Dh; ++qx) v += Bs[qx + Dh * dx] * u[qx + Dh * r];
-        t1[i] = v;
-    }
+    const bool acty = valid && b < DL;  // y: thread (qx, dz)
+    double u[DH];
+    if (acty)
+#pragma unroll
+        for (int q = 0; q < DH; ++q) u[q] = ss[le][a + DH * (q + DH * b)];
     __syncthreads();
-    for (int i = threadIdx.x; i < Dl * Dl * Dh; i += blockDim.x) {
-        const int dx = i % Dl, dy = (i / Dl) % Dl, qz = i / (Dl * Dl);
-        double v = 0.0;
-        for (int qy = 0; qy < Dh; ++qy) v += Bs[qy + Dh * dy] * t1[dx + Dl * (qy + Dh * qz)];
-        t2[i] = v;
-    }
+    if (acty)
+#pragma unroll
+        for (int dy = 0; dy < DL; ++dy) {
+            double c = 0.0;
+#pragma unroll
+            for (int q = 0; q < DH; ++q) c = fma(B[q + DH * dy], u[q], c);
+            ss[le][a + DH * (dy + DL * b)] = c;
+        }
     __syncthreads();
-    for (int i = threadIdx.x; i < nl; i += blockDim.x) {
-        const int dxy = i % (Dl * Dl), dz = i / (Dl * Dl);
-        double v = 0.0;
-        for (int qz = 0; qz < Dh; ++qz) v += Bs[qz + Dh * dz] * t2[dxy + Dl * Dl * qz];
-        yle[e * nl + i] = v;
+    if (acty && a < DL) {  // x: thread (dy, dz)
+#pragma unroll
+        for (int q = 0; q < DH; ++q) u[q] = ss[le][q + DH * (a + DL * b)];
+        double yv[DL];
+#pragma unroll
+        for (int dx = 0; dx < DL; ++dx) {
+            double c = 0.0;
+#pragma unroll
+            for (int q = 0; q < DH; ++q) c = fma(B[q + DH * dx], u[q], c);
+            yv[dx] = c;
+        }
+        store_line<DL, double>(out, e, a, b, yv, 0);
     }
 }
 
@@ -136,23 +178,45 @@ void first_entry_mask(int64_t nE, const int *gmap, const int *offsets, const int
     H1PA_HIP(hipGetLastError());
 }
 
+// (pl + 1, ph + 1) pairs, pl < ph <= 8
+#define H1PA_TR_ALL(X)                                                                 \
+    X(2, 3) X(2, 4) X(2, 5) X(2, 6) X(2, 7) X(2, 8) X(2, 9) X(3, 4) X(3, 5) X(3, 6)    \
+    X(3, 7) X(3, 8) X(3, 9) X(4, 5) X(4, 6) X(4, 7) X(4, 8) X(4, 9) X(5, 6) X(5, 7)    \
+    X(5, 8) X(5, 9) X(6, 7) X(6, 8) X(6, 9) X(7, 8) X(7, 9) X(8, 9)
+
 void transfer_prolong(int64_t ne, int pl, int ph, const double *B, const int *gmap_l,
                       const int *gmap_h, const uint8_t *emask_h, const double *xl, double *yh,
-                      hipStream_t s) {
-    H1PA_CHECK(pl >= 1 && ph <= kMaxD - 1 && pl < ph, H1PA_EUNSUP, "transfer: orders");
+                      bool add, hipStream_t s) {
+    H1PA_CHECK(pl >= 1 && ph <= 8 && pl < ph, H1PA_EUNSUP, "transfer: orders");
     if (ne <= 0) return;
-    hipLaunchKernelGGL(k_prolong, dim3((unsigned)ne), dim3(kThreads), 0, s, ne, pl + 1, ph + 1, B,
-                       gmap_l, gmap_h, emask_h, xl, yh);
-    H1PA_HIP(hipGetLastError());
+#define X(L, H)                                                                              \
+    if (pl + 1 == L && ph + 1 == H) {                                                        \
+        constexpr int NB = tr_nb<L, H>();                                                    \
+        hipLaunchKernelGGL((k_prolong<L, H>), dim3((unsigned)((ne + NB - 1) / NB)),          \
+                           dim3(NB * H * H), 0, s, ne, B, gmap_l, gmap_h, emask_h, xl, yh,   \
+                           add ? 1 : 0);                                                     \
+        H1PA_HIP(hipGetLastError());                                                         \
+        return;                                                                              \
+    }
+    H1PA_TR_ALL(X)
+#undef X
 }
 
 void transfer_restrict_e(int64_t ne, int pl, int ph, const double *B, const int *gmap_h,
-                         const uint8_t *emask_h, const double *xh, double *yle, hipStream_t s) {
-    H1PA_CHECK(pl >= 1 && ph <= kMaxD - 1 && pl < ph, H1PA_EUNSUP, "transfer: orders");
+                         const uint8_t *emask_h, const double *xh, const EOut &out,
+                         hipStream_t s) {
+    H1PA_CHECK(pl >= 1 && ph <= 8 && pl < ph, H1PA_EUNSUP, "transfer: orders");
     if (ne <= 0) return;
-    hipLaunchKernelGGL(k_restrict, dim3((unsigned)ne), dim3(kThreads), 0, s, ne, pl + 1, ph + 1, B,
-                       gmap_h, emask_h, xh, yle);
-    H1PA_HIP(hipGetLastError());
+#define X(L, H)                                                                              \
+    if (pl + 1 == L && ph + 1 == H) {                                                        \
+        constexpr int NB = tr_nb<L, H>();                                                    \
+        hipLaunchKernelGGL((k_restrict<L, H>), dim3((unsigned)((ne + NB - 1) / NB)),         \
+                           dim3(NB * H * H), 0, s, ne, B, gmap_h, emask_h, xh, out);         \
+        H1PA_HIP(hipGetLastError());                                                         \
+        return;                                                                              \
+    }
+    H1PA_TR_ALL(X)
+#undef X
 }
 
 }  // namespace kern

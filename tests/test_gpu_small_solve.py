@@ -107,3 +107,54 @@ def test_threads_and_streams(h1pa, torch_cuda):
     for t in ts:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("order", [1, 2, 3])
+@pytest.mark.parametrize("pre,post,cycle", [(1, 1, "V"), (2, 2, "V"), (0, 1, "V"), (1, 0, "V"),
+                                            (1, 1, "W")])
+def test_cycle_is_its_public_pieces(h1pa, torch_cuda, order, pre, post, cycle):
+    """The fused two-level cycle against the same cycle composed of the public
+    operators, smoothers and transfers (rounding: 1e-12 on quantities that a
+    cycle amplifies by less than 100)."""
+    M, torch = h1pa, torch_cuda
+    s = _system(M, torch, 4, 3)
+    mesh, fes = s["mesh"], s["fes"]
+    mg = M.PMultigrid(s["a"], [1, 4], smoother_order=order, pre_smoothing=pre,
+                      post_smoothing=post, cycle=cycle, coarse_rel_tol=1e-12, coarse_max_iter=500)
+    lo = M.FiniteElementSpace(mesh, M.H1_FECollection(1, 3))
+    al = M.BilinearForm(lo)
+    al.SetAssemblyLevel(M.AssemblyLevel.PARTIAL)
+    al.AddDomainIntegrator(M.DiffusionIntegrator(M.SinCosCoefficient()))
+    al.Assemble()
+    essl, essh = lo.GetBoundaryTrueDofs(), fes.GetBoundaryTrueDofs()
+    Al = M.ConstrainedOperator(al, essl)
+    T = M.TransferOperator(lo, fes)
+    S = M.OperatorChebyshevSmoother(s["A"], None, essh, order)
+    cg = M.CGSolver()
+    cg.SetRelTol(1e-13)
+    cg.SetMaxIter(2000)
+    cg.SetOperator(Al)
+    cg.SetPreconditioner(M.OperatorJacobiSmoother(al, essl))
+
+    def apply(op, v, n):
+        out = torch.full((n,), float("nan"), dtype=torch.float64, device="cuda")
+        (op.MultTranspose if op is T else op.Mult)(v, out)
+        return out
+
+    N, n = fes.GetNDofs(), lo.GetNDofs()
+    x = s["b"]
+    y = torch.zeros_like(x)
+    for _ in range(pre):
+        y = y + apply(S, x - apply(s["A"], y, N), N)
+    r = apply(T, x - apply(s["A"], y, N), n)
+    c = torch.empty_like(r)
+    cg.Mult(r, c)
+    up = torch.empty_like(x)
+    T.Mult(c, up)
+    y = y + up
+    for _ in range(post):
+        y = y + apply(S, x - apply(s["A"], y, N), N)
+    got = torch.full_like(x, float("nan"))
+    mg.Mult(x, got)
+    # the coarse solves stop at 1e-12 and 1e-13 of their right-hand side
+    assert float((got - y).norm() / y.norm()) < 1e-9
