@@ -21,8 +21,9 @@
 //    is unrolled, the output-line loop is not: each iteration needs one row
 //    of the even-odd tables, loaded with wide scalar loads, so the SGPR file
 //    never spills;
-//  * one LDS buffer of max(2 D^2 Q, 3 D Q^2) values per element, reused
-//    across the stages with a barrier between the reads and the writes.
+//  * one LDS buffer of about max(2 D^2 Q, 3 D Q^2) values per element, padded
+//    against bank conflicts (ElemLds in apply_body.hpp) and reused across the
+//    stages with a barrier between the reads and the writes.
 //
 // basis layout: [ B(q,d) q-fastest | G q-fastest | B d-fastest | G d-fastest |
 //                 even-odd tables (EO<D, Q> in apply_body.hpp) ]; the diagonal
@@ -49,7 +50,7 @@ __global__ void __launch_bounds__(NB * Q * Q)
 k_mass_apply(int64_t ne, const T *__restrict__ basis, const TP *__restrict__ pa,
              const int *__restrict__ gmap, const uint8_t *__restrict__ mask,
              const T *__restrict__ x, const EOutT<T> out, int accumulate) {
-    __shared__ T smem[NB * D * Q * Q];
+    __shared__ T smem[NB * mass_buf<D, Q>()];
     mass_elements<T, TP, D, Q, NB>((int64_t)blockIdx.x * NB, ne, basis, pa, gmap, mask,
                                    x, out, accumulate, smem);
 }

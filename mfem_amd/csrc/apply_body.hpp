@@ -192,17 +192,50 @@ struct EO {
     static constexpr int SIZE = BG + (HD + OD) * RB;  // total basis length
 };
 
+// LDS strides of one element's stages.  x-lines (forward x to forward y, and
+// back): value (qx, dy, dz) at qx + XS dy + ZS dz; planes (y to z and back):
+// (qx, qy, dz) at qx + Q qy + ZP dz.  With XS = Q, ZS = D Q, ZP = Q^2 and an
+// even Q the threads of a wave, which step by XS or ZP, meet in few of the 32
+// eight-byte banks (Q = 8: eight threads at XS = 8 in four banks, four planes
+// at ZP = 64 in one).  Even Q therefore takes XS = Q + 1, ZS = Q (Q + 1), and
+// ZP = Q^2 padded, by at most Q, towards Q mod 32, which makes consecutive
+// threads read and write consecutive banks.  LDS cycles of a diffusion apply's
+// element group counted from the banks, 8-byte values (4-byte): Q = 8, D = 7
+// 3568 -> 1200 (2520 -> 600), Q = 10 2424 -> 1464, Q = 6 1960 -> 1520, Q = 4
+// 1200 -> 1120; an odd Q has few conflicts, and the same padding adds some.
+// Measured: p = 6 BF16-PA 40^3 element kernel 140 -> 135 us, 24 batched solves of
+// orders 2-6 21.7 -> 20.5 ms, p = 2 152k elements 112.5 -> 111 us an apply; the FP64
+// kernels from p = 4 on are bound by HBM or by latency elsewhere and did not move.
+template <int D, int Q>
+struct ElemLds {
+    static constexpr bool even = Q % 2 == 0;
+    static constexpr int to_q = (Q - Q * Q) & 31;  // from Q^2 up to Q modulo 32
+    static constexpr int XS = even ? Q + 1 : Q;
+    static constexpr int ZS = even ? Q * (Q + 1) : D * Q;
+    static constexpr int ZP = Q * Q + (even ? (to_q < Q ? to_q : Q) : 0);
+    static constexpr int XB = D * ZS, PB = D * ZP;  // one component
+};
+
+// LDS values per element of the diffusion body; OM 1 (see there) keeps the
+// element's D^3 results beside the last stage's lines.
+template <int D, int Q, int OM = 0>
+constexpr int diffusion_buf() {
+    using L = ElemLds<D, Q>;
+    constexpr int x = 2 * L::XB + (OM ? D * D * D : 0);
+    return x > 3 * L::PB ? x : 3 * L::PB;
+}
+// ... and of the mass body.
+template <int D, int Q>
+constexpr int mass_buf() {
+    using L = ElemLds<D, Q>;
+    return L::XB > L::PB ? L::XB : L::PB;
+}
+
 // U: unroll factor of the output-line loops (1 or 2).
 // K: PA-data pipeline depth in z-planes.  0: the 12 values of a plane pair
 //    are loaded in its own iteration.  K > 0: (K+1)/2 plane pairs are loaded
 //    at kernel entry (their latency hides behind the x/y stages) and pair
 //    j + (K+1)/2 is issued while pair j is computed.
-// LDS doubles (or floats) per element of the diffusion body.
-template <int D, int Q>
-constexpr int diffusion_buf() {
-    return (2 * D * D * Q > 3 * D * Q * Q) ? 2 * D * D * Q : 3 * D * Q * Q;
-}
-
 // Waves per SIMD that the LDS of an NB-element diffusion block allows: a CU's
 // 160 KiB holds floor(160 KiB / block LDS) blocks, each putting ceil(waves/4)
 // waves on every SIMD.  Used as the minimum-waves launch bound of the
@@ -220,7 +253,7 @@ constexpr int lds_waves() {
 // The elements e0 + (threadIdx.x / Q^2), NB per work-group, of one problem.
 // OM (output mode) 0: the element result goes to `out` (store_line).  OM 1
 // (the column-sweep apply): e0 is this thread's element itself, valid when
-// ne != 0; the element's D^3 results are left in LDS at s + 2 D^2 Q in
+// ne != 0; the element's D^3 results are left in LDS at s + 2 XB in
 // lexicographic order (a region the last stage does not read) and its gather
 // indices at sg + le D^3; `out` is not used.
 template <typename T, typename TP, int D, int Q, int NB, int U, int K, int OM = 0>
@@ -232,8 +265,9 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
     using E = EO<D, Q>;
     constexpr int HD = E::HD, OD = E::OD, HQ = E::HQ, R = E::R, W = E::W, RB = E::RB;
     constexpr int QQ = Q * Q, QQQ = Q * Q * Q, DDD = D * D * D;
-    constexpr int DDQ = D * D * Q, DQQ = D * Q * Q;
-    constexpr int BUF = diffusion_buf<D, Q>();
+    using L = ElemLds<D, Q>;
+    constexpr int XS = L::XS, ZS = L::ZS, ZP = L::ZP, XB = L::XB, PB = L::PB;
+    constexpr int BUF = diffusion_buf<D, Q, OM>();
     const T *__restrict__ FBt = basis + E::FB;  // forward rows of B
     const T *__restrict__ FGt = basis + E::FG;  // forward rows of G
     const T *__restrict__ BBt = basis + E::BB;  // backward rows of B
@@ -283,7 +317,7 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
             }
             if constexpr (OD) um = u[HD];
         }
-        T *o = s + Q * (a + D * b);
+        T *o = s + XS * a + ZS * b;
 #pragma unroll U
         for (int q = 0; q < R; ++q) {
             const T *fb = FBt + W * q, *fg = FGt + W * q;
@@ -297,10 +331,10 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
                 Cg = fma(fg[HD + d], uo[d], Cg);
             }
             o[q] = Ab + Cb;
-            o[DDQ + q] = Ag + Cg;
+            o[XB + q] = Ag + Cg;
             if (q < HQ) {
                 o[Q - 1 - q] = Ab - Cb;
-                o[DDQ + Q - 1 - q] = Cg - Ag;
+                o[XB + Q - 1 - q] = Cg - Ag;
             }
         }
     }
@@ -315,16 +349,16 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
         if (act) {
 #pragma unroll
             for (int d = 0; d < HD; ++d) {
-                const T p0 = s[a + Q * (d + D * b)], q0 = s[a + Q * (D - 1 - d + D * b)];
-                const T p1 = s[DDQ + a + Q * (d + D * b)], q1 = s[DDQ + a + Q * (D - 1 - d + D * b)];
+                const T p0 = s[a + XS * d + ZS * b], q0 = s[a + XS * (D - 1 - d) + ZS * b];
+                const T p1 = s[XB + a + XS * d + ZS * b], q1 = s[XB + a + XS * (D - 1 - d) + ZS * b];
                 r0e[d] = p0 + q0;
                 r0o[d] = p0 - q0;
                 r1e[d] = p1 + q1;
                 r1o[d] = p1 - q1;
             }
             if constexpr (OD) {
-                r0m = s[a + Q * (HD + D * b)];
-                r1m = s[DDQ + a + Q * (HD + D * b)];
+                r0m = s[a + XS * HD + ZS * b];
+                r1m = s[XB + a + XS * HD + ZS * b];
             }
         }
         __syncthreads();
@@ -345,15 +379,15 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
                     C1 = fma(fb[HD + d], r1o[d], C1);
                 }
                 // bb = B_y B_x u (-> d/dz), gb = G_y B_x u (-> d/dy), bg = B_y G_x u (-> d/dx)
-                T *o = s + a + Q * (q + Q * b);
-                o[0 * DQQ] = A1 + C1;
-                o[1 * DQQ] = G0 + H0;
-                o[2 * DQQ] = A0 + C0;
+                T *o = s + a + Q * q + ZP * b;
+                o[0 * PB] = A1 + C1;
+                o[1 * PB] = G0 + H0;
+                o[2 * PB] = A0 + C0;
                 if (q < HQ) {
-                    T *o2 = s + a + Q * (Q - 1 - q + Q * b);
-                    o2[0 * DQQ] = A1 - C1;
-                    o2[1 * DQQ] = H0 - G0;
-                    o2[2 * DQQ] = A0 - C0;
+                    T *o2 = s + a + Q * (Q - 1 - q) + ZP * b;
+                    o2[0 * PB] = A1 - C1;
+                    o2[1 * PB] = H0 - G0;
+                    o2[2 * PB] = A0 - C0;
                 }
             }
         }
@@ -368,20 +402,20 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
         if (valid) {
 #pragma unroll
             for (int d = 0; d < HD; ++d) {
-                const T *i = s + a + Q * (b + Q * d);
-                const T *k = s + a + Q * (b + Q * (D - 1 - d));
-                z0e[d] = i[0 * DQQ] + k[0 * DQQ];
-                z0o[d] = i[0 * DQQ] - k[0 * DQQ];
-                z1e[d] = i[1 * DQQ] + k[1 * DQQ];
-                z1o[d] = i[1 * DQQ] - k[1 * DQQ];
-                z2e[d] = i[2 * DQQ] + k[2 * DQQ];
-                z2o[d] = i[2 * DQQ] - k[2 * DQQ];
+                const T *i = s + a + Q * b + ZP * d;
+                const T *k = s + a + Q * b + ZP * (D - 1 - d);
+                z0e[d] = i[0 * PB] + k[0 * PB];
+                z0o[d] = i[0 * PB] - k[0 * PB];
+                z1e[d] = i[1 * PB] + k[1 * PB];
+                z1o[d] = i[1 * PB] - k[1 * PB];
+                z2e[d] = i[2 * PB] + k[2 * PB];
+                z2o[d] = i[2 * PB] - k[2 * PB];
             }
             if constexpr (OD) {
-                const T *i = s + a + Q * (b + Q * HD);
-                z0m = i[0 * DQQ];
-                z1m = i[1 * DQQ];
-                z2m = i[2 * DQQ];
+                const T *i = s + a + Q * b + ZP * HD;
+                z0m = i[0 * PB];
+                z1m = i[1 * PB];
+                z2m = i[2 * PB];
             }
         }
         __syncthreads();
@@ -464,20 +498,20 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
             }
 #pragma unroll
             for (int d = 0; d < HD; ++d) {
-                T *o = s + a + Q * (b + Q * d);
-                T *k = s + a + Q * (b + Q * (D - 1 - d));
-                o[0 * DQQ] = E0[d] + F0[d];
-                k[0 * DQQ] = E0[d] - F0[d];
-                o[1 * DQQ] = E1[d] + F1[d];
-                k[1 * DQQ] = E1[d] - F1[d];
-                o[2 * DQQ] = E2[d] + F2[d];
-                k[2 * DQQ] = E2[d] - F2[d];
+                T *o = s + a + Q * b + ZP * d;
+                T *k = s + a + Q * b + ZP * (D - 1 - d);
+                o[0 * PB] = E0[d] + F0[d];
+                k[0 * PB] = E0[d] - F0[d];
+                o[1 * PB] = E1[d] + F1[d];
+                k[1 * PB] = E1[d] - F1[d];
+                o[2 * PB] = E2[d] + F2[d];
+                k[2 * PB] = E2[d] - F2[d];
             }
             if constexpr (OD) {
-                T *o = s + a + Q * (b + Q * HD);
-                o[0 * DQQ] = M0;
-                o[1 * DQQ] = M1;
-                o[2 * DQQ] = M2;
+                T *o = s + a + Q * b + ZP * HD;
+                o[0 * PB] = M0;
+                o[1 * PB] = M1;
+                o[2 * PB] = M2;
             }
         }
     }
@@ -491,19 +525,19 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
         if (act) {
 #pragma unroll
             for (int j = 0; j < R; ++j) {
-                const T *i = s + a + Q * (j + Q * b);
+                const T *i = s + a + Q * j + ZP * b;
                 if (j < HQ) {
-                    const T *k = s + a + Q * (Q - 1 - j + Q * b);
-                    P0[j] = i[0 * DQQ] + k[0 * DQQ];
-                    N0[j] = i[0 * DQQ] - k[0 * DQQ];
-                    P1[j] = i[1 * DQQ] - k[1 * DQQ];  // G
-                    N1[j] = i[1 * DQQ] + k[1 * DQQ];
-                    P2[j] = i[2 * DQQ] + k[2 * DQQ];
-                    N2[j] = i[2 * DQQ] - k[2 * DQQ];
+                    const T *k = s + a + Q * (Q - 1 - j) + ZP * b;
+                    P0[j] = i[0 * PB] + k[0 * PB];
+                    N0[j] = i[0 * PB] - k[0 * PB];
+                    P1[j] = i[1 * PB] - k[1 * PB];  // G
+                    N1[j] = i[1 * PB] + k[1 * PB];
+                    P2[j] = i[2 * PB] + k[2 * PB];
+                    N2[j] = i[2 * PB] - k[2 * PB];
                 } else {
-                    P0[j] = N0[j] = i[0 * DQQ];
-                    P1[j] = N1[j] = i[1 * DQQ];
-                    P2[j] = N2[j] = i[2 * DQQ];
+                    P0[j] = N0[j] = i[0 * PB];
+                    P1[j] = N1[j] = i[1 * PB];
+                    P2[j] = N2[j] = i[2 * PB];
                 }
             }
         }
@@ -523,10 +557,10 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
                         Eb = fma(bb[j], P2[j], Eb);
                         Fb = fma(bb[R + j], N2[j], Fb);
                     }
-                    s[a + Q * (d + D * b)] = Ea + Fa;
-                    s[a + Q * (D - 1 - d + D * b)] = Ea - Fa;
-                    s[DDQ + a + Q * (d + D * b)] = Eb + Fb;
-                    s[DDQ + a + Q * (D - 1 - d + D * b)] = Eb - Fb;
+                    s[a + XS * d + ZS * b] = Ea + Fa;
+                    s[a + XS * (D - 1 - d) + ZS * b] = Ea - Fa;
+                    s[XB + a + XS * d + ZS * b] = Eb + Fb;
+                    s[XB + a + XS * (D - 1 - d) + ZS * b] = Eb - Fb;
                 } else {  // middle d of an odd D
 #pragma unroll
                     for (int j = 0; j < R; ++j) {
@@ -534,8 +568,8 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
                         Eb = fma(bg[j], P1[j], Eb);
                         Eb = fma(bb[j], P2[j], Eb);
                     }
-                    s[a + Q * (d + D * b)] = Ea;
-                    s[DDQ + a + Q * (d + D * b)] = Eb;
+                    s[a + XS * d + ZS * b] = Ea;
+                    s[XB + a + XS * d + ZS * b] = Eb;
                 }
             }
         }
@@ -545,19 +579,19 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
     // ---- backward x: thread (dy, dz) = (a, b); v = G_x^T sa + B_x^T sb
     if (valid && a < D && b < D) {
         T Pa[R], Na[R], Pb[R], Nb[R];
-        const T *in = s + Q * (a + D * b);
+        const T *in = s + XS * a + ZS * b;
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             if (j < HQ) {
                 const T sa0 = in[j], sa1 = in[Q - 1 - j];
-                const T sb0 = in[DDQ + j], sb1 = in[DDQ + Q - 1 - j];
+                const T sb0 = in[XB + j], sb1 = in[XB + Q - 1 - j];
                 Pa[j] = sa0 - sa1;  // G
                 Na[j] = sa0 + sa1;
                 Pb[j] = sb0 + sb1;  // B
                 Nb[j] = sb0 - sb1;
             } else {
                 Pa[j] = Na[j] = in[j];
-                Pb[j] = Nb[j] = in[DDQ + j];
+                Pb[j] = Nb[j] = in[XB + j];
             }
         }
         T yv[D];
@@ -587,7 +621,7 @@ diffusion_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const
         if constexpr (OM == 0) {
             store_line<D, T>(out, e, a, b, yv, accumulate);
         } else {
-            T *o = s + 2 * DDQ + D * (a + D * b);
+            T *o = s + 2 * XB + D * (a + D * b);
 #pragma unroll
             for (int dx = 0; dx < D; ++dx) o[dx] = yv[dx];
         }
@@ -603,8 +637,8 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
     using E = EO<D, Q>;
     constexpr int HD = E::HD, OD = E::OD, HQ = E::HQ, R = E::R, W = E::W, RB = E::RB;
     constexpr int QQ = Q * Q, QQQ = Q * Q * Q, DDD = D * D * D;
-    constexpr int DQQ = D * Q * Q;
-    constexpr int BUF = DQQ;
+    using L = ElemLds<D, Q>;
+    constexpr int XS = L::XS, ZS = L::ZS, ZP = L::ZP, BUF = mass_buf<D, Q>();
     const T *__restrict__ FBt = basis + E::FB;
     const T *__restrict__ BBt = basis + E::BB;
     const int le = threadIdx.x / QQ;
@@ -657,8 +691,8 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
         for (int q = 0; q < R; ++q) {
             T lo, hi;
             fwd(ue, uo, um, q, lo, hi);
-            s[q + Q * (a + D * b)] = lo;
-            if (q < HQ) s[Q - 1 - q + Q * (a + D * b)] = hi;
+            s[q + XS * a + ZS * b] = lo;
+            if (q < HQ) s[Q - 1 - q + XS * a + ZS * b] = hi;
         }
     }
     __syncthreads();
@@ -670,11 +704,11 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
         if (act) {
 #pragma unroll
             for (int d = 0; d < HD; ++d) {
-                const T p = s[a + Q * (d + D * b)], k = s[a + Q * (D - 1 - d + D * b)];
+                const T p = s[a + XS * d + ZS * b], k = s[a + XS * (D - 1 - d) + ZS * b];
                 re[d] = p + k;
                 ro[d] = p - k;
             }
-            if constexpr (OD) rm = s[a + Q * (HD + D * b)];
+            if constexpr (OD) rm = s[a + XS * HD + ZS * b];
         }
         __syncthreads();
         if (act)
@@ -682,8 +716,8 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
             for (int q = 0; q < R; ++q) {
                 T lo, hi;
                 fwd(re, ro, rm, q, lo, hi);
-                s[a + Q * (q + Q * b)] = lo;
-                if (q < HQ) s[a + Q * (Q - 1 - q + Q * b)] = hi;
+                s[a + Q * q + ZP * b] = lo;
+                if (q < HQ) s[a + Q * (Q - 1 - q) + ZP * b] = hi;
             }
     }
     __syncthreads();
@@ -693,11 +727,11 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
         if (valid) {
 #pragma unroll
             for (int d = 0; d < HD; ++d) {
-                const T p = s[a + Q * (b + Q * d)], k = s[a + Q * (b + Q * (D - 1 - d))];
+                const T p = s[a + Q * b + ZP * d], k = s[a + Q * b + ZP * (D - 1 - d)];
                 ze[d] = p + k;
                 zo[d] = p - k;
             }
-            if constexpr (OD) zm = s[a + Q * (b + Q * HD)];
+            if constexpr (OD) zm = s[a + Q * b + ZP * HD];
         }
         __syncthreads();
         if (valid) {
@@ -727,10 +761,10 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
             }
 #pragma unroll
             for (int d = 0; d < HD; ++d) {
-                s[a + Q * (b + Q * d)] = Ez[d] + Fz[d];
-                s[a + Q * (b + Q * (D - 1 - d))] = Ez[d] - Fz[d];
+                s[a + Q * b + ZP * d] = Ez[d] + Fz[d];
+                s[a + Q * b + ZP * (D - 1 - d)] = Ez[d] - Fz[d];
             }
-            if constexpr (OD) s[a + Q * (b + Q * HD)] = Mz;
+            if constexpr (OD) s[a + Q * b + ZP * HD] = Mz;
         }
     }
     __syncthreads();
@@ -759,9 +793,9 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
         if (act) {
 #pragma unroll
             for (int j = 0; j < R; ++j) {
-                const T v0 = s[a + Q * (j + Q * b)];
+                const T v0 = s[a + Q * j + ZP * b];
                 if (j < HQ) {
-                    const T v1 = s[a + Q * (Q - 1 - j + Q * b)];
+                    const T v1 = s[a + Q * (Q - 1 - j) + ZP * b];
                     P[j] = v0 + v1;
                     N[j] = v0 - v1;
                 } else {
@@ -775,15 +809,15 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
             for (int d = 0; d < HD + OD; ++d) {
                 T lo, hi;
                 bwd(P, N, d, lo, hi);
-                s[a + Q * (d + D * b)] = lo;
-                if (d < HD) s[a + Q * (D - 1 - d + D * b)] = hi;
+                s[a + XS * d + ZS * b] = lo;
+                if (d < HD) s[a + XS * (D - 1 - d) + ZS * b] = hi;
             }
     }
     __syncthreads();
     // x^T: thread (dy, dz)
     if (valid && a < D && b < D) {
         T P[R], N[R];
-        const T *in = s + Q * (a + D * b);
+        const T *in = s + XS * a + ZS * b;
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             if (j < HQ) {
@@ -815,7 +849,7 @@ mass_elements_eo(int64_t e0, int64_t ne, const T *__restrict__ basis, const TP *
 // The elements e0 + (threadIdx.x / Q^2), NB per work-group, of one problem.
 // OM (output mode) 0: the element result goes to `out` (store_line).  OM 1
 // (the column-sweep apply): e0 is this thread's element itself, valid when
-// ne != 0; the element's D^3 results are left in LDS at s + 2 D^2 Q in
+// ne != 0; the element's D^3 results are left in LDS at s + 2 XB in
 // lexicographic order (a region the last stage does not read) and its gather
 // indices at sg + le D^3; `out` is not used.
 template <typename T, typename TP, int D, int Q, int NB, int U, int K, int OM = 0>
@@ -825,8 +859,9 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
                    const T *__restrict__ x, const EOutT<T> &out, int accumulate,
                    T *__restrict__ smem, int *__restrict__ sg = nullptr) {
     constexpr int QQ = Q * Q, QQQ = Q * Q * Q, DDD = D * D * D;
-    constexpr int DDQ = D * D * Q, DQQ = D * Q * Q;
-    constexpr int BUF = diffusion_buf<D, Q>();
+    using L = ElemLds<D, Q>;
+    constexpr int XS = L::XS, ZS = L::ZS, ZP = L::ZP, XB = L::XB, PB = L::PB;
+    constexpr int BUF = diffusion_buf<D, Q, OM>();
     const T *__restrict__ Bq = basis;              // B[q + Q d]
     const T *__restrict__ Gq = basis + Q * D;
     const T *__restrict__ Bd = basis + 2 * Q * D;  // B[d + D q]
@@ -860,7 +895,7 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
         const int64_t base = (int64_t)DDD * e + D * (a + D * b);
         load_line<D, T, OM == 1>(gmap, mask, x, base, u,
                                      OM == 1 ? sg + le * DDD + D * (a + D * b) : nullptr);
-        T *out = s + Q * (a + D * b);
+        T *out = s + XS * a + ZS * b;
 #pragma unroll U
         for (int qx = 0; qx < Q; ++qx) {
             const T *br = Bd + D * qx, *gr = Gd + D * qx;
@@ -871,7 +906,7 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
                 gu = fma(gr[dx], u[dx], gu);
             }
             out[qx] = bu;
-            out[DDQ + qx] = gu;
+            out[XB + qx] = gu;
         }
     }
     __syncthreads();
@@ -884,8 +919,8 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
         if (act) {
 #pragma unroll
             for (int dy = 0; dy < D; ++dy) {
-                r0[dy] = s[a + Q * (dy + D * b)];
-                r1[dy] = s[DDQ + a + Q * (dy + D * b)];
+                r0[dy] = s[a + XS * dy + ZS * b];
+                r1[dy] = s[XB + a + XS * dy + ZS * b];
             }
         }
         __syncthreads();
@@ -900,10 +935,10 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
                     gb = fma(gr[dy], r0[dy], gb);
                     bg = fma(br[dy], r1[dy], bg);
                 }
-                T *o = s + a + Q * (qy + Q * b);
-                o[0 * DQQ] = bg;  // -> d/dx
-                o[1 * DQQ] = gb;  // -> d/dy
-                o[2 * DQQ] = bb;  // -> d/dz
+                T *o = s + a + Q * qy + ZP * b;
+                o[0 * PB] = bg;  // -> d/dx
+                o[1 * PB] = gb;  // -> d/dy
+                o[2 * PB] = bb;  // -> d/dz
             }
         }
     }
@@ -915,10 +950,10 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
         if (valid) {
 #pragma unroll
             for (int dz = 0; dz < D; ++dz) {
-                const T *i = s + a + Q * (b + Q * dz);
-                z0[dz] = i[0 * DQQ];
-                z1[dz] = i[1 * DQQ];
-                z2[dz] = i[2 * DQQ];
+                const T *i = s + a + Q * b + ZP * dz;
+                z0[dz] = i[0 * PB];
+                z1[dz] = i[1 * PB];
+                z2[dz] = i[2 * PB];
             }
         }
         __syncthreads();
@@ -963,10 +998,10 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
             }
 #pragma unroll
             for (int dz = 0; dz < D; ++dz) {
-                T *o = s + a + Q * (b + Q * dz);
-                o[0 * DQQ] = T0[dz];
-                o[1 * DQQ] = T1[dz];
-                o[2 * DQQ] = T2[dz];
+                T *o = s + a + Q * b + ZP * dz;
+                o[0 * PB] = T0[dz];
+                o[1 * PB] = T1[dz];
+                o[2 * PB] = T2[dz];
             }
         } else if (valid) {
             T T0[D], T1[D], T2[D];
@@ -997,10 +1032,10 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
             }
 #pragma unroll
             for (int dz = 0; dz < D; ++dz) {
-                T *o = s + a + Q * (b + Q * dz);
-                o[0 * DQQ] = T0[dz];
-                o[1 * DQQ] = T1[dz];
-                o[2 * DQQ] = T2[dz];
+                T *o = s + a + Q * b + ZP * dz;
+                o[0 * PB] = T0[dz];
+                o[1 * PB] = T1[dz];
+                o[2 * PB] = T2[dz];
             }
         }
     }
@@ -1013,10 +1048,10 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
         if (act) {
 #pragma unroll
             for (int qy = 0; qy < Q; ++qy) {
-                const T *i = s + a + Q * (qy + Q * b);
-                t0[qy] = i[0 * DQQ];
-                t1[qy] = i[1 * DQQ];
-                t2[qy] = i[2 * DQQ];
+                const T *i = s + a + Q * qy + ZP * b;
+                t0[qy] = i[0 * PB];
+                t1[qy] = i[1 * PB];
+                t2[qy] = i[2 * PB];
             }
         }
         __syncthreads();
@@ -1031,8 +1066,8 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
                     sb = fma(gc[qy], t1[qy], sb);
                     sb = fma(bc[qy], t2[qy], sb);
                 }
-                s[a + Q * (dy + D * b)] = sa;
-                s[DDQ + a + Q * (dy + D * b)] = sb;
+                s[a + XS * dy + ZS * b] = sa;
+                s[XB + a + XS * dy + ZS * b] = sb;
             }
         }
     }
@@ -1041,11 +1076,11 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
     // ---- backward x: thread (dy, dz) = (a, b)
     if (valid && a < D && b < D) {
         T sa[Q], sb[Q];
-        const T *in = s + Q * (a + D * b);
+        const T *in = s + XS * a + ZS * b;
 #pragma unroll
         for (int qx = 0; qx < Q; ++qx) {
             sa[qx] = in[qx];
-            sb[qx] = in[DDQ + qx];
+            sb[qx] = in[XB + qx];
         }
         T yv[D];
 #pragma unroll
@@ -1062,7 +1097,7 @@ diffusion_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, c
         if constexpr (OM == 0) {
             store_line<D, T>(out, e, a, b, yv, accumulate);
         } else {
-            T *o = s + 2 * DDQ + D * (a + D * b);
+            T *o = s + 2 * XB + D * (a + D * b);
 #pragma unroll
             for (int dx = 0; dx < D; ++dx) o[dx] = yv[dx];
         }
@@ -1076,8 +1111,8 @@ mass_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, const 
               const T *__restrict__ x, const EOutT<T> &out, int accumulate,
               T *__restrict__ smem) {
     constexpr int QQ = Q * Q, QQQ = Q * Q * Q, DDD = D * D * D;
-    constexpr int DQQ = D * Q * Q;
-    constexpr int BUF = DQQ;
+    using L = ElemLds<D, Q>;
+    constexpr int XS = L::XS, ZS = L::ZS, ZP = L::ZP, BUF = mass_buf<D, Q>();
     const T *__restrict__ Bq = basis;
     const T *__restrict__ Bd = basis + 2 * Q * D;
     const int le = threadIdx.x / QQ;
@@ -1109,7 +1144,7 @@ mass_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, const 
             T v = 0.0;
 #pragma unroll
             for (int dx = 0; dx < D; ++dx) v = fma(br[dx], u[dx], v);
-            s[qx + Q * (a + D * b)] = v;
+            s[qx + XS * a + ZS * b] = v;
         }
     }
     __syncthreads();
@@ -1119,7 +1154,7 @@ mass_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, const 
         const bool act = valid && b < D;
         if (act)
 #pragma unroll
-            for (int dy = 0; dy < D; ++dy) r[dy] = s[a + Q * (dy + D * b)];
+            for (int dy = 0; dy < D; ++dy) r[dy] = s[a + XS * dy + ZS * b];
         __syncthreads();
         if (act)
 #pragma unroll 1
@@ -1128,7 +1163,7 @@ mass_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, const 
                 T v = 0.0;
 #pragma unroll
                 for (int dy = 0; dy < D; ++dy) v = fma(br[dy], r[dy], v);
-                s[a + Q * (qy + Q * b)] = v;
+                s[a + Q * qy + ZP * b] = v;
             }
     }
     __syncthreads();
@@ -1136,7 +1171,7 @@ mass_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, const 
         T z[D];
         if (valid)
 #pragma unroll
-            for (int dz = 0; dz < D; ++dz) z[dz] = s[a + Q * (b + Q * dz)];
+            for (int dz = 0; dz < D; ++dz) z[dz] = s[a + Q * b + ZP * dz];
         __syncthreads();
         if (valid) {
             T tz[D];
@@ -1153,7 +1188,7 @@ mass_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, const 
                 for (int dz = 0; dz < D; ++dz) tz[dz] = fma(br[dz], v, tz[dz]);
             }
 #pragma unroll
-            for (int dz = 0; dz < D; ++dz) s[a + Q * (b + Q * dz)] = tz[dz];
+            for (int dz = 0; dz < D; ++dz) s[a + Q * b + ZP * dz] = tz[dz];
         }
     }
     __syncthreads();
@@ -1162,7 +1197,7 @@ mass_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, const 
         const bool act = valid && b < D;
         if (act)
 #pragma unroll
-            for (int qy = 0; qy < Q; ++qy) tq[qy] = s[a + Q * (qy + Q * b)];
+            for (int qy = 0; qy < Q; ++qy) tq[qy] = s[a + Q * qy + ZP * b];
         __syncthreads();
         if (act)
 #pragma unroll 1
@@ -1171,14 +1206,14 @@ mass_elements_direct(int64_t e0, int64_t ne, const T *__restrict__ basis, const 
                 T v = 0.0;
 #pragma unroll
                 for (int qy = 0; qy < Q; ++qy) v = fma(bc[qy], tq[qy], v);
-                s[a + Q * (dy + D * b)] = v;
+                s[a + XS * dy + ZS * b] = v;
             }
     }
     __syncthreads();
     if (valid && a < D && b < D) {
         T sx[Q];
 #pragma unroll
-        for (int qx = 0; qx < Q; ++qx) sx[qx] = s[qx + Q * (a + D * b)];
+        for (int qx = 0; qx < Q; ++qx) sx[qx] = s[qx + XS * a + ZS * b];
         T yv[D];
 #pragma unroll
         for (int dx = 0; dx < D; ++dx) {

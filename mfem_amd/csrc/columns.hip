@@ -67,10 +67,9 @@ k_diffusion_columns(const ColumnGrid g, const double *__restrict__ basis,
                     const double *__restrict__ x, double *__restrict__ y,
                     double *__restrict__ iface) {
     using T = double;
-    constexpr int P = D - 1, NB = A * B, QQ = Q * Q, DDD = D * D * D, DDQ = D * D * Q;
-    constexpr int BUF = diffusion_buf<D, Q>();
+    constexpr int P = D - 1, NB = A * B, QQ = Q * Q, DDD = D * D * D;
+    constexpr int XB = ElemLds<D, Q>::XB, BUF = diffusion_buf<D, Q, 1>();
     constexpr int PX = A * P + 1, PY = B * P + 1;
-    static_assert(2 * DDQ + DDD <= BUF, "element result does not fit beside the last stage");
     __shared__ T smem[NB * BUF];
     __shared__ int sg[NB * DDD];
     __shared__ T carry[2][PX * PY];
@@ -109,7 +108,7 @@ k_diffusion_columns(const ColumnGrid g, const double *__restrict__ basis,
             T sum = 0.0;
             for (int j = jlo; j <= jhi; ++j)
                 for (int i = ilo; i <= ihi; ++i)
-                    sum += smem[(j * A + i) * BUF + 2 * DDQ + (xq - i * P) +
+                    sum += smem[(j * A + i) * BUF + 2 * XB + (xq - i * P) +
                                 D * ((yq - j * P) + D * zq)];
             if (zq == P && !last) {
                 cout[xq + PX * yq] = sum;

@@ -1,6 +1,5 @@
-// row_sum.hpp -- the E -> L reduction of one L-DOF row, shared by the
-// restriction transpose (restriction.hip) and the solver scatter kernels
-// (pcg.hip, batch.hip).
+// row_sum.hpp -- the E -> L reduction of one L-DOF row through the transpose
+// table (restriction.hip; the fused operators' passes read row_table.hpp).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -36,9 +35,8 @@ __device__ __forceinline__ T row_sum_batch(const int *__restrict__ indices, int 
 //
 // A row's first entries are read as one batch of 2, 4 or 8 -- the smallest
 // that holds every row of the wave (face, edge and vertex rows of a Cartesian
-// hexahedral mesh; in the fused operator's row order the vertex rows come
-// first, so its waves are mostly of one kind, while the element-major order of
-// the lexicographic scatters mixes them and takes the batch of 8): every index
+// hexahedral mesh; the element-major order of the lexicographic scatters mixes
+// them and mostly takes the batch of 8): every index
 // load is issued before any value load, with no branch between them, so a row
 // costs two dependent memory round trips instead of two per entry.  Entries
 // past the 8th continue in a loop.

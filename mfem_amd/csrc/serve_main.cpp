@@ -126,7 +126,7 @@ int64_t estimate_bytes(int n, int p, int precision, bool batch) {
     int64_t b = 0;
     b += ne * 6 * Q3 * 8;                    // PA data
     b += ne * D3 * 8;                        // form E scratch
-    b += ne * D3 * 4 * 4 + N * 4 * 2;        // gather, indices, indices_nat, elem_dof, offsets, perm
+    b += ne * D3 * 4 * 4 + N * 4 * 2;        // gather, indices, row table, elem_dof, offsets, perm
     b += ne * (29 * 4 + 18 + 8 * 3 * 8);     // topology, orientations, nodes
     b += N;                                  // boundary mask
     b += 4 * N * 8;                          // b, x, B, X
