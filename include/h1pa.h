@@ -431,7 +431,8 @@ int h1pa_pcg_solve_multigrid(h1pa_multigrid *mg, const double *d_b, double *d_x,
  * (config/config.hpp:41-48) and it has no mixed-precision PA or PCG.  The
  * operator data of the reduced-precision applies are shadows of the FP64 PA
  * data made by h1pa_form_assemble's output (FP64 -> FP32 round-to-nearest-even,
- * BF16 from that FP32 value, round-to-nearest-even). */
+ * BF16 from that FP32 value, round-to-nearest-even); a re-assembly drops them,
+ * and the next use makes them again. */
 enum {
     H1PA_PREC_FP64 = 0,     /* FP64 PA data, vectors and arithmetic                  */
     H1PA_PREC_FP32 = 1,     /* FP32 PA data, basis, vectors and arithmetic           */

@@ -561,6 +561,9 @@ int h1pa_form_assemble(h1pa_form *form, void *stream) {
     Space &sp = *f.space;
     hipStream_t s = as_stream(stream);
     sp.mesh->ensure_nodes(s);
+    // a reduced-precision copy of the operator data that is about to change is
+    // made again on its next use (ensure_low_precision)
+    f.lp_kind = -1;
     const int Q = f.q1d, D = sp.p + 1;
     std::vector<double> xq(Q), wq(Q), B(Q * D), G(Q * D);
     gauss_legendre(Q, xq.data(), wq.data());

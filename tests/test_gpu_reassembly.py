@@ -1,0 +1,81 @@
+"""GPU: Assemble called again on a form whose coefficient or geometry changed.
+
+Bars: bitwise against a form created afterwards: the same kernels on the same
+operator data.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _form(M, fes, k, mass=False):
+    a = M.BilinearForm(fes)
+    a.SetAssemblyLevel(M.AssemblyLevel.PARTIAL)
+    c = M.PWConstCoefficient(k)
+    a.AddDomainIntegrator(M.DiffusionIntegrator(c))
+    if mass:
+        a.AddDomainIntegrator(M.MassIntegrator(c))
+    a.Assemble()
+    return a
+
+
+def _space(M, p, n):
+    mesh = M.Mesh.MakeCartesian3D(n, n, n)
+    mesh.Perturb(0.2, p)
+    return mesh, M.FiniteElementSpace(mesh, M.H1_FECollection(p, 3))
+
+
+def _low(torch, a, x, prec):
+    y = torch.full_like(x, float("nan"))
+    a.MultLowPrecision(x, y, prec)
+    return y
+
+
+@pytest.mark.parametrize("prec", ["PREC_FP32", "PREC_BF16_PA"])
+@pytest.mark.parametrize("p,mass", [(1, False), (3, True), (6, False)])
+def test_reduced_precision_follows_the_operator(h1pa, torch_cuda, prec, p, mass):
+    """The reduced-precision copy of the operator data is made again after a
+    re-assembly, for a coefficient changed in place and for moved nodes."""
+    M, torch = h1pa, torch_cuda
+    prec = getattr(M, prec)
+    mesh, fes = _space(M, p, 4)
+    rng = np.random.default_rng(p)
+    k = torch.from_numpy(rng.uniform(0.5, 2.0, fes.GetNE())).cuda()
+    x = torch.from_numpy(rng.uniform(-1, 1, fes.GetNDofs())).cuda().float()
+    a = _form(M, fes, k, mass)
+    old = _low(torch, a, x, prec)
+    k.mul_(3.0).add_(torch.linspace(0, 1, fes.GetNE(), dtype=k.dtype, device=k.device))
+    a.Assemble()
+    got = _low(torch, a, x, prec)
+    assert not torch.equal(got, old)
+    assert torch.equal(got, _low(torch, _form(M, fes, k, mass), x, prec))
+    mesh.Perturb(0.1, 77)
+    a.Assemble()
+    moved = _low(torch, a, x, prec)
+    assert not torch.equal(moved, got)
+    assert torch.equal(moved, _low(torch, _form(M, fes, k, mass), x, prec))
+
+
+def test_bf16_cycle_follows_the_operator(h1pa, torch_cuda):
+    """A multigrid cycle in BF16, set up after a re-assembly."""
+    M, torch = h1pa, torch_cuda
+    mesh, fes = _space(M, 4, 4)
+    rng = np.random.default_rng(1)
+    k = torch.from_numpy(rng.uniform(0.5, 2.0, fes.GetNE())).cuda()
+    x = torch.from_numpy(rng.uniform(-1, 1, fes.GetNDofs())).cuda()
+    a = _form(M, fes, k)
+
+    def cycle(form):
+        mg = M.PMultigrid(form, [1, 2, 4], cycle_precision=M.PREC_BF16_PA)
+        y = torch.full_like(x, float("nan"))
+        mg.Mult(x, y)
+        torch.cuda.synchronize()
+        return y
+
+    old = cycle(a)
+    k.copy_(k.flip(0) * 2.0)
+    a.Assemble()
+    got = cycle(a)
+    assert not torch.equal(got, old)
+    assert torch.equal(got, cycle(_form(M, fes, k)))
