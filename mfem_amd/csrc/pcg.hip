@@ -41,6 +41,7 @@ struct PcgState {
     int converged;
     int final_iter;
     int nonfinite;   // a (B r, r) or (A d, d) was not finite: MFEM_VERIFY fails
+    int den_ends;    // small systems: (A d, d) of this iteration ends the loop
 };
 
 namespace kern {
@@ -407,9 +408,11 @@ k_small_scatter(int n, int bb, RowTab tb, const T *__restrict__ ye,
     if (threadIdx.x == 0) pden[blockIdx.x] = p;
 }
 
-// x += alpha d, r -= alpha z, z = dinv r; partials of (r, z).  Block 0 records
-// (A d, d); a block that finds `done` already set by it stops as it would on its
-// own total.
+// x += alpha d, r -= alpha z, z = dinv r; partials of (r, z).  Every block finds
+// (A d, d) and stops on it alike; block 0 records it in `den` and `den_ends`, which
+// only the next launch reads (k_small_dir ends the loop): what a wave reads here
+// must not depend on how far block 0 has come, or a block's waves would part
+// before the barriers of its sum.
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
 k_small_update(int n, const T *__restrict__ dinv, T *__restrict__ x, T *__restrict__ r,
@@ -424,8 +427,12 @@ k_small_update(int n, const T *__restrict__ dinv, T *__restrict__ x, T *__restri
     const T vd = d[j], vx = x[j], vr = r[j], vz = z[j], vi = dinv[j];
     if (done) return;
     const double den = fold_total(fs, sh);
-    if (blockIdx.x == 0 && threadIdx.x == 0) write_den(st, den);
-    if (den_ends(den)) return;
+    const bool ends = den_ends(den);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->den = den;
+        st->den_ends = ends ? 1 : 0;
+    }
+    if (ends) return;
     const T alpha = (T)(nom / den);
     const T ri = vr - alpha * vz, zi = vi * ri;
     if (t < n) {
@@ -461,6 +468,7 @@ __device__ __forceinline__ void write_step(const PcgState &st, PcgState *o, doub
     o->converged = st.converged | u.converged;
     o->nonfinite = st.nonfinite | u.nonfinite;
     o->done = u.done;
+    o->den_ends = 0;
     o->beta = u.done ? beta : betanom / nom;
     o->nom = u.done ? nom : betanom;
     o->iter = u.done ? i : i + 1;
@@ -488,13 +496,17 @@ k_small_dir(int n, const T *__restrict__ z, T *__restrict__ d, const double *__r
     __shared__ double sh[4];
     const int t = blockIdx.x * kThreads + threadIdx.x;
     const int j = t < n ? t : n - 1;
-    const int done = st->done, iter = st->iter, max_iter = st->max_iter;
+    const int done = st->done | st->den_ends, iter = st->iter, max_iter = st->max_iter;
     const double nom = st->nom, r0 = st->r0;
     const FoldSum fs = fold_load(prho, gridDim.x);
     const T vz = z[j], vd = d[j];
     const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
     if (done) {
-        if (writer) *next = *st;
+        if (writer) {
+            *next = *st;
+            if (!st->done) write_den(next, st->den);
+            next->den_ends = 0;
+        }
         return;
     }
     const double rho = fold_total(fs, sh);
