@@ -52,6 +52,7 @@ struct SlotState {
     int iter, in_loop, max_iter, converged, final_iter;
     int phase, outer;
     int nonfinite;  // a (B r, r) or (A d, d) was not finite: retired with a failed status
+    int den_ends;   // folded update: (A d, d) ends the inner iterations (write_den is due)
 };
 
 struct SlotDesc {
@@ -310,6 +311,7 @@ __device__ __forceinline__ void write_update(const SlotState &st, SlotState *o, 
     o->nom = on ? rho : nom;
     o->nonfinite = st.nonfinite | u.nonfinite;
     o->phase = u.phase;
+    o->den_ends = 0;
     if (MIXED) {
         o->iter = i;
         o->converged = converged;
@@ -593,9 +595,11 @@ kb_fin_den(const int *__restrict__ runlist, const SlotDesc *__restrict__ desc,
 
 // x += alpha d, r -= alpha z, z = dinv r, partials of (r, z); x is the
 // solution (FP64 mode) or the FP32 update xs (mixed).  FOLD: the slot's
-// (A d, d) is summed here, by every block from the partials pden, and the
-// block of chunk 0 applies the step's scalar logic (a block that reads the
-// phase it writes stops either way: it finds the same total).
+// (A d, d) is summed here, by every block from the partials pden, and every block
+// stops on it alike.  The block of chunk 0 records it in `den` and `den_ends`,
+// which only the next launch reads (kb_dir_fold or kb_fin_update applies it): the
+// phase that the blocks read at entry is not written here, or a block's waves
+// could part before the barriers of its sum.
 template <typename T, bool MIXED, bool FOLD>
 __global__ void __launch_bounds__(kT)
 kb_update(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
@@ -620,8 +624,12 @@ kb_update(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
     }
     if constexpr (FOLD) {
         den = fold_total(fs, sh);
-        if (tk.chunk == 0 && threadIdx.x == 0) write_den<MIXED>(states + tk.slot, den);
-        if (after_den<MIXED>(den).phase != PH_INNER) return;
+        const bool ends = after_den<MIXED>(den).phase != PH_INNER;
+        if (tk.chunk == 0 && threadIdx.x == 0) {
+            states[tk.slot].den = den;
+            states[tk.slot].den_ends = ends ? 1 : 0;
+        }
+        if (ends) return;
     } else {
         den = states[tk.slot].den;
     }
@@ -650,6 +658,11 @@ kb_fin_update(const int *__restrict__ runlist, const SlotDesc *__restrict__ desc
     double tot[1];
     slot_totals<1>(sd, partials, sh, tot);
     if (threadIdx.x != 0) return;
+    if (st->den_ends) {  // the folded update stored no (r, z)
+        write_den<MIXED>(st, st->den);
+        st->den_ends = 0;
+        return;
+    }
     const double thresh = update_thresh<MIXED>(*st, sd);
     write_update<MIXED>(*st, st, tot[0], thresh,
                         after_update<MIXED>(tot[0], thresh, MIXED ? st->iter + 1 : st->iter,
@@ -691,8 +704,13 @@ kb_dir_fold(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc
     const SlotDesc &sd = desc[tk.slot];
     const SlotState &st = states[tk.slot];
     const bool writer = tk.chunk == 0 && threadIdx.x == 0;
-    if (st.phase != PH_INNER) {
-        if (writer) next[tk.slot] = st;
+    const int phase = st.phase;
+    if (phase != PH_INNER || st.den_ends) {
+        if (writer) {
+            next[tk.slot] = st;
+            if (phase == PH_INNER) write_den<MIXED>(next + tk.slot, st.den);
+            next[tk.slot].den_ends = 0;
+        }
         return;
     }
     const FoldSum fs = fold_load(partials, sd.part0, sd.nchunks);

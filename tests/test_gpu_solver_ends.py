@@ -1,6 +1,7 @@
 """GPU: solves that end on (A d, d) = 0 or on an (A d, d) that is not finite, in
 the first iteration: nothing may be written after it, on either side of the
-size from which CG sums its products in kernels of their own.
+size from which CG sums its products in kernels of their own, and in a batch with
+and without a slot too large for folded sums.
 
 The right-hand sides make (B r, r) an ordinary number and (A d, d) not: with
 b = s D v and d = D^-1 b = s v, (B r, r) = s^2 (v, D v) and (A d, d) = s^2 (v, A v).
@@ -21,7 +22,7 @@ def _system(M, torch, p, n):
     fes = M.FiniteElementSpace(mesh, M.H1_FECollection(p, 3))
     a = M.BilinearForm(fes)
     a.SetAssemblyLevel(M.AssemblyLevel.PARTIAL)
-    a.AddDomainIntegrator(M.DiffusionIntegrator(M.ConstantCoefficient(1.0)))
+    a.AddDomainIntegrator(M.DiffusionIntegrator(M.ConstantCoefficient(100.0)))
     a.Assemble()
     ess = fes.GetBoundaryTrueDofs()
     zero = torch.zeros(fes.GetNDofs(), dtype=torch.float64, device="cuda")
@@ -95,3 +96,41 @@ def test_cg_ends_before_an_update(h1pa, torch_cuda, p, n):
     cg.Mult(b, x)
     r = b - _apply(torch, s, x)
     assert cg.GetConverged() and float(r.norm() / b.norm()) < 1e-8
+
+
+@pytest.mark.parametrize("K", [1, 2, 3, 8])
+@pytest.mark.parametrize("large", [False, True])
+@pytest.mark.parametrize("prec", ["PREC_FP64", "PREC_FP32", "PREC_BF16_PA"])
+def test_batch_ends_before_an_update(h1pa, torch_cuda, prec, large, K):
+    """As above; mixed slots run FP32 inner iterations, in which (A d, d) is zero
+    because b = 1e-60 rounds to zero, and not finite because A d overflows FP32.
+    They share the batch with ordinary solves, and (large) with a slot of 1.1M
+    DOFs, which no folded sum takes."""
+    M, torch = h1pa, torch_cuda
+    mode = getattr(M, prec)
+    s = _system(M, torch, 2, 8)
+    if mode == M.PREC_FP64:
+        zero, inf = _ends_at_zero(torch, s), _ends_at_infinity(torch, s)[0]
+    else:
+        zero = s["D"] * s["free"] * 1e-60
+        v = _ends_at_infinity(torch, s)[1]
+        inf = s["D"] * v
+        inf = inf * (3.3e38 / inf.abs().max())
+    b = s["D"] * s["free"]
+    rhs = [zero, b, inf, b * 2.0]
+    xs = [torch.full_like(b, float("nan")) for _ in rhs]
+    bs = M.BatchSolver(precision=mode, iters_per_replay=K)
+    tags = [bs.Add(s["A"], q, x, rel_tol=1e-10, max_iter=400) for q, x in zip(rhs, xs)]
+    if large:
+        t = _system(M, torch, 3, 35)
+        bl = t["D"] * t["free"]
+        xl = torch.empty_like(bl)
+        tags.append(bs.Add(t["A"], bl, xl, rel_tol=1e-2, max_iter=400))
+    bs.Run()
+    res = dict(bs.Poll())
+    assert not res[tags[0]]["converged"] and not bool(xs[0].any())
+    assert res[tags[2]]["status"] == M.H1PA_ENONFINITE and not bool(xs[2].any())
+    for k, f in ((1, 1.0), (3, 2.0)):
+        assert res[tags[k]]["converged"]
+        r = b * f - _apply(torch, s, xs[k])
+        assert float(r.norm() / b.norm()) < 1e-7
