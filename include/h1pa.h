@@ -225,7 +225,11 @@ int h1pa_form_create(h1pa_space *space, const h1pa_form_desc *desc, h1pa_form **
 int h1pa_form_destroy(h1pa_form *form);
 /* a.Assemble(): geometric factors, coefficient and PA data on the device
  * (DiffusionIntegrator::AssemblePA, fem/integ/bilininteg_diffusion_pa.cpp:108-171;
- *  MassIntegrator::AssemblePA, fem/integ/bilininteg_mass_pa.cpp:25-90). */
+ *  MassIntegrator::AssemblePA, fem/integ/bilininteg_mass_pa.cpp:25-90).
+ * Called again it writes the same buffers: it first waits for the work queued
+ * on the device, so products already queued on other streams still apply the
+ * operator they were queued with.  With the block cache on
+ * (h1pa_set_device_cache) it does not wait, and the caller orders such calls. */
 int h1pa_form_assemble(h1pa_form *form, void *stream);
 /* Operator::Mult: y = A x on L-vectors, y overwritten
  * (PABilinearFormExtension::Mult, fem/bilinearform_ext.cpp:487-560). */

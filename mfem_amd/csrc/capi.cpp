@@ -561,6 +561,9 @@ int h1pa_form_assemble(h1pa_form *form, void *stream) {
     Space &sp = *f.space;
     hipStream_t s = as_stream(stream);
     sp.mesh->ensure_nodes(s);
+    // A re-assembly writes the buffers of the last one, which saves freeing and
+    // allocating them; products queued on other streams may still read them.
+    if (f.assembled) device_wait_reuse();
     // a reduced-precision copy of the operator data that is about to change is
     // made again on its next use (ensure_low_precision)
     f.lp_kind = -1;
@@ -581,7 +584,6 @@ int h1pa_form_assemble(h1pa_form *form, void *stream) {
     even_odd_tables(D, Q, B.data(), G.data(), pack.data() + 4 * Q * D);
     f.basis.upload(pack.data(), pack.size(), s);
     const int64_t nq = (int64_t)Q * Q * Q;
-    // a re-assembly keeps its buffers: a hipFree waits for the whole device
     auto keep = [](DevBuf<double> &b, int64_t n) {
         if (b.n != (size_t)n) b.alloc((size_t)n);
     };

@@ -111,6 +111,14 @@ void device_free(void *p, size_t cap, int dev) {
     (void)hipFree(p);
 }
 
+void device_wait_reuse() {
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        if (g_limit > 0) return;
+    }
+    H1PA_HIP(hipDeviceSynchronize());
+}
+
 void device_cache_set(int64_t max_bytes) {
     std::lock_guard<std::mutex> lock(g_mu);
     g_limit = max_bytes;

@@ -47,6 +47,10 @@ struct bf16_t {
 // release an object while device work on its buffers is pending.
 void *device_alloc(size_t bytes, size_t &cap, int &dev);
 void device_free(void *p, size_t cap, int dev);
+// Before a block that earlier calls on other streams may still read is written
+// again in place: waits for the device as freeing and allocating it would (not
+// with the cache on, where the caller orders such calls).
+void device_wait_reuse();
 void device_cache_set(int64_t max_bytes);  // 0: off (kept blocks are freed)
 int64_t device_cache_bytes();               // bytes kept, all devices
 

@@ -79,3 +79,28 @@ def test_bf16_cycle_follows_the_operator(h1pa, torch_cuda):
     got = cycle(a)
     assert not torch.equal(got, old)
     assert torch.equal(got, cycle(_form(M, fes, k)))
+
+
+def test_products_queued_on_another_stream(h1pa, torch_cuda):
+    """Products queued on one stream when another re-assembles apply the operator
+    they were queued with: bitwise the product before."""
+    M, torch = h1pa, torch_cuda
+    mesh, fes = _space(M, 4, 24)
+    k = torch.full((fes.GetNE(),), 2.0, dtype=torch.float64, device="cuda")
+    x = torch.rand(fes.GetNDofs(), dtype=torch.float64, device="cuda")
+    a = _form(M, fes, k)
+    want = torch.empty_like(x)
+    a.Mult(x, want)
+    st = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for round_ in range(5):
+        ys = [torch.full_like(x, float("nan")) for _ in range(40)]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(st[0]):
+            for y in ys:
+                a.Mult(x, y)
+        with torch.cuda.stream(st[1]):
+            k.add_(1.0)
+            a.Assemble()
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, want) for y in ys), round_
+        a.Mult(x, want)
