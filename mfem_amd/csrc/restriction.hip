@@ -438,8 +438,14 @@ k_scatter_rows(int64_t nrows, RowTab tb, const T *__restrict__ ye,
     T s[R];
     rows_sum<R, NT>(tb, t, ye, s);
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-        if (t0 + r * kBlock < nrows) y[i[r]] = (mask && mask[i[r]]) ? xin[i[r]] : s[r];
+    for (int r = 0; r < R; ++r) {
+        if (t0 + r * kBlock >= nrows) continue;
+        // (as a conditional expression this selects an address, and the sums go
+        // through private memory)
+        T v = s[r];
+        if (mask && mask[i[r]]) v = xin[i[r]];
+        y[i[r]] = v;
+    }
 }
 
 __global__ void k_native_indices(int64_t nE, int dof, int es, const int *__restrict__ indices,
