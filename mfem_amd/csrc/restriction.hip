@@ -645,14 +645,17 @@ template <typename T>
 void launch_scatter_rows(const Restriction &r, int64_t nrows, const T *ye, const uint8_t *mask,
                          const T *xin, T *y, hipStream_t s) {
     if (nrows <= 0) return;
-    // Rows per thread.  Below a block per CU of two-row threads one row each
-    // (p = 3, 16^3 elements, 86k rows: 7.05 -> 6.27 us between events); from 6M
-    // rows on, where the E-vector and the table no longer stay in the caches,
-    // four with the table streamed (p = 4, 79^3, 18.6M rows: 174 -> 165 us; p = 2, 100^3: 154 ->
-    // 145; at 4M rows, p = 8: 30.9 -> 31.7 us); two between.
+    // Rows per thread.  One row each while the E-vector and the table stay in the
+    // caches, where waves hide more than loads in flight of one wave do (us of the
+    // kernel with one, two, four rows a thread, FP64: p = 1, 40^3 elements, 67k rows
+    // 4.1, 4.4, 7.2; p = 3, 26^3, 339k rows 5.8, 7.2, 10.9; p = 1, 100^3, 1.0M rows
+    // 33, 41, 43; p = 4, 30^3, 1.0M rows 11.4, 12.7, 17.1; FP32 alike: 339k rows 4.9,
+    // 6.4, 9.9).  Two above 1.5M rows (p = 2, 60^3, 1.5M rows 32.0, 30.0, 30.4; p = 3,
+    // 55^3, 3.2M rows 36.3, 35.3, 35.9); four with the table streamed from 6M rows
+    // on (p = 6, 48^3, 10.1M rows 74.6, 71.6, 70.2).
     const RowTab tb = r.rows();
     auto grid = [&](int R) { return dim3(nblocks((nrows + R - 1) / R)); };
-    if (nrows <= 256 * 2 * kBlock)
+    if (nrows <= (int64_t)3 << 19)
         hipLaunchKernelGGL((k_scatter_rows<1, false, T>), grid(1), dim3(kBlock), 0, s, nrows, tb,
                            ye, mask, xin, y);
     else if (nrows < (int64_t)6 << 20)
