@@ -99,40 +99,29 @@ __device__ __forceinline__ Grp grp_of(int64_t b, int64_t end) {
          g##_b < g##_e; g##_b += (int64_t)kGrp * kThreads)                                     \
         for (const Grp g = grp_of(g##_b, g##_e), *g##_1 = &g; g##_1; g##_1 = nullptr)
 
-// E -> L sums of the group's rows (positions g.lt): v[k] = the row's sum for a
-// position below bb, z[ii[k]] (written by the element kernel) for an interior
-// DOF.  A wave of interior DOFs alone reads no row.
+// Blocks of a row kernel without a product: one entry a thread.
+inline dim3 row_blocks(int64_t n) { return dim3((unsigned)((n + kThreads - 1) / kThreads)); }
+
+// The E -> L kernels take one row at a time (H1PA_CHUNK): a row is two dependent
+// loads, which other waves hide, and these kernels run eight waves per SIMD so.
+// Four rows at once left three or four (us of k_pcg_scatter<double>, four rows ->
+// one: p = 6, 11^3 elements 7.0 -> 5.3; 13^3 10.6 -> 7.4; 26^3 31 -> 33; 48^3 210 ->
+// 173; k_ir_scatter at 48^3 168 -> 129).
+// The E -> L sum of the row at position t, L-DOF i: of its E-entries below bb,
+// z[i] (written by the element kernel) for an interior DOF.  A wave of interior
+// DOFs alone reads no row.
 template <typename T>
-__device__ __forceinline__ void group_rows(const RowTab &tb, int64_t bb, int per, const Grp &g,
-                                           const int (&ii)[kGrp], const T *__restrict__ ye,
-                                           const T *z, T (&v)[kGrp]) {
-    const bool rows = __ballot(g.lt[0] < bb), inner = __ballot(g.lt[kGrp - 1] >= bb);
-    T vz[kGrp];
-    if (inner)
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k)
-            if (k < per) vz[k] = z[ii[k]];
-    if (rows) {
-        int t[kGrp];
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) t[k] = (int)(g.lt[k] < bb ? g.lt[k] : bb - 1);
-        if (per >= kGrp) {
-            rows_sum<kGrp>(tb, t, ye, v);
-        } else {
-#pragma unroll
-            for (int k = 0; k < kGrp; ++k) {
-                if (k >= per) break;
-                const int t1[1] = {t[k]};
-                T v1[1];
-                rows_sum<1>(tb, t1, ye, v1);
-                v[k] = v1[0];
-            }
-        }
+__device__ __forceinline__ T row_value(const RowTab &tb, int64_t bb, int t, int i,
+                                       const T *__restrict__ ye, const T *z) {
+    T v = T(0);
+    if (__ballot(t < bb)) {
+        const int t1[1] = {t < bb ? t : (int)bb - 1};
+        T v1[1];
+        rows_sum<1>(tb, t1, ye, v1);
+        v = v1[0];
     }
-    if (inner)
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k)
-            if (k < per && g.lt[k] >= bb) v[k] = vz[k];
+    if (t >= bb) v = z[i];
+    return v;
 }
 
 // Block sum in a fixed tree order, returned to every thread.
@@ -299,27 +288,16 @@ k_pcg_scatter(int64_t n, int per, int64_t bb, RowTab tb, const T *__restrict__ y
     __shared__ double sh[kThreads];
     if (st->done) return;
     double acc[1] = {0.0};
-    H1PA_GROUPS(g, n) {
-        int ii[kGrp];
-        T vd[kGrp], v[kGrp];
-        bool m[kGrp];
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (k >= per) break;  // past this thread's entries
-            ii[k] = row_dof(tb, (int)g.lt[k]);
-            vd[k] = d[ii[k]];
-            m[k] = mask && mask[ii[k]];
+    H1PA_CHUNK(t, n) {
+        const int i = row_dof(tb, (int)t);
+        const T vd = d[i];
+        const bool m = mask && mask[i];
+        T v = row_value(tb, bb, (int)t, i, ye, z);
+        if (t < bb) {
+            v = m ? vd : v;
+            z[i] = v;
         }
-        group_rows(tb, bb, per, g, ii, ye, z, v);
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
-            if (g.t[k] < bb) {
-                v[k] = m[k] ? vd[k] : v[k];
-                z[ii[k]] = v[k];
-            }
-            acc[0] += (double)vd[k] * (double)v[k];
-        }
+        acc[0] += (double)vd * (double)v;
     }
     store_partials<1>(acc, partials, sh);
 }
@@ -635,27 +613,16 @@ k_ir_scatter(int64_t n, int per, int64_t bb, RowTab tb, const float *__restrict_
     __shared__ double sh[kThreads];
     if (st->done) return;
     double acc[1] = {0.0};
-    H1PA_GROUPS(g, n) {
-        int ii[kGrp];
-        float vd[kGrp], v[kGrp];
-        bool m[kGrp];
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (k >= per) break;  // past this thread's entries
-            ii[k] = row_dof(tb, (int)g.lt[k]);
-            vd[k] = d[ii[k]];
-            m[k] = mask && mask[ii[k]];
+    H1PA_CHUNK(t, n) {
+        const int i = row_dof(tb, (int)t);
+        const float vd = d[i];
+        const bool m = mask && mask[i];
+        float v = row_value(tb, bb, (int)t, i, ye, q);
+        if (t < bb) {
+            v = m ? vd : v;
+            q[i] = v;
         }
-        group_rows(tb, bb, per, g, ii, ye, q, v);
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
-            if (g.t[k] < bb) {
-                v[k] = m[k] ? vd[k] : v[k];
-                q[ii[k]] = v[k];
-            }
-            acc[0] += (double)vd[k] * (double)v[k];
-        }
+        acc[0] += (double)vd * (double)v;
     }
     store_partials<1>(acc, partials, sh);
 }
@@ -762,31 +729,20 @@ k_ir_ru_res(int64_t n, int per, int64_t bb, RowTab tb, const double *__restrict_
     __shared__ double sh[kThreads];
     if (!st->ru) return;
     double acc[3] = {0.0, 0.0, 0.0};
-    H1PA_GROUPS(g, n) {
-        int ii[kGrp];
-        double v[kGrp];
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (k >= per) break;  // past this thread's entries
-            ii[k] = row_dof(tb, (int)g.lt[k]);
-        }
+    H1PA_CHUNK(t, n) {
+        const int i = row_dof(tb, (int)t);
         // interior DOFs: (A x)_i was written into r64 by the element kernel
-        group_rows(tb, bb, per, g, ii, ye64, r64, v);
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
-            const int64_t i = ii[k];
-            const double y = (g.t[k] < bb && mask && mask[i]) ? x[i] : v[k];
-            const double ri = b[i] - y;
-            r64[i] = ri;
-            const float rf = (float)ri;
-            const float zf = dinv[i] * rf;
-            r[i] = rf;
-            z[i] = zf;
-            acc[0] += (double)rf * (double)zf;
-            acc[1] += ri * dinv64[i] * ri;
-            acc[2] += ri * ri;
-        }
+        double y = row_value(tb, bb, (int)t, i, ye64, r64);
+        if (t < bb && mask && mask[i]) y = x[i];
+        const double ri = b[i] - y;
+        r64[i] = ri;
+        const float rf = (float)ri;
+        const float zf = dinv[i] * rf;
+        r[i] = rf;
+        z[i] = zf;
+        acc[0] += (double)rf * (double)zf;
+        acc[1] += ri * dinv64[i] * ri;
+        acc[2] += ri * ri;
     }
     store_partials<3>(acc, partials, sh);
 }
@@ -871,41 +827,28 @@ k_cheb_first(int64_t n, int per, const double *__restrict__ dinv, const double *
 // smoothing step's correction, without a pass of its own).
 template <bool ADD>
 __global__ void __launch_bounds__(kThreads)
-k_cheb_scatter(int64_t n, int per, int64_t bb, RowTab tb, const double *__restrict__ ye,
+k_cheb_scatter(int64_t n, int64_t bb, RowTab tb, const double *__restrict__ ye,
                const uint8_t *__restrict__ mask, const double *__restrict__ dinv,
                const double *__restrict__ u, double *__restrict__ t, double *y, double *to,
                double ck, const int *stop) {
     if (stop && *stop) return;
-    H1PA_GROUPS(g, n) {
-        int ii[kGrp];
-        double vi[kGrp], vy[kGrp], vt[kGrp], vo[kGrp], v[kGrp];
-        bool m[kGrp];
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (k >= per) break;  // past this thread's entries
-            ii[k] = row_dof(tb, (int)g.lt[k]);
-            vi[k] = dinv[ii[k]];
-            vy[k] = y[ii[k]];
-            vt[k] = t[ii[k]];
-            if constexpr (ADD) vo[k] = to[ii[k]];
-            m[k] = mask && mask[ii[k]];
-        }
-        group_rows(tb, bb, per, g, ii, ye, u, v);
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
-            if (g.t[k] < bb && m[k]) v[k] = vt[k];
-            const double ti = v[k] * vi[k];
-            const double yi = vy[k] + ck * ti;
-            if (!to) {
-                t[ii[k]] = ti;
-                y[ii[k]] = yi;
-            } else if constexpr (ADD) {
-                to[ii[k]] = vo[k] + yi;
-            } else {
-                to[ii[k]] = yi;
-            }
-        }
+    const int64_t p = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+    if (p >= n) return;
+    const int i = row_dof(tb, (int)p);
+    const double vi = dinv[i], vy = y[i], vt = t[i];
+    double vo = 0.0;
+    if constexpr (ADD) vo = to[i];
+    const bool m = mask && mask[i];
+    double v = row_value(tb, bb, (int)p, i, ye, u);
+    if (p < bb && m) v = vt;
+    const double ti = v * vi, yi = vy + ck * ti;
+    if (!to) {
+        t[i] = ti;
+        y[i] = yi;
+    } else if constexpr (ADD) {
+        to[i] = vo + yi;
+    } else {
+        to[i] = yi;
     }
 }
 
@@ -914,37 +857,26 @@ k_cheb_scatter(int64_t n, int per, int64_t bb, RowTab tb, const double *__restri
 // r is not stored; else r is stored (it may be u).
 template <bool FIRST>
 __global__ void __launch_bounds__(kThreads)
-k_residual(int64_t n, int per, int64_t bb, RowTab tb, const double *__restrict__ ye,
+k_residual(int64_t n, int64_t bb, RowTab tb, const double *__restrict__ ye,
            const uint8_t *__restrict__ mask, const double *__restrict__ x,
            const double *__restrict__ y, const double *u, const double *__restrict__ dinv,
            double *r, double *__restrict__ z, double c0) {
-    H1PA_GROUPS(g, n) {
-        int ii[kGrp];
-        double vx[kGrp], vy[kGrp], vi[kGrp], v[kGrp];
-        bool m[kGrp];
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (k >= per) break;  // past this thread's entries
-            ii[k] = row_dof(tb, (int)g.lt[k]);
-            vx[k] = x[ii[k]];
-            vy[k] = y[ii[k]];
-            if constexpr (FIRST) vi[k] = dinv[ii[k]];
-            m[k] = mask && mask[ii[k]];
-        }
-        group_rows(tb, bb, per, g, ii, ye, u, v);
-#pragma unroll
-        for (int k = 0; k < kGrp; ++k) {
-            if (!g.ok[k]) continue;  // (every slot past `per` is not ok)
-            if (g.t[k] < bb && m[k]) v[k] = vy[k];
-            const double ri = vx[k] - v[k];
-            if constexpr (FIRST) {
-                const double ti = ri * vi[k];
-                r[ii[k]] = ti;
-                z[ii[k]] = 0.0 + c0 * ti;
-            } else {
-                r[ii[k]] = ri;
-            }
-        }
+    const int64_t t = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+    if (t >= n) return;
+    const int i = row_dof(tb, (int)t);
+    const double vx = x[i], vy = y[i];
+    double vi = 0.0;
+    if constexpr (FIRST) vi = dinv[i];
+    const bool m = mask && mask[i];
+    double v = row_value(tb, bb, (int)t, i, ye, u);
+    if (t < bb && m) v = vy;
+    const double ri = vx - v;
+    if constexpr (FIRST) {
+        const double ti = ri * vi;
+        r[i] = ti;
+        z[i] = 0.0 + c0 * ti;
+    } else {
+        r[i] = ri;
     }
 }
 
@@ -1685,7 +1617,7 @@ void chebyshev_steps(Chebyshev &c, double *y, double *to, bool add, const int *s
     Form &f = *c.f;
     Space &sp = *f.space;
     const int64_t n = sp.ndofs;
-    const kern::Chunks ch = kern::chunks(n);
+    const dim3 grid = kern::row_blocks(n);
     const int64_t bb = direct_rows(sp, c.mask);
     const RowTab rows = sp.restr.rows();
     for (int k = 1; k < c.order; ++k) {
@@ -1693,13 +1625,13 @@ void chebyshev_steps(Chebyshev &c, double *y, double *to, bool add, const int *s
         pcg_element_apply<double>(f, c.prec, c.mask, c.t.p, f.ework0.p,
                                   bb < n ? c.u.p : nullptr, stop, s);
         if (last && add)
-            hipLaunchKernelGGL(kern::k_cheb_scatter<true>, dim3(ch.blocks), dim3(kern::kThreads),
-                               0, s, n, ch.per, bb, rows, f.ework0.p, c.mask, c.dinv.p, c.u.p,
-                               c.t.p, y, to, c.coeffs[k], stop);
+            hipLaunchKernelGGL(kern::k_cheb_scatter<true>, grid, dim3(kern::kThreads), 0, s, n,
+                               bb, rows, f.ework0.p, c.mask, c.dinv.p, c.u.p, c.t.p, y, to,
+                               c.coeffs[k], stop);
         else
-            hipLaunchKernelGGL(kern::k_cheb_scatter<false>, dim3(ch.blocks), dim3(kern::kThreads),
-                               0, s, n, ch.per, bb, rows, f.ework0.p, c.mask, c.dinv.p, c.u.p,
-                               c.t.p, y, last ? to : nullptr, c.coeffs[k], stop);
+            hipLaunchKernelGGL(kern::k_cheb_scatter<false>, grid, dim3(kern::kThreads), 0, s, n,
+                               bb, rows, f.ework0.p, c.mask, c.dinv.p, c.u.p, c.t.p, y,
+                               last ? to : nullptr, c.coeffs[k], stop);
     }
     H1PA_HIP(hipGetLastError());
 }
@@ -1782,10 +1714,9 @@ void constrained_residual(Form &f, const uint8_t *mask, const double *x, const d
                           double *r, hipStream_t s, int prec) {
     Space &sp = *f.space;
     const int64_t n = sp.ndofs, bb = direct_rows(sp, mask);
-    const kern::Chunks ch = kern::chunks(n);
     pcg_element_apply<double>(f, prec, mask, y, f.ework0.p, bb < n ? r : nullptr, nullptr, s);
-    hipLaunchKernelGGL(kern::k_residual<false>, dim3(ch.blocks), dim3(kern::kThreads), 0, s, n,
-                       ch.per, bb, sp.restr.rows(), f.ework0.p, mask, x, y, r, nullptr, r, nullptr,
+    hipLaunchKernelGGL(kern::k_residual<false>, kern::row_blocks(n), dim3(kern::kThreads), 0, s,
+                       n, bb, sp.restr.rows(), f.ework0.p, mask, x, y, r, nullptr, r, nullptr,
                        0.0);
     H1PA_HIP(hipGetLastError());
 }
@@ -1795,12 +1726,11 @@ void chebyshev_smooth(Chebyshev &c, const double *x, double *y, double *z, hipSt
     Form &f = *c.f;
     Space &sp = *f.space;
     const int64_t n = sp.ndofs, bb = direct_rows(sp, c.mask);
-    const kern::Chunks ch = kern::chunks(n);
     pcg_element_apply<double>(f, c.prec, c.mask, y, f.ework0.p, bb < n ? c.u.p : nullptr, nullptr,
                               s);
-    hipLaunchKernelGGL(kern::k_residual<true>, dim3(ch.blocks), dim3(kern::kThreads), 0, s, n,
-                       ch.per, bb, sp.restr.rows(), f.ework0.p, c.mask, x, y, c.u.p, c.dinv.p,
-                       c.t.p, z, c.coeffs[0]);
+    hipLaunchKernelGGL(kern::k_residual<true>, kern::row_blocks(n), dim3(kern::kThreads), 0, s,
+                       n, bb, sp.restr.rows(), f.ework0.p, c.mask, x, y, c.u.p, c.dinv.p, c.t.p, z,
+                       c.coeffs[0]);
     if (c.order == 1) kern::axpy(n, 1.0, z, y, s);
     else chebyshev_steps(c, z, y, true, nullptr, s);
     H1PA_HIP(hipGetLastError());

@@ -94,10 +94,39 @@ __device__ __forceinline__ void rows_of_width(const RowTab &tb, const int *__res
             if (ix[r][0] == kRowOver) s[r] = row_overflow(tb, t[r], xe);
 }
 
+// A row of any kind, for the few waves that hold several kinds: eight entries, of
+// which a row narrower than that leaves the rest out.  Interior-DOF rows
+// (position bbeg on) have one entry, in the same order after the surface ones.
+template <bool NT, typename T>
+__device__ __forceinline__ T row_any(const RowTab &tb, int t, const T *__restrict__ xe) {
+    const bool in = t >= tb.bbeg;
+    if (!__ballot(!in)) return T(0) + xe[tb.ebub + (t - tb.bbeg)];
+    const int q = in ? tb.bbeg - 1 : t;
+    const int w = q < tb.ebeg ? 8 : q < tb.fbeg ? 4 : 2;
+    const int nv = min(q, tb.ebeg), ne = min(max(q - tb.ebeg, 0), tb.fbeg - tb.ebeg),
+              nf = max(q - tb.fbeg, 0);
+    const int *const p = tb.tab + (8 * (int64_t)nv + 4 * (int64_t)ne + 2 * (int64_t)nf);
+    int ix[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int *const pk = p + (k < w ? k : w - 1);
+        ix[k] = NT ? __builtin_nontemporal_load(pk) : *pk;
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        if (in || k >= w) ix[k] = -1;
+    if (in) ix[0] = (int)(tb.ebub + (t - tb.bbeg));
+    T v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = xe[ix[k] >= 0 ? ix[k] : 0];
+    T s = row_add<8>(ix, v);
+    if (tb.over && ix[0] == kRowOver) s = row_overflow(tb, t, xe);
+    return s;
+}
+
 // s[r] = sum of the E-entries of the row at position t[r], t[0] <= ... <= t[R-1]
 // (rows of any kind; a wave whose rows are all vertices, edges or faces --
-// nearly every wave -- takes the loop of that width).  Interior-DOF rows
-// (position bbeg on) have one entry, in the same order after the surface ones.
+// nearly every wave -- takes the loop of that width).
 // NT: the table is streamed past the caches.
 template <int R, bool NT = false, typename T>
 __device__ __forceinline__ void rows_sum(const RowTab &tb, const int (&t)[R],
@@ -118,13 +147,7 @@ __device__ __forceinline__ void rows_sum(const RowTab &tb, const int (&t)[R],
         }
     } else {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int q = t[r];
-            if (q < tb.ebeg) rows_of_width<1, 8, NT>(tb, ev, 0, &q, xe, s + r);
-            else if (q < tb.fbeg) rows_of_width<1, 4, NT>(tb, ee, tb.ebeg, &q, xe, s + r);
-            else if (q < tb.bbeg) rows_of_width<1, 2, NT>(tb, ef, tb.fbeg, &q, xe, s + r);
-            else s[r] = T(0) + xe[tb.ebub + (q - tb.bbeg)];
-        }
+        for (int r = 0; r < R; ++r) s[r] = row_any<NT>(tb, t[r], xe);
     }
 }
 

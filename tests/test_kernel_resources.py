@@ -73,3 +73,13 @@ def _of(kernels, name):
 def test_scatter_rows_keeps_its_sums_in_registers(kernels):
     for name, k in _of(kernels, "k_scatter_rows").items():
         assert k[".private_segment_fixed_size"] == 0, name
+
+
+@pytest.mark.parametrize("name", ["k_pcg_scatter", "k_ir_scatter", "k_ir_ru_res", "k_cheb_scatter",
+                                  "k_residual", "k_small_scatter", "k_small_update",
+                                  "k_small_dir"])
+def test_solver_row_kernels_run_eight_waves(kernels, name):
+    """512 registers a SIMD lane: 64 a wave for eight waves."""
+    for full, k in _of(kernels, name).items():
+        assert k[".vgpr_count"] <= 64 and k.get(".agpr_count", 0) == 0, full
+        assert k[".private_segment_fixed_size"] == 0, full
