@@ -211,27 +211,20 @@ __device__ __forceinline__ RowTab slot_rows(const SlotDesc &sd) {
     return t;
 }
 
-// E -> L sums of the share's rows: v[k] = the row's sum for a position below
-// bb, z[ii[k]] (written by the element kernel) for an interior DOF.
+// E -> L sum of the row at position t, L-DOF i: of its E-entries below bb, z[i]
+// (written by the element kernel) for an interior DOF.
 template <typename T>
-__device__ __forceinline__ void share_rows(const RowTab &tb, int64_t bb, const Share &h,
-                                           const int (&ii)[kPer], const T *ye, const T *z,
-                                           T (&v)[kPer]) {
-    const bool rows = __ballot(h.lt[0] < bb), inner = __ballot(h.lt[kPer - 1] >= bb);
-    T vz[kPer];
-    if (inner)
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) vz[k] = z[ii[k]];
-    if (rows) {
-        int t[kPer];
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) t[k] = (int)(h.lt[k] < bb ? h.lt[k] : bb - 1);
-        rows_sum<kPer>(tb, t, ye, v);
+__device__ __forceinline__ T row_value(const RowTab &tb, int64_t bb, int t, int i, const T *ye,
+                                       const T *z) {
+    T v = T(0);
+    if (__ballot(t < bb)) {
+        const int t1[1] = {t < bb ? t : (int)bb - 1};
+        T v1[1];
+        rows_sum<1>(tb, t1, ye, v1);
+        v = v1[0];
     }
-    if (inner)
-#pragma unroll
-        for (int k = 0; k < kPer; ++k)
-            if (h.lt[k] >= bb) v[k] = vz[k];
+    if (t >= bb) v = z[i];
+    return v;
 }
 
 // Producer kernels run one block per (slot, chunk) work item and skip the
@@ -546,7 +539,11 @@ kb_diffusion_any(const ElemTask *__restrict__ tasks, const SlotDesc *__restrict_
 #undef X
 }
 
-// z = A d for PH_INNER slots (DIAG_ONE rows copy d); partials of (d, z).
+// z = A d for PH_INNER slots (DIAG_ONE rows copy d); partials of (d, z).  One row
+// at a time, as in the single solves: sums of a share's four rows at once took 102
+// registers (FP64; 4 waves per SIMD) and 90 (FP32; 5) against 38 and 29 (8), and
+// 512 solves of 186M DOFs in all 7.11 s against 6.90 (FP64), 3.73 against 3.60 (BF16);
+// 24 small solves take the same either way.
 template <typename T>
 __global__ void __launch_bounds__(kT)
 kb_scatter(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
@@ -557,26 +554,20 @@ kb_scatter(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
     T *z = gv<T>(sd.z);
     const uint8_t *mask = sd.mask ? global_ptr(sd.mask) : nullptr;
     const RowTab tb = slot_rows(sd);
-    const Share h = share_of(tk.chunk, sd.n);
-    int ii[kPer];
-    T vd[kPer], v[kPer];
-    bool m[kPer];
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        ii[k] = row_dof(tb, (int)h.lt[k]);
-        vd[k] = d[ii[k]];
-        m[k] = mask && mask[ii[k]];
-    }
-    share_rows(tb, sd.bb, h, ii, ye, z, v);
     double acc[1] = {0.0};
-#pragma unroll
+#pragma unroll 1
     for (int k = 0; k < kPer; ++k) {
-        if (!h.ok[k]) continue;
-        if (h.t[k] < sd.bb) {
-            v[k] = m[k] ? vd[k] : v[k];
-            z[ii[k]] = v[k];
+        const int64_t q = (int64_t)tk.chunk * kChunk + k * kT + threadIdx.x;
+        if (q >= sd.n) break;
+        const int t = (int)q, i = row_dof(tb, t);
+        const T vd = d[i];
+        const bool m = mask && mask[i];
+        T v = row_value(tb, sd.bb, t, i, ye, z);
+        if (t < sd.bb) {
+            v = m ? vd : v;
+            z[i] = v;
         }
-        acc[0] += (double)vd[k] * (double)v[k];
+        acc[0] += (double)vd * (double)v;
     }
     store_chunk<1>(acc, sd, tk.chunk, partials, sh);
 }
@@ -772,19 +763,15 @@ kbm_ru_res(const VecTask *__restrict__ tasks, const SlotDesc *__restrict__ desc,
     double *r64 = sd.r64;
     const uint8_t *mask = sd.mask;
     const RowTab tb = slot_rows(sd);
-    const Share h = share_of(tk.chunk, sd.n);
-    int ii[kPer];
-    double v[kPer];
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) ii[k] = row_dof(tb, (int)h.lt[k]);
-    // interior DOFs: (A x)_i was written into r64 by the element kernel
-    share_rows(tb, sd.bb, h, ii, ye64, r64, v);
     double acc[3] = {0.0, 0.0, 0.0};
-#pragma unroll
+#pragma unroll 1
     for (int k = 0; k < kPer; ++k) {
-        if (!h.ok[k]) continue;
-        const int64_t i = ii[k];
-        const double y = (h.t[k] < sd.bb && mask && mask[i]) ? x[i] : v[k];
+        const int64_t q = (int64_t)tk.chunk * kChunk + k * kT + threadIdx.x;
+        if (q >= sd.n) break;
+        const int t = (int)q, i = row_dof(tb, t);
+        // interior DOFs: (A x)_i was written into r64 by the element kernel
+        double y = row_value(tb, sd.bb, t, i, ye64, r64);
+        if (t < sd.bb && mask && mask[i]) y = x[i];
         const double ri = b[i] - y;
         r64[i] = ri;
         const float rf = (float)ri;

@@ -77,7 +77,7 @@ def test_scatter_rows_keeps_its_sums_in_registers(kernels):
 
 @pytest.mark.parametrize("name", ["k_pcg_scatter", "k_ir_scatter", "k_ir_ru_res", "k_cheb_scatter",
                                   "k_residual", "k_small_scatter", "k_small_update",
-                                  "k_small_dir"])
+                                  "k_small_dir", "kb_scatter", "kbm_ru_res"])
 def test_solver_row_kernels_run_eight_waves(kernels, name):
     """512 registers a SIMD lane: 64 a wave for eight waves."""
     for full, k in _of(kernels, name).items():
