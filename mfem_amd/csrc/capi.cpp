@@ -561,9 +561,6 @@ int h1pa_form_assemble(h1pa_form *form, void *stream) {
     Space &sp = *f.space;
     hipStream_t s = as_stream(stream);
     sp.mesh->ensure_nodes(s);
-    // A re-assembly writes the buffers of the last one, which saves freeing and
-    // allocating them; products queued on other streams may still read them.
-    if (f.assembled) device_wait_reuse();
     // a reduced-precision copy of the operator data that is about to change is
     // made again on its next use (ensure_low_precision)
     f.lp_kind = -1;
@@ -582,6 +579,9 @@ int h1pa_form_assemble(h1pa_form *form, void *stream) {
             pack[3 * Q * D + d + D * q] = G[q + Q * d];
         }
     even_odd_tables(D, Q, B.data(), G.data(), pack.data() + 4 * Q * D);
+    // A re-assembly writes the buffers of the last one, which saves freeing and
+    // allocating them; products queued on other streams may still read them.
+    if (f.assembled) device_wait_reuse();
     f.basis.upload(pack.data(), pack.size(), s);
     const int64_t nq = (int64_t)Q * Q * Q;
     auto keep = [](DevBuf<double> &b, int64_t n) {
