@@ -369,8 +369,15 @@ void nodes_curved(const Mesh &m, int pg, double amp, double *d_nodes, hipStream_
 }
 
 // Launches K_(Q, WP, DG) for the number of points and the node count: the field's
-// own order (isoparametric, Q = Dg, Dg + 1 and, for the interpolator, Dg + 2)
-// has its node count compiled in; other curved orders read it at run time.
+// own order (isoparametric, Q = Dg, Dg + 1 and, for the interpolator, Dg + 2) and
+// quadratic geometry under any field have their node count compiled in; other
+// curved orders read it at run time.  Quadratic geometry, run time -> compiled, us
+// of Assemble (of the geometric factors): p = 4, 30^3 elements 128 -> 109 (180 ->
+// 162), p = 6, 20^3 77 -> 63 (109 -> 100), p = 8, 16^3 80 -> 67 (142 -> 118); 2^3
+// elements at p = 8 38 -> 34 (34 -> 30, as long as one thread a point took).  A mesh
+// of a few elements is all latency, and a column's points one after another cost
+// more than a thread each where the coefficient is long (8 cosines a point: 48 us
+// then, 56 now at p = 8, 2^3; 94 and 59 at 7^3).
 #define W_(Q, DG)                                                                             \
     do {                                                                                      \
         if (wp) K_(Q, true, DG);                                                              \
@@ -379,6 +386,7 @@ void nodes_curved(const Mesh &m, int pg, double amp, double *d_nodes, hipStream_
 #define X_(Q)                                                                                 \
     if (q1d == Q) {                                                                           \
         if (gb.Dg == 2) W_(Q, 2);                                                             \
+        else if (gb.Dg == 3 && Q > 3) W_(Q, (Q > 3 ? 3 : 0));                                 \
         else if (gb.Dg == Q && Q > 2 && Q < 10) W_(Q, (Q > 2 && Q < 10 ? Q : 0));             \
         else if (gb.Dg == Q - 1 && Q > 3) W_(Q, (Q > 3 ? Q - 1 : 0));                         \
         else if (gb.Dg == Q - 2 && Q > 4 && ISO2) W_(Q, (Q > 4 && ISO2 ? Q - 2 : 0));         \
@@ -446,6 +454,7 @@ void domain_lf(const Mesh &m, int p, double f, const double *fq, const EOut &out
     if (D == D_) {                                                                            \
         if (gb.Dg == 2) K_(D_, 2);                                                            \
         else if (gb.Dg == D_) K_(D_, D_);                                                     \
+        else if (gb.Dg == 3) K_(D_, 3);                                                       \
         else K_(D_, 0);                                                                       \
     }
     X_(2) X_(3) X_(4) X_(5) X_(6) X_(7) X_(8) X_(9)
