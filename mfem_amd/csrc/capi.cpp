@@ -3,6 +3,7 @@
 // Every entry point catches h1pa::Error (and std::exception) and turns it into
 // a status code plus a thread-local message; nothing throws across the ABI.
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -524,11 +525,13 @@ void autotune_diffusion(Form &f, hipStream_t s) {
     out.l2n = sp.restr.lex2nat.p;
     out.yL = x.p + sp.ndofs;
     out.bb = sp.restr.bubble_begin;
-    // three interleaved rounds (1 warm-up + 4 timed launches per variant each),
-    // so that a drift of the clock or of the other work on the device does
-    // not pick the variant that happened to run in a quiet moment
+    // three interleaved rounds (1 warm-up + 4 timed launches per variant each) and
+    // each variant's middle time, so that neither a drift of the clock nor one
+    // delay in one round decides (p = 1, 38^3 elements: the best variant leads by
+    // 1 us of 20; a sum over the rounds took another in one process of thirty, and
+    // its products of 78^3 elements ran in 162 us instead of 130)
     const int nv = kern::diffusion_variant_count();
-    std::vector<float> total(nv, 0.f);
+    std::vector<std::array<float, 3>> times(nv);
     for (int round = 0; round < 3; ++round)
         for (int v = 0; v < nv; ++v) {
             kern::diffusion_apply_variant(v, p, Q, sp.ne, f.basis.p, f.pa_diff.p,
@@ -541,9 +544,12 @@ void autotune_diffusion(Form &f, hipStream_t s) {
             H1PA_HIP(hipEventSynchronize(e1));
             float ms = 0.f;
             H1PA_HIP(hipEventElapsedTime(&ms, e0, e1));
-            total[v] += ms;
+            times[v][round] = ms;
         }
-    const int best = (int)(std::min_element(total.begin(), total.end()) - total.begin());
+    for (auto &t : times) std::sort(t.begin(), t.end());
+    const int best = (int)(std::min_element(times.begin(), times.end(),
+                                            [](auto &a, auto &b) { return a[1] < b[1]; }) -
+                           times.begin());
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     kern::set_diffusion_variant(p, Q, best);
