@@ -49,6 +49,28 @@ def test_transfer_matches_oracle(orc, h1pa, torch_cuda, pl, ph):
     assert _rel(yl.cpu().numpy(), To.mult_transpose(xh)) < 1e-13
 
 
+@pytest.mark.parametrize("pl,ph", [(l, h) for h in range(2, 9) for l in range(1, h)])
+def test_every_pair_of_orders(orc, h1pa, torch_cuda, pl, ph):
+    """Each pair is a kernel of its own; 31 elements leave the last block partly
+    filled at every number of elements a block (28 to 3).  The bar as above."""
+    M, torch = h1pa, torch_cuda
+    dims = (31, 1, 1)
+    mesh = _mesh(M, dims, 0.2, 9, 0.0, 1)
+    lo = M.FiniteElementSpace(mesh, M.H1_FECollection(pl, 3))
+    hi = M.FiniteElementSpace(mesh, M.H1_FECollection(ph, 3))
+    Pl = orc.Problem(None, pl, perturb=0.2, seed=9, dims=dims)
+    Ph = orc.Problem(None, ph, perturb=0.2, seed=9, dims=dims)
+    To, T = orc.Transfer(Pl, Ph), M.TransferOperator(lo, hi)
+    rng = np.random.default_rng(10 * pl + ph)
+    xl, xh = rng.uniform(-1, 1, Pl.ndofs), rng.uniform(-1, 1, Ph.ndofs)
+    yh = torch.full((Ph.ndofs,), float("nan"), dtype=torch.float64, device="cuda")
+    yl = torch.full((Pl.ndofs,), float("nan"), dtype=torch.float64, device="cuda")
+    T.Mult(torch.from_numpy(xl).cuda(), yh)
+    T.MultTranspose(torch.from_numpy(xh).cuda(), yl)
+    assert _rel(yh.cpu().numpy(), To.mult(xl)) < 1e-13
+    assert _rel(yl.cpu().numpy(), To.mult_transpose(xh)) < 1e-13
+
+
 class MgCase:
     """A fine PA diffusion form (per-element log-uniform k, curved order-p
     geometry) and p-multigrid levels, built by the product and the oracle."""
