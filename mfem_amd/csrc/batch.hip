@@ -6,8 +6,9 @@
 // graph advances all of them by K iterations:
 //
 //   init      slots in INIT: x = 0, r = b, z = dinv r, d = z, (z, r)
-//   K x {     element kernels, one launch per (p, Q) group, over all slots'
-//               elements (a work list of (slot, first element) blocks)
+//   K x {     element kernels over all slots' elements (a work list of (slot,
+//               first element) blocks): one launch per (p, Q) group that fills
+//               the chip by itself, one for all smaller groups together
 //             scatter   z = A d (DIAG_ONE rows copy d), den = (d, z)
 //             update    x += a d, r -= a z, z = dinv r, (r, z), stop test
 //             [mixed, last iteration of the replay: refinement step of the
@@ -19,11 +20,14 @@
 // FP64 mode is MFEM's CGSolver on each slot.  Mixed mode is an FP32 inner CG
 // (FP32 or BF16-stored PA data) with FP64 reliable updates, stopping on
 // CGSolver's measure taken on the FP64 true residual.  Every kernel skips,
-// block-uniformly, the slots that are not in the phase it serves.  Dot
-// products are reduced per slot over fixed chunks of that slot's DOFs: each
-// chunk's block stores its partial, and a finalize kernel (one block per
-// running slot) sums them in index order and applies the step's scalar
-// logic.  So a slot's iterates do not depend on which other slots share the
+// block-uniformly, the slots that are not in the phase it serves, and no launch
+// writes a phase that other blocks of it read.  Dot products are reduced per slot
+// over fixed chunks of that slot's DOFs: each chunk's block stores its partial.
+// They are summed in a fixed order, with the step's scalar logic, by a finalize
+// kernel (one block per running slot) or, where every slot has at most 1024
+// chunks, by every block of the update and direction kernels (the last iteration
+// of a mixed replay, and the first of a replay where that leaves an odd number,
+// keep the finalize kernel before the direction).  Both orders give the same bits.  So a slot's iterates do not depend on which other slots share the
 // batch: a solve gives bitwise the same result alone and in any mix.
 #include <hip/hip_runtime.h>
 
@@ -171,7 +175,7 @@ template <typename T>
 __device__ inline T *vp(void *p) { return reinterpret_cast<T *>(p); }
 
 // The kPer DOFs t[k] = chunk kChunk + k kT + tid of this thread's share of a
-// chunk (ok[k]: t[k] < n).  Kernels load every operand of all kPer DOFs at
+// chunk (ok[k]: t[k] < n).  The vector kernels load every operand of all kPer DOFs at
 // the clamped index lt[k] (in bounds for every k) before the first store, so
 // the loads of a share go out together instead of one DOF's round trip after
 // another; stores and sums then run over the ok entries in k order.

@@ -12,9 +12,10 @@
 //   dir    : d = z + beta d
 //   apply  : element kernel on d (constrained entries read as 0)
 //   scatter: z = A d (DIAG_ONE rows copy d), partials of (d, z) -> fin_den
-// Dot products: each block reduces its chunk of kChunk entries in a fixed
-// tree and stores the partial; a one-block finalize kernel sums the partials
-// in index order.  No block waits for or fences against another (a
+// Systems of up to 262,144 DOFs leave fin_update and fin_den out (k_small_*).
+// Dot products: each block reduces its chunk in a fixed tree and stores the
+// partial; a one-block finalize kernel (small systems: every block of the kernel
+// that needs the product) sums the partials in a fixed order.  No block waits for or fences against another (a
 // device-scope fence writes back and invalidates the whole L2 on this GPU),
 // and the result does not depend on timing.  The vector type T is double or
 // float; scalars and dot accumulation are double.
@@ -174,12 +175,12 @@ __device__ inline void sum_partials(const double *partials, int nb, double *sh,
 
 // Small systems: up to kFoldBlocks blocks of one entry per thread.  The blocks of
 // the kernel that needs a product sum its partials themselves -- four loads a
-// thread that go out with the kernel's other ones -- instead of a one-block
-// kernel of 3-4 us in between, and every load is issued before the first wait,
-// the test of `done` included.  Every block gets the same bits (same loads,
-// same order).  p = 3, 16^3 elements (117,649 DOFs), an iteration: six launches
-// of 29 us together -> four
-// of 22 (6.98 instead of 9.25 ms for a solve of 296 iterations).
+// thread that go out with the vector loads -- instead of a one-block kernel of
+// 3-4 us in between.  Every block gets the same bits (same loads, same order).
+// (The state is read first and waited for: the early return on `done` keeps the
+// compiler from moving vector loads ahead of it, whatever their order here.)
+// p = 3, 16^3 elements (117,649 DOFs), an iteration: six launches of 29 us
+// together -> four of 22 (6.98 instead of 9.25 ms for a solve of 296 iterations).
 constexpr int kFoldBlocks = 4 * kThreads;
 inline bool small_system(const Chunks &c) { return c.per == 1 && c.blocks <= (unsigned)kFoldBlocks; }
 struct FoldSum {
@@ -950,20 +951,6 @@ k_dot(int64_t n, int per, const double *__restrict__ a, const double *__restrict
             if (g.ok[k]) acc[0] += va[k] * vb[k];
     }
     store_partials<1>(acc, partials, sh);
-}
-
-__global__ void __launch_bounds__(kThreads)
-k_dot_fin(int nb, const double *__restrict__ partials, double *__restrict__ out) {
-    __shared__ double sh[kThreads];
-    double tot[1];
-    sum_partials<1>(partials, nb, sh, tot);
-    if (threadIdx.x == 0) out[0] = tot[0];
-}
-
-// v *= m
-__global__ void __launch_bounds__(kThreads)
-k_scale(int64_t n, int per, double *__restrict__ v, double m) {
-    H1PA_CHUNK(i, n) v[i] *= m;
 }
 
 // ---- PowerMethod::EstimateLargestEigenvalue (linalg/operator.cpp:886-935)
