@@ -226,10 +226,12 @@ int h1pa_form_destroy(h1pa_form *form);
 /* a.Assemble(): geometric factors, coefficient and PA data on the device
  * (DiffusionIntegrator::AssemblePA, fem/integ/bilininteg_diffusion_pa.cpp:108-171;
  *  MassIntegrator::AssemblePA, fem/integ/bilininteg_mass_pa.cpp:25-90).
- * Called again it writes the same buffers: it first waits for the work queued
- * on the device, so products already queued on other streams still apply the
- * operator they were queued with.  With the block cache on
- * (h1pa_set_device_cache) it does not wait, and the caller orders such calls. */
+ * Called again it writes the same buffers.  Products queued before on this
+ * stream come first; where the operator data were read on other streams since
+ * the last call, or h1pa_form_pa_data gave them out, it first waits for the
+ * device, so those products still apply the operator they were queued with.
+ * With the block cache on (h1pa_set_device_cache) it does not wait, and the
+ * caller orders such calls. */
 int h1pa_form_assemble(h1pa_form *form, void *stream);
 /* Operator::Mult: y = A x on L-vectors, y overwritten
  * (PABilinearFormExtension::Mult, fem/bilinearform_ext.cpp:487-560). */

@@ -586,8 +586,11 @@ int h1pa_form_assemble(h1pa_form *form, void *stream) {
         }
     even_odd_tables(D, Q, B.data(), G.data(), pack.data() + 4 * Q * D);
     // A re-assembly writes the buffers of the last one, which saves freeing and
-    // allocating them; products queued on other streams may still read them.
-    if (f.assembled) device_wait_reuse();
+    // allocating them; products queued on other streams may still read them (those
+    // on this stream come first by themselves: a wait in every call costs the host
+    // work that runs beside the device, 50 -> 61 us at p = 5, 5^3 elements).
+    if (f.assembled && f.pa_use.beside(s)) device_wait_reuse();
+    f.pa_use.reset();
     f.basis.upload(pack.data(), pack.size(), s);
     const int64_t nq = (int64_t)Q * Q * Q;
     auto keep = [](DevBuf<double> &b, int64_t n) {
@@ -626,6 +629,7 @@ void element_apply(Form &f, const int *gmap, const uint8_t *mask, const double *
         out.l2n = f.space->restr.lex2nat.p;
     }
     Space &sp = *f.space;
+    f.pa_use.note(s);
     const bool diff = f.desc.integrators & H1PA_INTEG_DIFFUSION;
     const bool mass = f.desc.integrators & H1PA_INTEG_MASS;
     if (diff)
@@ -644,6 +648,7 @@ void element_apply(Form &f, const int *gmap, const uint8_t *mask, const double *
 // are set up on the first call.
 bool columns_ready(Form &f, hipStream_t s) {
     if (f.use_columns == 0) return false;
+    f.pa_use.note(s);
     Space &sp = *f.space;
     Mesh &m = *sp.mesh;
     if (f.use_columns < 0) {
@@ -743,6 +748,7 @@ void h1pa::keep_stream_pool() {
 // rest in native order), then AbsMultTranspose of the other rows.
 void h1pa::operator_diagonal(Form &f, double *diag, hipStream_t s) {
     Space &sp = *f.space;
+    f.pa_use.note(s);
     const bool diff = f.desc.integrators & H1PA_INTEG_DIFFUSION;
     const bool mass = f.desc.integrators & H1PA_INTEG_MASS;
     kern::EOut out;
@@ -934,6 +940,7 @@ int h1pa_form_assemble_diagonal(h1pa_form *form, double *diag, void *stream) {
 int h1pa_form_pa_data(const h1pa_form *form, const double **dd, const double **dm) {
     API_BEGIN
     REQUIRE(form, "form: null");
+    form->f.pa_use.unknown();
     if (dd) *dd = form->f.pa_diff.p;
     if (dm) *dm = form->f.pa_mass.p;
     API_END

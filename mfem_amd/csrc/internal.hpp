@@ -254,6 +254,20 @@ struct Space {
     DevBuf<uint8_t> ess_mask;  // [ndofs] 1 on boundary DOFs
 };
 
+// The streams on which kernels reading some data were queued since reset().
+struct StreamUse {
+    hipStream_t first = nullptr;
+    bool any = false, several = false;
+    void note(hipStream_t s) {
+        several |= any && s != first;
+        if (!any) first = s;
+        any = true;
+    }
+    void unknown() { any = several = true; }  // read by others than this library
+    bool beside(hipStream_t s) const { return any && (several || s != first); }
+    void reset() { any = several = false; }
+};
+
 struct Form {
     Space *space = nullptr;
     h1pa_form_desc desc{};
@@ -265,6 +279,7 @@ struct Form {
     DevBuf<double> lwork0, lwork1;  // L-vector scratch
     DevBuf<uint8_t> cmask;          // constraint mask of the last ess list passed in
     bool assembled = false;
+    mutable StreamUse pa_use;  // readers of pa_diff and pa_mass since the last Assemble
     // Reduced-precision shadows for the inner solver (built on first use from
     // the FP64 data): basis in FP32, PA data in FP32 or BF16 (lp_kind 0 / 1).
     DevBuf<float> basis32;

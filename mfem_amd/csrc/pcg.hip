@@ -1068,6 +1068,7 @@ template <typename T>
 void pcg_element_apply(Form &f, int prec, const uint8_t *mask, const T *d, T *ye, T *yL,
                        const int *stop, hipStream_t s, bool stop_late = false) {
     Space &sp = *f.space;
+    f.pa_use.note(s);
     const bool diff = f.desc.integrators & H1PA_INTEG_DIFFUSION;
     const bool mass = f.desc.integrators & H1PA_INTEG_MASS;
     kern::EOutT<T> out;
@@ -1392,6 +1393,7 @@ void require_no_batch_refs(const Form &f, const char *what) {
 void ensure_low_precision(Form &f, int precision, hipStream_t s) {
     const int kind = precision == H1PA_PREC_BF16_PA ? 1 : 0;
     if (f.lp_kind == kind) return;
+    f.pa_use.note(s);  // the conversions read the FP64 data
     // replacing the shadow frees the buffers live batch slots read
     if (f.lp_kind >= 0) require_no_batch_refs(f, "reduced-precision shadow of another kind");
     Space &sp = *f.space;

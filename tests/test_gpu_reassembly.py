@@ -81,26 +81,48 @@ def test_bf16_cycle_follows_the_operator(h1pa, torch_cuda):
     assert torch.equal(got, cycle(_form(M, fes, k)))
 
 
-def test_products_queued_on_another_stream(h1pa, torch_cuda):
+def _queue(M, torch, what, fes, a, x, n):
+    """n results of one kind queued on the current stream, which read the operator
+    data; and the vector that each writes."""
+    ess = fes.GetBoundaryTrueDofs()
+    if what == "low":
+        x = x.float()
+    ys = [torch.full_like(x, float("nan")) for _ in range(n)]
+    if what == "mult":
+        f = [lambda y: a.Mult(x, y)]
+    elif what == "low":
+        f = [lambda y: a.MultLowPrecision(x, y, M.PREC_BF16_PA)]
+    elif what == "diagonal":
+        f = [a.AssembleDiagonal]
+    else:
+        A = M.ConstrainedOperator(a, ess)
+        S = M.OperatorChebyshevSmoother(A, None, ess, 2) if what == "smoother" else A
+        f = [lambda y: S.Mult(x, y)]
+    return ys, f[0]
+
+
+@pytest.mark.parametrize("what", ["mult", "low", "diagonal", "constrained", "smoother"])
+def test_products_queued_on_another_stream(h1pa, torch_cuda, what):
     """Products queued on one stream when another re-assembles apply the operator
-    they were queued with: bitwise the product before."""
+    they were queued with: bitwise the product before.  On the same stream they
+    need no wait, and with a second stream in between they do again."""
     M, torch = h1pa, torch_cuda
     mesh, fes = _space(M, 4, 24)
     k = torch.full((fes.GetNE(),), 2.0, dtype=torch.float64, device="cuda")
     x = torch.rand(fes.GetNDofs(), dtype=torch.float64, device="cuda")
     a = _form(M, fes, k)
-    want = torch.empty_like(x)
-    a.Mult(x, want)
-    st = [torch.cuda.Stream(), torch.cuda.Stream()]
-    for round_ in range(5):
-        ys = [torch.full_like(x, float("nan")) for _ in range(40)]
+    st = [torch.cuda.Stream() for _ in range(3)]
+    for queue, assemble in ((0, 1), (1, 1), (2, 0), (0, 0), (1, 0)):
+        want, f = _queue(M, torch, what, fes, a, x, 1)
+        f(want[0])
+        ys, f = _queue(M, torch, what, fes, a, x, 30)
+        f(ys[0])
         torch.cuda.synchronize()
-        with torch.cuda.stream(st[0]):
+        with torch.cuda.stream(st[queue]):
             for y in ys:
-                a.Mult(x, y)
-        with torch.cuda.stream(st[1]):
+                f(y)
+        with torch.cuda.stream(st[assemble]):
             k.add_(1.0)
             a.Assemble()
         torch.cuda.synchronize()
-        assert all(torch.equal(y, want) for y in ys), round_
-        a.Mult(x, want)
+        assert all(torch.equal(y, want[0]) for y in ys), (queue, assemble)
