@@ -54,9 +54,10 @@ struct SlotState {
     double nom, nom0, den, betanom, beta, r0;  // PCG scalars (mixed: nom = inner (r, z))
     double rho_ref, rho64, rho64_0, r2, b2;    // mixed: refinement bookkeeping
     int iter, in_loop, max_iter, converged, final_iter;
-    int phase, outer;
-    int nonfinite;  // a (B r, r) or (A d, d) was not finite: retired with a failed status
+    int phase;
     int den_ends;   // folded update: (A d, d) ends the inner iterations (write_den is due)
+    int outer;
+    int nonfinite;  // a (B r, r) or (A d, d) was not finite: retired with a failed status
 };
 
 struct SlotDesc {

@@ -39,10 +39,10 @@ struct PcgState {
     int in_loop;     // 0 before the first update, then 1
     int max_iter;
     int done;
+    int den_ends;    // small systems: (A d, d) of this iteration ends the loop (read with done)
     int converged;
     int final_iter;
     int nonfinite;   // a (B r, r) or (A d, d) was not finite: MFEM_VERIFY fails
-    int den_ends;    // small systems: (A d, d) of this iteration ends the loop
 };
 
 namespace kern {
