@@ -652,7 +652,7 @@ def main():
             "traffic": traffic_from_profiles(args.p, n, "mult_" + r["path"], r["variant"]),
             "kernel": ("k_diffusion_columns + k_columns_interface (one Operator::Mult)"
                        if r["path"] == "columns" else
-                       "k_diffusion_apply + k_restrict_mult_t (one Operator::Mult)"),
+                       "k_diffusion_apply + k_scatter_rows (one Operator::Mult)"),
             "ms": round(r["event_ms"], 4),
             "bytes_per_launch": r["bytes_apply"],
             "bytes_formula": "NE (6 Q^3 8 + D^3 4) + 2 N 8",

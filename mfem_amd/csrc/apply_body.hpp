@@ -35,7 +35,7 @@ constexpr double lane_use(int nb, int QQ) {
 // each, counted without the padding of even Q (ElemLds): about 256 threads within
 // 48 KiB of LDS.  With the padding an FP64 block may take 55 KB (D = Q = 8, two
 // blocks per CU); three elements instead of its four measured no better with the
-// variant that is best for each (7^3 DOFs an element, q1d = 8: 9^3 elements 13.6
+// variant that is best for each (p = 7, q1d = 8: 9^3 elements 13.6
 // against 13.9 us a call, 20^3 63.4 against 66.2, 42^3 549 against 542).  Where that leaves more than
 // a tenth of the lanes idle (Q = 9, 10: 81 or 100 threads per element) and
 // the values are 4-byte, the count with the best lane use within 1024 threads
